@@ -8,6 +8,7 @@
 
 #include "hankel_internal.h"
 #include "hankel_j0.h"
+#include "sincos_reduced.h"
 
 namespace {
 
@@ -134,47 +135,6 @@ template __global__ void hk_direct_kernel<float2>(hk_planes, int, const double *
                                                   double, double);
 
 namespace {
-
-// sin and cos of x for |x| < kSincosLimit: Cody-Waite reduction x = n pi/2 + y with pi/2 split into
-// three doubles (each product n * c_i exact inside an FMA), then the Taylor series of sin y
-// (through y^17) and cos y (through y^18) on |y| <= pi/4, whose first omitted terms are below
-// 1e-19, and the quadrant n mod 4.  The constants are pi/2 = c1 + c2 + c3 and 1/k! rounded to
-// double.  Fewer registers and instructions than the general routine, which also serves
-// arguments up to 1e308.
-__device__ inline void sincos_reduced(double x, double *s, double *c)
-{
-    constexpr double c1 = 0x1.921fb54442d18p+0, c2 = 0x1.1a62633145c07p-54, c3 = -0x1.f1976b7ed8fbcp-110;
-    constexpr double two_over_pi = 0x1.45f306dc9c883p-1;
-    const double n = rint(x * two_over_pi);
-    double y = fma(-n, c1, x);
-    y = fma(-n, c2, y);
-    y = fma(-n, c3, y);
-    const double z = y * y;
-    // 1/k! with alternating signs
-    double ps = 2.8114572543455206e-15;
-    ps = fma(ps, z, -7.647163731819816e-13);
-    ps = fma(ps, z, 1.6059043836821613e-10);
-    ps = fma(ps, z, -2.505210838544172e-08);
-    ps = fma(ps, z, 2.7557319223985893e-06);
-    ps = fma(ps, z, -0.0001984126984126984);
-    ps = fma(ps, z, 0.008333333333333333);
-    ps = fma(ps, z, -0.16666666666666666);
-    const double sy = fma(y * z, ps, y);
-    double pc = -1.5619206968586225e-16;
-    pc = fma(pc, z, 4.779477332387385e-14);
-    pc = fma(pc, z, -1.1470745597729725e-11);
-    pc = fma(pc, z, 2.08767569878681e-09);
-    pc = fma(pc, z, -2.755731922398589e-07);
-    pc = fma(pc, z, 2.48015873015873e-05);
-    pc = fma(pc, z, -0.001388888888888889);
-    pc = fma(pc, z, 0.041666666666666664);
-    pc = fma(pc, z, -0.5);
-    const double cy = fma(z, pc, 1.0);
-    const int q = (int)n & 3;
-    const double sa = (q & 1) ? cy : sy, ca = (q & 1) ? sy : cy;
-    *s = (q & 2) ? -sa : sa;
-    *c = ((q + 1) & 2) ? -ca : ca;
-}
 
 // Lagrange basis of HK_GRID_P nodes at offsets d_i = i - (P/2 - 1) from floor(t), at f = frac(t)
 struct Lagrange {

@@ -2,6 +2,8 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include "sincos_reduced.h"
+
 #include "hankel.h"
 
 // Photon/medium constants of the Python unit set (shared_python/units.py:3-20,
@@ -36,8 +38,6 @@ template <int TYPE>
 __global__ void hk_spread_kernel(hk_planes p, const double *weights, int nq, double h, double inv_c, void *out,
                                  long long ld, long long row0);
 
-// range of sincos_reduced (hankel_contract.hip): |x| below it keeps n = rint(2x/pi) an exact int
-constexpr double kSincosLimit = 1e9;
 
 // hk_spread_window_kernel: doubles of per-plane factors in LDS after the bins (5 used, padded
 // to keep each plane's entry 16-byte aligned)
