@@ -35,7 +35,9 @@ sys.path.insert(0, ROOT)
 
 METRIC = "TDSE grid-pt-steps/s batched vs per-instance @≤1e-8 err; adjoint/fwd time ratio"
 HBM_PEAK_GBS = 8000.0
-BYTES_PER_PT_STEP = 32.0  # psi read + write, complex128
+BYTES_PER_PT_STEP = 32.0  # psi read + write, complex128 (the streaming kernels)
+FP64_PEAK_TFLOPS = 78.6   # vector units
+FLOP_PER_PT_STEP = 68.0   # right-hand side, the two recurrences, 1 / (1 + i g), phase and observables, FMA = 2
 # HBM bytes per launch on the default 64 x 64 workload, by steps per pass of the launch shape
 # (1: tdse_propagate_kernel at 4 x 3, 2: tdse_propagate_pair_stash_kernel at 4 x 2), from
 # rocprofv3 FETCH_SIZE and WRITE_SIZE counters scaled by their readings for a plain 1 GiB device
@@ -698,7 +700,12 @@ def main():
         "config": {"workload": "tdse-batch-gaussian-beam", "instances": n_inst, "grid_r_x_z": [args.n_r, args.n_z],
                    "Nx": nx, "dx": g["dx"], "dt": 0.25, "time_steps": n_steps, "atom": "Ar (a=1.1893)",
                    "field": "800nm 10-cycle sin2, 1.5e14 W/cm2 peak, w0=100um", "precision": "complex128"},
-        "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
+        "roofline": {"bound": "fp64", "achieved": FLOP_PER_PT_STEP * pt_steps / (kern_ms * 1e-3) / 1e12,
+                     "peak": FP64_PEAK_TFLOPS, "unit": "TFLOP/s",
+                     "frac": FLOP_PER_PT_STEP * pt_steps / (kern_ms * 1e-3) / 1e12 / FP64_PEAK_TFLOPS,
+                     "copy_ceiling": copy_gbs, "read_only_ceiling": read_gbs, "write_only_ceiling": write_gbs,
+                     "kernel": "tdse_resident_kernel"} if tuned.config.library_choice else
+                    {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": achieved / HBM_PEAK_GBS,
                      "copy_ceiling": copy_gbs, "frac_of_copy_ceiling": achieved / copy_gbs if copy_gbs else None,
                      "read_only_ceiling": read_gbs, "write_only_ceiling": write_gbs,
@@ -710,6 +717,7 @@ def main():
         "gpu_over_cpu_baseline": (value / cpu["value"]) if cpu else None,
         "parity_vs_reference": parity,
         "launch": {"form": "hipGraph replay of one persistent launch", "config": list(tuned.config.as_tuple()),
+                   "library_choice": tuned.config.library_choice,
                    "tune_table": [list(r) for r in tuned.table[:6]], "tune_s": t_tune, "cached": tuned.cached},
         "stepwise_form": stepwise,
         "persistent_over_stepwise": (value / stepwise["pt_steps_per_s"]) if stepwise else None,

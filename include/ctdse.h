@@ -200,10 +200,10 @@ int ctdse_propagate_batch(int n_inst, const ctdse_geometry *const *geom, const i
 /*
  * One instance alone, the propagation call1DTDSE runs (no counterpart of its own in the
  * reference: 1DTDSE/sources/singleTDSE.c:105 calls propagation there).  Arguments as for
- * one instance of ctdse_propagate_batch.  The segments of each step run side by side, one
- * launch per step, so one instance gets most of the GPU; both recurrences are truncated at a
- * halo on either side of a segment, so results equal the batch's to rounding (about 1e-13
- * relative on the dipole), not bitwise.  Returns once the work queued on `stream` has
+ * one instance of ctdse_propagate_batch.  The grid is cut into overlapping windows that run
+ * side by side, up to 16 steps per launch, so that one instance gets a good part of the GPU; both
+ * recurrences are truncated at a window's ends, so results equal the batch's to rounding (about
+ * 1e-13 relative on the dipole), not bitwise.  Returns once the work queued on `stream` has
  * finished.
  */
 int ctdse_propagate_one(const ctdse_geometry *geom, int n_steps, const double *field, double *out, void *stream);
@@ -212,13 +212,12 @@ int ctdse_propagate_one(const ctdse_geometry *geom, int n_steps, const double *f
  * ctdse_propagate_one without device allocation.  No counterpart in the reference: it is
  * for callers that cannot allocate (code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc).  Same arguments and results (bit for bit) as
- * ctdse_propagate_one; its scratch (two state vectors, the gated field, per-segment partial
- * sums, the descriptors) lives in a fixed device array of CTDSE_NOALLOC_SCRATCH_BYTES that
- * each GPU the library runs on holds until the process ends, and it calls no hipMalloc,
+ * ctdse_propagate_one; its scratch (two state vectors, the gated field, the windows' sums,
+ * the descriptors) lives in a fixed device array, of which a run may count on
+ * CTDSE_NOALLOC_SCRATCH_BYTES, that each GPU the library runs on holds until the process ends, and it calls no hipMalloc,
  * hipFree or allocating library routine.  A run needs about
  * 32 * ctdse_state_length(geom) + 8 * (n_steps + 1) bytes plus a few KiB: larger runs fail
- * with CTDSE_ERR_ARGUMENT; a geometry whose truncation halo leaves no room for the
- * step-parallel solve fails with CTDSE_ERR_UNSUPPORTED.  It queues the work on `stream` and
+ * with CTDSE_ERR_ARGUMENT.  It queues the work on `stream` and
  * returns without waiting.  Every call on one GPU shares that GPU's array and leaves its
  * contents behind (each call initialises what it reads): calls that overlap on one GPU, on
  * other streams or from other threads, race; order them on one stream.
@@ -240,7 +239,8 @@ int ctdse_geometry_create_batch(int n, const int *num_r, const double *dx, const
                                 const double *e_guess, const double *cv, const double *x_int, ctdse_geometry **out,
                                 int *status);
 
-/* Launch shape of the persistent propagation kernel: waves per workgroup (one segment
+/* Launch shape of the kernels that stream the states through memory; without one, the library
+ * runs the kernel that keeps each state on the chip (results equal to rounding).  Waves per workgroup (one segment
  * of the parallel tridiagonal solve covers 64 * waves_per_group chunks of 8 points),
  * resident workgroups per compute unit, and time steps per pass over the state (1, or 2:
  * the intermediate state stays on chip wherever no save or snapshot falls between the
@@ -252,14 +252,14 @@ typedef struct ctdse_launch_config {
     int steps_per_pass;
 } ctdse_launch_config;
 
-/* The shape ctdse_propagate_batch uses for these geometries. */
+/* The default shape of the streaming kernels for these geometries. */
 int ctdse_launch_config_default(int n_inst, const ctdse_geometry *const *geom, ctdse_launch_config *cfg);
 
 /*
  * Prepared batch (no counterpart in the reference).  ctdse_batch_plan_create takes the
  * arguments of ctdse_propagate_batch, the distance in doubles between an instance's five
  * output rows (out_row_stride >= n_steps[i]; 0: n_steps[i], rows packed as in
- * ctdse_propagate_batch) and a launch shape (NULL: the default); it validates them,
+ * ctdse_propagate_batch) and a launch shape (NULL: the library's own launch); it validates them,
  * uploads the instance descriptors and allocates a private work buffer, once.
  *   ctdse_batch_plan_enqueue:      queues the batch on `stream` and returns at once; it
  *                                  allocates, copies and waits for nothing, so a caller
@@ -279,7 +279,8 @@ int ctdse_batch_plan_create(int n_inst, const ctdse_geometry *const *geom, const
                             long long out_row_stride, const ctdse_launch_config *config, ctdse_batch_plan **plan);
 int ctdse_batch_plan_enqueue(ctdse_batch_plan *plan, void *stream);
 int ctdse_batch_plan_graph_launch(ctdse_batch_plan *plan, void *stream);
-/* Shape in use and the number of persistent workgroups of one run. */
+/* The shape given at creation (ctdse_launch_config_default's without one) and the number of
+ * persistent workgroups of one run. */
 int ctdse_batch_plan_info(const ctdse_batch_plan *plan, ctdse_launch_config *config, int *workgroups);
 void ctdse_batch_plan_destroy(ctdse_batch_plan *plan);
 

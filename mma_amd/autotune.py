@@ -1,6 +1,7 @@
-"""Launch-shape autotuner of the persistent TDSE propagator.
+"""Launch autotuner of the persistent TDSE propagator.
 
-The propagation kernel's launch parameters trade against each other:
+The library's own launch keeps the states on the chip and has nothing to tune; it is the first
+candidate.  The launch parameters of the kernels that stream the states trade against each other:
 
 * waves per workgroup sets the partition of the parallel tridiagonal solve: a segment is
   64 * waves chunks of 8 points, of which the truncation halo (H chunks, fixed by the
@@ -85,7 +86,9 @@ def _store_cache(key, entry):
 class TuneResult:
     def __init__(self, config, table, cached, key):
         self.config = config      # tdse.LaunchConfig
-        self.table = table        # [(waves, groups_per_cu, steps_per_pass, pt_steps_per_s)], fastest first
+        # [(waves, groups_per_cu, steps_per_pass, pt_steps_per_s)], fastest first; the row of the
+        # library's own launch has the shape of the streaming kernels' default
+        self.table = table
         self.cached = cached
         self.key = key
 
@@ -93,8 +96,14 @@ class TuneResult:
         return "TuneResult(%r, cached=%s, %d candidates)" % (self.config, self.cached, len(self.table))
 
 
+def _config(shape, library_choice):
+    cfg = tdse.LaunchConfig(*shape)
+    cfg.library_choice = bool(library_choice)
+    return cfg
+
+
 def tune(geometries, fields, n_steps=None, trial_steps=48, repeats=2, use_cache=True, stream=None, pairs=None):
-    """Pick the launch shape for a batch.
+    """Pick the launch for a batch: the library's own or a launch shape.
 
     geometries: one tdse.Geometry per row of `fields` (or one for all);
     fields:     the batch's (n_inst, L) float64 CUDA field tensor;
@@ -113,11 +122,11 @@ def tune(geometries, fields, n_steps=None, trial_steps=48, repeats=2, use_cache=
     key, blob = signature(props.name, props.multi_processor_count, [g.num_r + 1 for g in geoms], n_steps)
     if use_cache and pairs is None:
         hit = _load_cache().get(key)
-        if hit:
-            return TuneResult(tdse.LaunchConfig(*hit["config"]), [tuple(r) for r in hit["table"]], True, key)
+        if hit and "library_choice" in hit:  # without it: tuned before the library's own launch was a candidate
+            return TuneResult(_config(hit["config"], hit["library_choice"]), [tuple(r) for r in hit["table"]], True, key)
     halo = max(g.halo_points // CHUNK for g in geoms)
     full_search = pairs is None
-    pairs = list(pairs) if pairs is not None else candidates(halo)
+    pairs = list(pairs) if pairs is not None else [None] + candidates(halo)
     trial = [max(1, min(int(s), int(trial_steps))) for s in n_steps]  # even: whole pairs
     width = max(trial)
     scratch = torch.empty((n_inst, 5, width), dtype=torch.float64, device=dev)
@@ -138,11 +147,14 @@ def tune(geometries, fields, n_steps=None, trial_steps=48, repeats=2, use_cache=
                 ms = t0.elapsed_time(t1)
                 best = ms if best is None else min(best, ms)
         plan.close()
-        table.append(tuple(plan.config.as_tuple()) + (plan.pt_steps / (best * 1e-3),))
-    table.sort(key=lambda r: -r[-1])
-    cfg = tdse.LaunchConfig(*table[0][:3])
+        table.append((plan.config.as_tuple() + (plan.pt_steps / (best * 1e-3),), shape is None))
+    table.sort(key=lambda r: -r[0][-1])
+    library = table[0][1]
+    table = [row for row, _ in table]
+    cfg = _config(table[0][:3], library)
     if use_cache and full_search:
-        _store_cache(key, {"config": list(cfg.as_tuple()), "table": [list(r) for r in table], "batch": blob})
+        _store_cache(key, {"config": list(cfg.as_tuple()), "library_choice": library,
+                           "table": [list(r) for r in table], "batch": blob})
     return TuneResult(cfg, table, False, key)
 
 

@@ -31,6 +31,7 @@ SOURCES = [
     ("tdse_setup.hip", ["-ffp-contract=off"]),
     ("tdse_analysis.hip", ["-ffp-contract=off"]),
     ("tdse_propagate.hip", []),
+    ("tdse_resident.hip", []),
     ("tdse_adjoint.hip", []),
     ("tdse_reverse.hip", []),
     ("ctdse_abi.cpp", ["-x", "hip"]),
@@ -42,8 +43,8 @@ SOURCES = [
 ]
 
 LIBS = {
-    "libsingleTDSE.so": ["tdse_setup.hip", "tdse_analysis.hip", "tdse_propagate.hip", "tdse_adjoint.hip",
-                         "tdse_reverse.hip", "ctdse_abi.cpp"],
+    "libsingleTDSE.so": ["tdse_setup.hip", "tdse_analysis.hip", "tdse_propagate.hip", "tdse_resident.hip",
+                         "tdse_adjoint.hip", "tdse_reverse.hip", "ctdse_abi.cpp"],
     "libmmahankel.so": ["hankel_medium.hip", "hankel_contract.hip", "hankel_gemm.hip", "hankel_abi.cpp"],
     # bandwidth probes for bench.py only (not part of the product)
     "libmmaprobe.so": ["stream_probe.hip"],

@@ -20,7 +20,10 @@
 // Device memory of ctdse_propagate_one_noalloc, one copy per GPU for the life of the process.
 // Host code never uses this name as an address: the device address comes from
 // hipGetSymbolAddress (scratch_address below).
-static __device__ __align__(256) unsigned char scratch[CTDSE_NOALLOC_SCRATCH_BYTES];
+// The margin holds what the windows need beyond the two states, the field and the few KiB that callers count with:
+// their sums of 16 steps (80 KiB for 64 windows) and states in whole tiles of lanes (up to 48 KiB more).
+constexpr size_t kScratchBytes = CTDSE_NOALLOC_SCRATCH_BYTES + (size_t(256) << 10);
+static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 
 namespace {
 
@@ -92,6 +95,7 @@ constexpr double kTruncTol = 1e-17;   // relative truncation of the segmented so
 struct Lattice {
     static constexpr int kAlign = TDSE_CHUNK;
     DevMem g[kAlign], dpot[kAlign], ib[kAlign], chq[kAlign], chg[kAlign];
+    DevMem res[3];  // the resident kernel's tables (gv, s, b) for 16, 24 and 32 points per lane
 };
 
 struct ctdse_geometry {
@@ -100,7 +104,10 @@ struct ctdse_geometry {
     double dx = 0, dt = 0, a = 0, x_int = 0;
     double e_init = 0;
     int gs_iters = 0;
-    DevMem x, psi0_nat, g, dpot, ib, psi0, chq, chg, adq, adg;
+    bool psi0_real = false;  // Im psi0 = 0 at every point
+    int reach = 0;  // points after which the recurrences' carries are below kTruncTol
+    DevMem x, psi0_nat, g, dpot, ib, psi0, chq, chg, adq, adg, res[3];
+    std::shared_ptr<DevMem> core;  // the resident kernel's tables of each geometry made together
     std::shared_ptr<Lattice> lattice;  // null, or the batch's shared tables this geometry reads
     int lattice_shift = -1;            // the alignment of `lattice` it reads (0..7)
 };
@@ -218,6 +225,8 @@ int finish_tables(ctdse_geometry *G, const TableJob &J, const std::string &who)
     D.chg = G->chg.as<double2>();
     D.adq = G->adq.as<double2>();
     D.adg = G->adg.as<double2>();
+    G->reach = W;
+    G->psi0_real = J.psi0_real != 0;
     D.nx = nx;
     D.nchunks = nchunks;
     D.npad = tdse_tiled_size(nchunks);
@@ -270,6 +279,7 @@ int build_tables(const std::vector<ctdse_geometry *> &gs, const std::vector<int>
         J.p0_lo = Jh.p0_lo;
         J.p0_hi = Jh.p0_hi;
         J.pint0 = Jh.pint0;
+        J.psi0_real = Jh.psi0_real;
         HIP_CHECK(hipMemcpy(piv.p, piv_h.data(), 2 * nx * sizeof(double), hipMemcpyHostToDevice));
         HIP_CHECK(hipMemcpy(d_job.p, &J, sizeof(TableJob), hipMemcpyHostToDevice));
         const int nchunks = (int)((nx + TDSE_CHUNK - 1) / TDSE_CHUNK);
@@ -445,6 +455,216 @@ int share_lattices(const std::vector<ctdse_geometry *> &gs)
     return CTDSE_OK;
 }
 
+// How the resident kernel covers nx points whose carries reach `reach` points: lanes of C points,
+// waves and windows (TdseResident).  A function of the geometry alone, so an instance's results do
+// not depend on the batch around it.  Costs in instructions per lane and step, from the kernel's
+// listing: 55 per point and 330 for the scans, the phase and the sums.
+//   One window: (C, waves) by the work of a CU per instance and step (8 waves fit one, so a CU holds
+//   8 / waves workgroups), and within a quarter of the least by a step's latency: 16 points x 8 waves
+//   rather than 32 x 4 for 8001 points, 18 % more work in half the time per step.
+//   Several (the grid is larger than 8 waves x 32 lanes' points): `steps` steps between a window's load
+//   and store cost a halo of steps x reach points at each inner edge; loading, b included, and
+//   storing cost about 60 per point.
+bool plan_resident(int nx, int reach, TdseResident &R)
+{
+    static const int kChunks[3] = {16, 24, 32};
+    const int margin = reach + 2;  // per step: both recurrences, and the right-hand side's neighbours
+    R.chunk = 0;
+    auto per_step = [](int C) { return 55.0 * C + 330.0; };
+    double least = INFINITY;
+    for (int pass = 0; pass < 2; pass++) {
+        double best = INFINITY;
+        for (int C : kChunks) {
+            if (reach > 16 * C) continue;
+            const int waves = (nx + C - 1 + 64 * C - 1) / (64 * C);
+            if (waves > TDSE_MAX_WAVES) continue;
+            const double cost = per_step(C) / (TDSE_MAX_WAVES / waves);
+            if (pass == 0) {
+                least = std::min(least, cost);
+            } else if (cost <= 1.25 * least && per_step(C) < best) {
+                best = per_step(C);
+                R.chunk = C;
+                R.waves = waves;
+            }
+        }
+    }
+    R.reach = reach;
+    R.windows = 1;
+    R.steps = TDSE_RES_RING;
+    R.stride = R.halo = 0;
+    if (R.chunk) return true;
+    double best = INFINITY;
+    for (int C : kChunks) {
+        if (reach > 16 * C) continue;
+        const int lanes = 64 * TDSE_MAX_WAVES, total = (nx + C - 1 + C - 1) / C;
+        for (int T = TDSE_RES_RING; T >= 1; T--) {
+            const int halo = (T * margin + C - 1) / C, stride = lanes - 2 * halo;
+            if (stride < 64) continue;
+            const int n = 1 + (total - lanes + stride - 1) / stride;
+            const double cost = n * (T * per_step(C) + 60.0 * C) / T;
+            if (cost < best) {
+                best = cost;
+                R.chunk = C;
+                R.waves = TDSE_MAX_WAVES;
+                R.windows = n;
+                R.steps = T;
+                R.stride = stride;
+                R.halo = halo;
+            }
+        }
+    }
+    return R.chunk > 0;
+}
+
+// Dynamic LDS of a workgroup of plan R: the lanes' share of b.
+size_t lane_lds(const TdseResident &R)
+{
+    return (size_t)R.waves * 64 * std::min(R.chunk, TDSE_RES_LDS) * sizeof(double2);
+}
+
+// Entries of a resident table of nx points in lanes of C: whole tiles, one zero chunk at least.
+long long resident_entries(int nx, int C) { return (long long)(((nx + C - 1) / C + 1 + 63) / 64) * 64 * C; }
+
+// Points before a run of pivots from the double ones, whose error of 1e-16 decays by rho^2 a point: to
+// below 1e-20 (rho^reach = 1e-17).
+int resident_warm(int reach) { return reach / 8 + 4; }
+
+int build_resident(const ctdse_geometry *G, int C, DevMem &mem)
+{
+    const long long n = resident_entries(G->dev.nx, C);
+    HIP_CHECK(mem.alloc(3 * n * sizeof(double2)));
+    double2 *t = mem.as<double2>();
+    const int chunks = (int)(n / C);
+    const int threads = (int)(n / TDSE_RES_GROUP);
+    hipLaunchKernelGGL(tdse_resident_tables_kernel, dim3((threads + 63) / 64), dim3(64), 0, 0, G->dev.g, G->dev.dpot,
+                       G->dev.ib, G->dev.nx, G->dev.k36, C, chunks, resident_warm(G->reach), t, t + n, t + 2 * n);
+    HIP_CHECK(hipGetLastError());
+    return CTDSE_OK;
+}
+
+// The windows of one instance alone: lanes of 16 points (24 where carries reach further), four waves, one
+// per SIMD, a window; as many steps per launch as leave at most kOneWindows windows.  With 16001
+// points: 39 windows of 4096 points, 13 steps a launch.
+constexpr int kOneWindows = 64;
+void plan_one(int nx, int reach, TdseResident &R)
+{
+    const int C = reach <= 16 * 16 ? 16 : 24, total = (nx + C - 1 + C - 1) / C, margin = reach + 2;
+    R.chunk = C;
+    R.reach = reach;
+    R.windows = 1;
+    R.steps = TDSE_RES_RING;
+    R.stride = R.halo = 0;
+    R.waves = std::min(TDSE_ONE_WAVES, (total + 63) / 64);
+    const int lanes = 64 * TDSE_ONE_WAVES;
+    if (total <= lanes) return;
+    for (int T = TDSE_RES_RING; T >= 1; T--) {
+        const int halo = (T * margin + C - 1) / C, stride = lanes - 2 * halo;
+        if (stride < 1) continue;
+        R.windows = 1 + (total - lanes + stride - 1) / stride;
+        R.steps = T;
+        R.stride = stride;
+        R.halo = halo;
+        if (R.windows <= kOneWindows || T == 1) return;
+    }
+}
+
+// The lane-tile tables that a plan R of geometry G reads: its own, or those of its lattice (the widest
+// geometry's, whose pivots are replaced near G's own left wall); J: what the geometry needs besides.
+int attach_tables(ctdse_geometry *G, const ctdse_geometry *src, TdseResident &R, ResidentJob &J)
+{
+    DevMem &mem = G->lattice ? G->lattice->res[R.chunk / 8 - 2] : G->res[R.chunk / 8 - 2];
+    if (!mem.p && build_resident(src, R.chunk, mem) != CTDSE_OK) return g_status;
+    const TdseGeom &D = G->dev;
+    const long long n = resident_entries(src->dev.nx, R.chunk);
+    R.gv = mem.as<double2>();
+    R.s = R.gv + n;
+    R.b = R.s + n;
+    R.chunks = (src->dev.nx + R.chunk - 1) / R.chunk;
+    const int off = (src->num_r - G->num_r) / 2;
+    R.chunk0 = off / R.chunk;
+    R.lead = off % R.chunk;
+    R.head = src != G ? std::min(D.nx, G->reach) : 0;
+    // the chunks around the atom: rows of <psi0|psi> (p0_lo > p0_hi: psi0 is zero) and of PopInt
+    const int lo = std::min(std::min(D.p0_lo, D.pint_lo), std::max(D.pint_hi, 0));
+    const int hi = std::max(D.p0_hi, D.pint_hi);
+    R.core_chunk0 = (lo + R.lead) / R.chunk;
+    R.core_chunks = (hi + R.lead) / R.chunk - R.core_chunk0 + 1;
+    J = ResidentJob{};
+    J.g = D.g;
+    J.ib = D.ib;
+    J.psi0 = G->psi0_nat.as<double2>();
+    J.nx = D.nx;
+    J.C = R.chunk;
+    J.first = R.core_chunk0 * R.chunk - R.lead;
+    J.n = R.core_chunks;
+    J.lo = D.pint_lo;
+    J.hi = D.pint_hi;
+    J.head = R.head;
+    J.warm = resident_warm(G->reach);
+    J.k36 = D.k36;
+    return CTDSE_OK;
+}
+
+// The plans of every geometry, in a batch and alone, and their tables (what each has for itself in one
+// allocation and one launch: two of each per geometry took 0.2 ms a geometry).
+int add_resident(const std::vector<ctdse_geometry *> &gs)
+{
+    // here and not at a launch, which may be captured
+    HIP_CHECK(hipFuncSetAttribute((const void *)tdse_window_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                  TDSE_ONE_WAVES * 64 * TDSE_RES_LDS * (int)sizeof(double2)));
+    std::map<const Lattice *, ctdse_geometry *> widest;
+    for (ctdse_geometry *G : gs)
+        if (G && G->lattice) {
+            ctdse_geometry *&w = widest[G->lattice.get()];
+            if (!w || G->num_r > w->num_r) w = G;
+        }
+    std::vector<ResidentJob> jobs;
+    std::vector<std::pair<ctdse_geometry *, TdseResident *>> plans;
+    for (ctdse_geometry *G : gs) {
+        if (!G || !G->dev.g) continue;
+        const ctdse_geometry *src = G->lattice ? widest[G->lattice.get()] : G;
+        plan_one(G->dev.nx, G->reach, G->dev.one);
+        if (plan_resident(G->dev.nx, G->reach, G->dev.res)) plans.push_back({G, &G->dev.res});
+        plans.push_back({G, &G->dev.one});
+        while (jobs.size() < plans.size()) {
+            jobs.emplace_back();
+            if (attach_tables(G, src, *plans[jobs.size() - 1].second, jobs.back()) != CTDSE_OK) return g_status;
+        }
+    }
+    if (jobs.empty()) return CTDSE_OK;
+    auto pool = std::make_shared<DevMem>();
+    size_t entries = 0;  // of 16 bytes
+    auto size_of = [](const ResidentJob &J) { return (size_t)(J.C * J.n + J.head + (J.C * J.n + 1) / 2); };
+    for (const ResidentJob &J : jobs) entries += size_of(J);
+    DevMem d_jobs;
+    HIP_CHECK(pool->alloc(entries * sizeof(double2)));
+    HIP_CHECK(d_jobs.alloc(jobs.size() * sizeof(ResidentJob)));
+    double2 *at = pool->as<double2>();
+    int most = 0;
+    for (size_t k = 0; k < jobs.size(); k++) {
+        ResidentJob &J = jobs[k];
+        TdseResident &R = *plans[k].second;
+        const int m = J.C * J.n;
+        J.core = at;
+        J.head_b = at + m;
+        J.im = reinterpret_cast<double *>(at + m + J.head);
+        at += size_of(J);
+        R.core = J.core;
+        R.core_im = plans[k].first->psi0_real ? nullptr : J.im;
+        R.head_b = J.head_b;
+        plans[k].first->core = pool;
+        most = std::max(most, std::max(m, J.head));
+    }
+    HIP_CHECK(hipMemcpy(d_jobs.p, jobs.data(), jobs.size() * sizeof(ResidentJob), hipMemcpyHostToDevice));
+    constexpr size_t kMostRows = 32768;  // grid rows of one launch
+    for (size_t k = 0; k < jobs.size(); k += kMostRows)
+        hipLaunchKernelGGL(tdse_resident_core_kernel, dim3((most + 255) / 256, (unsigned)std::min(kMostRows, jobs.size() - k)),
+                           dim3(256), 0, 0, d_jobs.as<ResidentJob>() + k);
+    HIP_CHECK(hipGetLastError());
+    HIP_CHECK(hipStreamSynchronize(nullptr));
+    return CTDSE_OK;
+}
+
 // Builds geometries: ground states of all that need one in grouped launches, then the
 // tables.  out[i] is null where status[i] is a hard failure; a ground state that did not
 // converge (CTDSE_ERR_GS_NOT_CONVERGED) still yields a geometry, as in the reference, which
@@ -567,7 +787,7 @@ int geometries_from(const std::vector<GeomSpec> &spec, std::vector<ctdse_geometr
             out[i] = nullptr;
         }
     }
-    if (n > 1 && share_lattices(out) != CTDSE_OK) {
+    if ((n > 1 && share_lattices(out) != CTDSE_OK) || add_resident(out) != CTDSE_OK) {
         for (int i = 0; i < n; i++) {
             delete out[i];
             out[i] = nullptr;
@@ -677,7 +897,10 @@ int pick_waves(int *min_out, int max_halo_lanes)
 // chunks) and resident workgroups per CU (the persistent grid is CUs * per_cu).
 struct LaunchShape {
     int nw = 4, per_cu = 3, steps = 1;
+    ctdse_launch_config config{4, 3, 1};  // what callers are told: of the streaming kernels
     bool stash = false;  // two-step passes keep 1/beta in LDS between their stages
+    bool resident = false;  // tdse_resident_kernel
+    size_t lds = 0;         // its dynamic LDS
 };
 
 // Dynamic LDS of tdse_propagate_pair_stash_kernel: two segments' 1/beta.
@@ -698,6 +921,33 @@ bool stash_fits(const LaunchShape &sh)
     return (size_t)sh.per_cu * (attr.sharedSizeBytes + stash_bytes(sh.nw)) <= (size_t)lds;
 }
 
+// The resident kernel's shape for a batch: the widest workgroup any geometry needs, as many per
+// CU as its waves (2 per SIMD) and LDS allow.
+int resident_shape(const std::vector<const ctdse_geometry *> &geoms, LaunchShape &sh)
+{
+    sh.resident = true;
+    sh.nw = 1;
+    for (const ctdse_geometry *g : geoms) {
+        const TdseResident &R = g->dev.res;
+        sh.nw = std::max(sh.nw, R.waves);
+        sh.lds = std::max(sh.lds, lane_lds(R));
+    }
+    hipFuncAttributes attr;
+    int dev = 0, lds = 0;
+    HIP_CHECK(hipFuncGetAttributes(&attr, (const void *)tdse_resident_kernel));
+    HIP_CHECK(hipGetDevice(&dev));
+    HIP_CHECK(hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerMultiprocessor, dev));
+    const int fit = (int)((size_t)lds / (attr.sharedSizeBytes + sh.lds));
+    sh.per_cu = std::max(1, std::min(4 * TDSE_RES_WAVES_PER_SIMD / sh.nw, fit));
+    // the most any batch asks for, so that plans of different sizes live side by side
+    HIP_CHECK(hipFuncSetAttribute((const void *)tdse_resident_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                  TDSE_MAX_WAVES * 64 * TDSE_RES_LDS * (int)sizeof(double2)));
+    return CTDSE_OK;
+}
+
+// The launch of a batch.  Without a launch shape from the caller or the environment: the resident
+// kernel, 2 to 3 x the streaming kernels' rate from 48 instances of 6001 points (24.8 ms against 71.2) to
+// 2048 of 16001 (500 steps: 409 ms against 838).  With one: the streaming kernels in that shape.
 int shape_for(const std::vector<const ctdse_geometry *> &geoms, const ctdse_launch_config *cfg, LaunchShape *out)
 {
     int min_nw = 1, max_h = 0;
@@ -719,6 +969,14 @@ int shape_for(const std::vector<const ctdse_geometry *> &geoms, const ctdse_laun
         sh.nw = cfg->waves_per_group;
         sh.per_cu = cfg->groups_per_cu;
         sh.steps = cfg->steps_per_pass;
+    }
+    sh.config = {sh.nw, sh.per_cu, sh.steps};
+    if (!cfg && !std::getenv("MMA_TDSE_STEPS_PER_PASS") && !std::getenv("MMA_TDSE_WAVES") &&
+        !std::getenv("MMA_TDSE_WG_PER_CU") &&
+        std::all_of(geoms.begin(), geoms.end(), [](const ctdse_geometry *g) { return g->dev.res.chunk > 0; })) {
+        if (resident_shape(geoms, sh) != CTDSE_OK) return g_status;
+        *out = sh;
+        return CTDSE_OK;
     }
     sh.stash = sh.steps == 2 && stash_fits(sh);
     if (sh.stash)  // outside any stream capture: plans and immediate runs call this first
@@ -765,6 +1023,7 @@ struct BatchHost {
     std::vector<int> order;
     TdseQueues queues{};
     long long stride = 0;
+    long long res_stride = 0;  // of the resident kernel: one state of its windows
 };
 
 int describe(const std::vector<InstSpec> &spec, BatchHost &B)
@@ -804,6 +1063,9 @@ int describe(const std::vector<InstSpec> &spec, BatchHost &B)
         I.n_snap = s.n_snap;
         I.psi_final = s.psi_final;
         B.stride = std::max(B.stride, s.geom->dev.npad);
+        const TdseResident &R = s.geom->dev.res;
+        if (R.chunk && R.windows > 1)
+            B.res_stride = std::max(B.res_stride, (((long long)(R.windows - 1) * R.stride + 64 * R.waves + 63) / 64) * 64 * R.chunk);
     }
     // largest instances first (longest-processing-time order for the atomic queues)
     std::vector<int> lpt(n);
@@ -850,6 +1112,13 @@ int grid_slots(int n, const LaunchShape &sh, int *slots)
 int enqueue_plan(const ctdse_batch_plan &P, double2 *work, hipStream_t stream)
 {
     hipLaunchKernelGGL(tdse_fill_int_kernel, dim3(1), dim3(64), 0, stream, P.d_counter.as<int>(), TDSE_QUEUES, 0);
+    if (P.shape.resident) {
+        hipLaunchKernelGGL(tdse_resident_kernel, dim3(P.slots), dim3(64 * P.shape.nw), P.shape.lds, stream,
+                           P.d_geom.as<TdseGeom>(), P.d_inst.as<TdseInst>(), P.d_order.as<int>(), P.queues,
+                           P.d_counter.as<int>(), work, P.stride);
+        HIP_CHECK(hipGetLastError());
+        return CTDSE_OK;
+    }
     const bool stash = P.shape.steps == 2 && P.shape.stash;
     hipLaunchKernelGGL(stash ? tdse_propagate_pair_stash_kernel
                              : (P.shape.steps == 2 ? tdse_propagate_pair_kernel : tdse_propagate_kernel),
@@ -858,6 +1127,13 @@ int enqueue_plan(const ctdse_batch_plan &P, double2 *work, hipStream_t stream)
                        P.d_counter.as<int>(), work, P.stride);
     HIP_CHECK(hipGetLastError());
     return CTDSE_OK;
+}
+
+// A launch's work buffer: one state per workgroup; the resident kernel needs two, and only for
+// grids of several windows.
+size_t work_bytes(const ctdse_batch_plan &P)
+{
+    return (size_t)P.slots * P.stride * sizeof(double2) * (P.shape.resident ? 2 : 1);
 }
 
 // Immediate path: descriptors copied on `stream`, the shared work buffer, and a wait.
@@ -870,12 +1146,12 @@ int propagate(const std::vector<InstSpec> &spec, hipStream_t stream, const ctdse
     ctdse_batch_plan P;
     P.n = n;
     P.queues = B.queues;
-    P.stride = B.stride;
     if (shape_for(B.geoms, cfg, &P.shape) != CTDSE_OK) return g_status;
     if (grid_slots(n, P.shape, &P.slots) != CTDSE_OK) return g_status;
+    P.stride = P.shape.resident ? B.res_stride : B.stride;
 
     std::lock_guard<std::mutex> lock(g_launch_mutex);
-    const size_t need = (size_t)P.slots * P.stride * sizeof(double2);
+    const size_t need = work_bytes(P);
     if (need > g_work_bytes) {
         HIP_CHECK(g_work.alloc(need));
         g_work_bytes = need;
@@ -892,17 +1168,6 @@ int propagate(const std::vector<InstSpec> &spec, hipStream_t stream, const ctdse
     return queued;
 }
 
-// Waves per workgroup of the step-parallel path (MMA_TDSE_PAR_WAVES overrides): segments of
-// nw*64 - 2H own chunks, one workgroup each, one launch per step.
-int par_waves(int halo_lanes)
-{
-    int nw = 4;
-    if (const char *env = std::getenv("MMA_TDSE_PAR_WAVES")) nw = std::atoi(env);
-    nw = std::max(1, std::min(TDSE_MAX_WAVES, nw));
-    while (nw < TDSE_MAX_WAVES && nw * 64 - 2 * halo_lanes < 64) nw++;
-    return nw * 64 - 2 * halo_lanes >= 64 ? nw : 0;
-}
-
 // Descriptors of a step-parallel run written on the device from kernel arguments, so the
 // run needs no host-to-device copy (and no staging memory).
 __global__ void tdse_put_desc_kernel(TdseGeom g, TdseInst inst, TdseGeom *g_out, TdseInst *inst_out)
@@ -913,25 +1178,16 @@ __global__ void tdse_put_desc_kernel(TdseGeom g, TdseInst inst, TdseGeom *g_out,
     }
 }
 
-// Launch shape of a step-parallel run of one instance (propagate_steps): waves per
-// workgroup and segments per step.  Returns CTDSE_ERR_UNSUPPORTED (status untouched) when the
-// descriptor needs the persistent path.
-int steps_shape(const InstSpec &s, int *nw_out, int *nseg_out)
+// Entries of one state of a window run (lane-tile order).
+long long window_state(const TdseResident &R, int nx)
 {
-    if (!s.geom || s.n_run != 0 || s.k0 != 0 || s.psi_init || s.save || s.pregated || !s.out || s.n_steps < 1)
-        return CTDSE_ERR_UNSUPPORTED;
-    const TdseGeom &g = s.geom->dev;
-    const int nw = par_waves(g.halo_lanes);
-    if (nw == 0) return CTDSE_ERR_UNSUPPORTED;
-    const int own = nw * 64 - 2 * g.halo_lanes;
-    *nw_out = nw;
-    *nseg_out = (g.nchunks + own - 1) / own;
-    return CTDSE_OK;
+    return (long long)(((nx + R.lead + R.chunk - 1) / R.chunk + 63) / 64) * 64 * R.chunk;
 }
+// Doubles of its partial sums.
+size_t window_sums(const TdseResident &R) { return 2 * (size_t)TDSE_RES_RING * R.windows * 5; }
 
-// Device buffers of a step-parallel run: the two descriptors, per-segment partial sums of
-// the observables (2 x nseg x 5 doubles), the gated field (n_steps + 1 doubles) and two
-// state vectors (npad complex doubles each).
+// Device buffers of a window run: the two descriptors, the windows' sums of the observables, the
+// gated field (n_steps + 1 doubles) and two states.
 struct StepBufs {
     TdseGeom *geom;
     TdseInst *inst;
@@ -940,11 +1196,12 @@ struct StepBufs {
     double2 *psi[2];
 };
 
-// Queues a step-parallel run into the given buffers: no allocation and no wait.  Every
-// buffer is (re)initialised here, so buffers left over from an earlier run may be reused.
-int enqueue_steps(const InstSpec &s, int nw, int nseg, const StepBufs &b, hipStream_t stream)
+// Queues a window run into the given buffers: no allocation and no wait.  Every buffer is written
+// here before it is read, so buffers left over from an earlier run may be reused.
+int enqueue_steps(const InstSpec &s, const StepBufs &b, hipStream_t stream)
 {
     const TdseGeom &g = s.geom->dev;
+    const TdseResident &R = g.one;
     BatchHost B;
     if (describe({s}, B) != CTDSE_OK) return g_status;
     const int n_field = s.n_steps + 1;
@@ -952,57 +1209,58 @@ int enqueue_steps(const InstSpec &s, int nw, int nseg, const StepBufs &b, hipStr
     inst.field = b.gated;
     inst.pregated = 1;
     hipLaunchKernelGGL(tdse_put_desc_kernel, dim3(1), dim3(64), 0, stream, g, inst, b.geom, b.inst);
-    // psi0 into the first buffer; the second one zeroed (by a kernel, not a memset node), its
-    // zero tiles and padding rows stay zero (the steps write own chunks only)
-    HIP_CHECK(hipMemcpyAsync(b.psi[0], g.psi0, (size_t)g.npad * sizeof(double2), hipMemcpyDeviceToDevice, stream));
-    const long long n_int = 4 * g.npad;
-    hipLaunchKernelGGL(tdse_fill_int_kernel, dim3((unsigned)((n_int + 255) / 256)), dim3(256), 0, stream,
-                       reinterpret_cast<int *>(b.psi[1]), (int)n_int, 0);
     hipLaunchKernelGGL(tdse_gate_kernel, dim3(1), dim3(256), 0, stream, s.field, n_field, b.gated);
+    const size_t lds = lane_lds(R);
     const dim3 untile_grid((g.nx + 255) / 256);
     const int n_snap = s.snap ? s.n_snap : 0, every = std::max(1, s.snap_every);
-    int i_snap = 0;
-    for (int k = 0; k < s.n_steps; k++) {
-        hipLaunchKernelGGL(tdse_parallel_step_kernel, dim3(nseg, 1), dim3(64 * nw), 0, stream, b.geom, b.inst, k,
-                           b.psi[k & 1], b.psi[(k + 1) & 1], (long long)g.npad, b.partial, nseg);
+    int i_snap = 0, launch = 0, prev = 0;
+    for (int k = 0; k < s.n_steps;) {
+        int nb = std::min(R.steps, s.n_steps - k);
         // prop.c:248-255: row i_snap gets psi after step k when k % every == 0
-        if (k % every == 0 && i_snap < n_snap - 1)
-            hipLaunchKernelGGL(tdse_untile_kernel, untile_grid, dim3(256), 0, stream, b.psi[(k + 1) & 1], g.nx,
-                               s.snap + (size_t)i_snap++ * 2 * g.nx);
+        const bool snaps = i_snap < n_snap - 1;
+        const int next = (k + every - 1) / every * every;  // the next such step
+        if (snaps) nb = std::min(nb, next + 1 - k);
+        hipLaunchKernelGGL(tdse_window_kernel, dim3(R.windows + 1), dim3(64 * R.waves), lds, stream, b.geom, b.inst, R, k, nb,
+                           prev, launch, launch ? b.psi[launch & 1] : nullptr, b.psi[(launch + 1) & 1], b.partial);
+        if (snaps && k + nb == next + 1)
+            hipLaunchKernelGGL(tdse_window_untile_kernel, untile_grid, dim3(256), 0, stream, b.psi[(launch + 1) & 1], R.chunk,
+                               R.lead, g.nx, s.snap + (size_t)i_snap++ * 2 * g.nx);
+        k += nb;
+        prev = nb;
+        launch++;
     }
     // prop.c:256-262: after the last step, the last row gets the final state if every earlier
     // row was used; the final state itself is optional output
-    const double2 *fin = b.psi[s.n_steps & 1];
+    const double2 *fin = b.psi[launch & 1];
     if (n_snap > 0 && i_snap == n_snap - 1)
-        hipLaunchKernelGGL(tdse_untile_kernel, untile_grid, dim3(256), 0, stream, fin, g.nx,
+        hipLaunchKernelGGL(tdse_window_untile_kernel, untile_grid, dim3(256), 0, stream, fin, R.chunk, R.lead, g.nx,
                            s.snap + (size_t)(n_snap - 1) * 2 * g.nx);
-    if (s.psi_final) hipLaunchKernelGGL(tdse_untile_kernel, untile_grid, dim3(256), 0, stream, fin, g.nx, s.psi_final);
-    hipLaunchKernelGGL(tdse_parallel_finish_kernel, dim3(1), dim3(64), 0, stream, b.inst, 1, b.partial, nseg);
+    if (s.psi_final)
+        hipLaunchKernelGGL(tdse_window_untile_kernel, untile_grid, dim3(256), 0, stream, fin, R.chunk, R.lead, g.nx,
+                           s.psi_final);
+    hipLaunchKernelGGL(tdse_window_finish_kernel, dim3(1), dim3(64), 0, stream, b.inst, R.windows, s.n_steps - prev, prev,
+                       launch - 1, b.partial);
     HIP_CHECK(hipGetLastError());
     return CTDSE_OK;
 }
 
-// One instance over its whole run with no partial runs or saved states: the segments of a
-// step are solved side by side (tdse_parallel_step_kernel, psi double-buffered), so a step
-// costs one segment's latency instead of nseg of them; snapshots and the final state are
-// copied out between steps.  Returns CTDSE_ERR_UNSUPPORTED (status untouched) when the
-// descriptor needs the persistent path.
+// One instance over its whole run with no partial runs or saved states: its windows are solved side
+// by side (tdse_window_kernel, psi double-buffered), several steps per launch; snapshots and the final
+// state are copied out between launches.
 int propagate_steps(const InstSpec &s, hipStream_t stream)
 {
-    int nw = 0, nseg = 0;
-    const int shaped = steps_shape(s, &nw, &nseg);
-    if (shaped != CTDSE_OK) return shaped;
     const TdseGeom &g = s.geom->dev;
+    const long long state = window_state(g.one, g.nx);
     DevMem states, partial, gated, d_geom, d_inst;
-    HIP_CHECK(states.alloc(2 * (size_t)g.npad * sizeof(double2)));
-    HIP_CHECK(partial.alloc(2 * (size_t)nseg * 5 * sizeof(double)));
+    HIP_CHECK(states.alloc(2 * (size_t)state * sizeof(double2)));
+    HIP_CHECK(partial.alloc(window_sums(g.one) * sizeof(double)));
     HIP_CHECK(gated.alloc((size_t)(s.n_steps + 1) * sizeof(double)));
     HIP_CHECK(d_geom.alloc(sizeof(TdseGeom)));
     HIP_CHECK(d_inst.alloc(sizeof(TdseInst)));
     const StepBufs b{d_geom.as<TdseGeom>(), d_inst.as<TdseInst>(), partial.as<double>(), gated.as<double>(),
-                     {states.as<double2>(), states.as<double2>() + g.npad}};
+                     {states.as<double2>(), states.as<double2>() + state}};
     std::lock_guard<std::mutex> lock(g_launch_mutex);
-    const int queued = enqueue_steps(s, nw, nseg, b, stream);
+    const int queued = enqueue_steps(s, b, stream);
     // wait before returning (also after a launch error): the buffers freed on return may
     // still be in use
     HIP_CHECK(hipStreamSynchronize(stream));
@@ -1042,10 +1300,10 @@ int make_plan(const std::vector<InstSpec> &spec, const ctdse_launch_config *cfg,
     if (describe(spec, B) != CTDSE_OK) return g_status;
     P.n = n;
     P.queues = B.queues;
-    P.stride = B.stride;
     if (shape_for(B.geoms, cfg, &P.shape) != CTDSE_OK) return g_status;
     if (grid_slots(std::max(n, 1), P.shape, &P.slots) != CTDSE_OK) return g_status;
-    HIP_CHECK(P.work.alloc((size_t)P.slots * P.stride * sizeof(double2)));
+    P.stride = P.shape.resident ? B.res_stride : B.stride;
+    HIP_CHECK(P.work.alloc(work_bytes(P)));
     HIP_CHECK(P.d_geom.alloc(B.gdev.size() * sizeof(TdseGeom)));
     HIP_CHECK(P.d_inst.alloc(B.insts.size() * sizeof(TdseInst)));
     HIP_CHECK(P.d_order.alloc(B.order.size() * sizeof(int)));
@@ -1266,10 +1524,7 @@ int ctdse_propagate_one(const ctdse_geometry *geom, int n_steps, const double *f
     s.n_steps = n_steps;
     s.field = field;
     s.out = out;
-    const int st = propagate_steps(s, (hipStream_t)stream);
-    if (st != CTDSE_ERR_UNSUPPORTED) return st;
-    const ctdse_launch_config single{TDSE_MAX_WAVES, 1, 1};
-    return propagate({s}, (hipStream_t)stream, &single);
+    return propagate_steps(s, (hipStream_t)stream);
 }
 
 int ctdse_propagate_one_noalloc(const ctdse_geometry *geom, int n_steps, const double *field, double *out,
@@ -1283,11 +1538,8 @@ int ctdse_propagate_one_noalloc(const ctdse_geometry *geom, int n_steps, const d
     s.n_steps = n_steps;
     s.field = field;
     s.out = out;
-    int nw = 0, nseg = 0;
-    if (steps_shape(s, &nw, &nseg) != CTDSE_OK)
-        return set_status(CTDSE_ERR_UNSUPPORTED, "the geometry's truncation halo leaves no room for the step-parallel "
-                                                 "solve, which is the only form without a work buffer");
     const TdseGeom &g = geom->dev;
+    const long long state = window_state(g.one, g.nx);
     // layout of the scratch array: descriptors, partial sums, gated field, two states
     size_t off = 0;
     const size_t o_geom = off;
@@ -1295,13 +1547,17 @@ int ctdse_propagate_one_noalloc(const ctdse_geometry *geom, int n_steps, const d
     const size_t o_inst = off;
     off += align256(sizeof(TdseInst));
     const size_t o_part = off;
-    off += align256(2 * (size_t)nseg * 5 * sizeof(double));
+    off += align256(window_sums(g.one) * sizeof(double));
     const size_t o_gated = off;
     off += align256((size_t)(n_steps + 1) * sizeof(double));
     const size_t o_psi = off;
-    off += 2 * (size_t)g.npad * sizeof(double2);
-    if (off > (size_t)CTDSE_NOALLOC_SCRATCH_BYTES)
-        return set_status(CTDSE_ERR_ARGUMENT, "ctdse_propagate_one_noalloc: this run needs " + std::to_string(off) +
+    off += 2 * (size_t)state * sizeof(double2);
+    // counted: two state vectors, the field, 512 bytes and 80 for every 256 chunks less a halo on each side
+    const int segment = 4 * TDSE_WAVE - 2 * g.halo_lanes;
+    const size_t counted = 512 + align256(80 * (size_t)((g.nchunks + segment - 1) / segment)) +
+                           align256((size_t)(n_steps + 1) * sizeof(double)) + 2 * (size_t)g.npad * sizeof(double2);
+    if (counted > (size_t)CTDSE_NOALLOC_SCRATCH_BYTES || off > kScratchBytes)
+        return set_status(CTDSE_ERR_ARGUMENT, "ctdse_propagate_one_noalloc: this run needs " + std::to_string(counted) +
                                                   " bytes of scratch (two states of " + std::to_string(g.npad) +
                                                   " complex doubles, " + std::to_string(n_steps + 1) +
                                                   " field samples), more than the " +
@@ -1312,9 +1568,9 @@ int ctdse_propagate_one_noalloc(const ctdse_geometry *geom, int n_steps, const d
     double2 *psi = reinterpret_cast<double2 *>(p + o_psi);
     const StepBufs b{reinterpret_cast<TdseGeom *>(p + o_geom), reinterpret_cast<TdseInst *>(p + o_inst),
                      reinterpret_cast<double *>(p + o_part), reinterpret_cast<double *>(p + o_gated),
-                     {psi, psi + g.npad}};
+                     {psi, psi + state}};
     std::lock_guard<std::mutex> lock(g_launch_mutex);
-    return enqueue_steps(s, nw, nseg, b, (hipStream_t)stream);
+    return enqueue_steps(s, b, (hipStream_t)stream);
 }
 
 int ctdse_geometry_create_batch(int n, const int *num_r, const double *dx, const double *dt, const double *a,
@@ -1347,9 +1603,7 @@ int ctdse_launch_config_default(int n_inst, const ctdse_geometry *const *geom, c
     }
     LaunchShape sh;
     if (shape_for(gs, nullptr, &sh) != CTDSE_OK) return g_status;
-    cfg->waves_per_group = sh.nw;
-    cfg->groups_per_cu = sh.per_cu;
-    cfg->steps_per_pass = sh.steps;
+    *cfg = sh.config;
     return CTDSE_OK;
 }
 
@@ -1419,11 +1673,7 @@ int ctdse_batch_plan_info(const ctdse_batch_plan *plan, ctdse_launch_config *con
 {
     clear_status();
     if (!plan) return set_status(CTDSE_ERR_ARGUMENT, "null plan");
-    if (config) {
-        config->waves_per_group = plan->shape.nw;
-        config->groups_per_cu = plan->shape.per_cu;
-        config->steps_per_pass = plan->shape.steps;
-    }
+    if (config) *config = plan->shape.config;
     if (workgroups) *workgroups = plan->slots;
     return CTDSE_OK;
 }
@@ -1677,13 +1927,9 @@ void call1DTDSE(inputs_def *inputs, outputs_def *outputs)
         s.snap_every = spd;
         s.n_snap = n_snap;
     }
-    // one instance alone: its segments run side by side, one launch per step; where that
-    // path cannot run, the persistent kernel with the widest segments (8 waves: the fewest
-    // serial segments per step, 145 ms against 178 ms with 4 waves for 4416 steps of 16001
-    // points)
-    const ctdse_launch_config single{TDSE_MAX_WAVES, 1, 1};
-    st = std::getenv("MMA_TDSE_NO_STEP_PARALLEL") ? (int)CTDSE_ERR_UNSUPPORTED : propagate_steps(s, 0);
-    if (st == CTDSE_ERR_UNSUPPORTED) st = propagate({s}, 0, &single);
+    // one instance alone: its windows run side by side (MMA_TDSE_NO_STEP_PARALLEL: one after the other
+    // in one workgroup, as in a batch)
+    st = std::getenv("MMA_TDSE_NO_STEP_PARALLEL") ? propagate({s}, 0) : propagate_steps(s, 0);
     if (st != CTDSE_OK) return;
     hipLaunchKernelGGL(tdse_tgrid_kernel, dim3(1), dim3(64), 0, 0, tgrid.as<double>(), nt_out, in.tmin, dt);
 

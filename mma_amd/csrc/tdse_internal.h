@@ -26,6 +26,11 @@
 #define TDSE_ADJ_WAVES_PER_CU 8    // adjoint kernel: 2 waves per SIMD (224 VGPRs)
 #define TDSE_REV_WAVES_PER_SIMD 2  // reconstructing adjoint kernel: 256-VGPR budget, 8 waves per CU
 #define TDSE_MAX_HALO 40           // largest truncation depth in chunks
+#define TDSE_RES_WAVES_PER_SIMD 2  // resident propagation kernel: 256-VGPR budget, 8 waves per CU
+#define TDSE_RES_LDS 19            // its points per lane whose factor sits in LDS
+#define TDSE_RES_RING 16           // its steps between two writes of observables
+#define TDSE_RES_GROUP 4           // points per thread of its table builders
+#define TDSE_ONE_WAVES 4           // waves per window of one instance alone (one per SIMD)
 
 // Instance queues of a persistent propagation launch, one per XCD: queue q holds
 // order[off[q] .. off[q + 1]).  A workgroup takes instances from the queue of the XCD it runs
@@ -46,6 +51,27 @@ __host__ __device__ inline long long tdse_index(long long j)
 
 // number of elements of a tiled array for nchunks chunks (with the two zero tiles)
 __host__ __device__ inline long long tdse_tiled_size(long long nchunks) { return ((nchunks + 63) / 64 + 2) * TDSE_TILE; }
+
+// How the resident kernel (tdse_resident.hip) covers a grid: lanes of `chunk` consecutive points,
+// `waves` waves, `windows` overlapping windows of that size every `stride` chunks, `steps` steps
+// between a window's load and store.  Its tables lie in tiles of 64 chunks, row i of a chunk 64
+// entries after row i - 1, for the whole lattice when the geometry shares one: the grid starts
+// `lead` points into table chunk chunk0.
+struct TdseResident {
+    const double2 *gv;    // {g_j, V'(x_j)}
+    const double2 *s;     // 1 / (1 + i g_j)
+    const double2 *b;     // (1 + i g_j) / beta_j
+    int chunk;            // points per lane (0: this kernel does not serve the geometry)
+    int waves, windows, steps;
+    int stride, halo;     // chunks: from window to window, and not owned at an inner edge
+    int lead, chunk0, chunks;  // chunks: table chunks before the first zero one
+    const double2 *core;  // {Re psi0, 1 in the PopInt window}: row i of core_chunks chunks per point of a chunk
+    const double *core_im;  // Im psi0 likewise, null where it is 0
+    int core_chunk0, core_chunks;
+    const double2 *head_b;  // b of the leading `head` points, which feel the geometry's own left wall
+    int head;
+    int reach;            // points after which a carry is below 1e-17
+};
 
 // Step-independent tables of one geometry (num_r, dx, dt, a, x_int), device pointers.
 // The Crank-Nicolson system of one step, scaled by 12, is
@@ -82,6 +108,8 @@ struct TdseGeom {
     const double2 *sib;
     const double2 *schq, *schg;  // the lattice's chunk transfer maps at shared chunk k + 64
     int s_off, head_chunks;
+    TdseResident res;  // in a batch
+    TdseResident one;  // alone: small windows side by side
 };
 
 // One instance of a batch.
@@ -150,6 +178,18 @@ struct TableJob {
     double *pivot_work;     // 2 (num_r + 1) scratch (natural-order 1/beta)
     double rho_fwd, rho_bwd, pint0;
     int pint_lo, pint_hi, p0_lo, p0_hi;
+    int psi0_real;          // Im psi0 = 0 at every point
+};
+
+// The tables of the resident kernel that a geometry has for itself (tdse_resident_core_kernel).
+struct ResidentJob {
+    const double *g;        // tiled
+    const double2 *ib;      // tiled
+    const double2 *psi0;    // natural order
+    int nx, C, first, n, lo, hi, head, warm;
+    double k36;
+    double2 *core, *head_b;
+    double *im;
 };
 
 // kernels (defined in the .hip files)
@@ -173,10 +213,15 @@ __global__ void tdse_propagate_pair_kernel(const TdseGeom *geoms, const TdseInst
 __global__ void tdse_propagate_pair_stash_kernel(const TdseGeom *geoms, const TdseInst *insts, const int *order,
                                                  TdseQueues queues, int *counter, double2 *work,
                                                  long long work_stride);
-__global__ void tdse_untile_kernel(const double2 *psi, int nx, double *row);
-__global__ void tdse_parallel_step_kernel(const TdseGeom *geom, const TdseInst *insts, int k, const double2 *psi_in,
-                                          double2 *psi_out, long long state_stride, double *partial, int nseg);
-__global__ void tdse_parallel_finish_kernel(const TdseInst *insts, int n_inst, const double *partial, int nseg);
+__global__ void tdse_resident_kernel(const TdseGeom *geoms, const TdseInst *insts, const int *order,
+                                     TdseQueues queues, int *counter, double2 *work, long long work_stride);
+__global__ void tdse_resident_tables_kernel(const double *g, const double *dpot, const double2 *ib, int nx, double k36, int C,
+                                            int chunks, int warm, double2 *gv, double2 *s, double2 *b);
+__global__ void tdse_window_kernel(const TdseGeom *geom, const TdseInst *inst, TdseResident R, int k, int nb, int nb_prev,
+                                   int launch, const double2 *src, double2 *dst, double *part);
+__global__ void tdse_window_finish_kernel(const TdseInst *inst, int windows, int k, int nb, int launch, const double *part);
+__global__ void tdse_window_untile_kernel(const double2 *psi, int C, int lead, int nx, double *dst);
+__global__ void tdse_resident_core_kernel(const ResidentJob *jobs);
 __global__ void tdse_gate_kernel(const double *f, int n, double *F);
 __global__ void tdse_adjoint_kernel(const TdseGeom *geoms, const TdseAdjInst *insts, const int *order, int n_inst,
                                     int *counter);

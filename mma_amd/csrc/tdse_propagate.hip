@@ -31,9 +31,8 @@
 //
 // Also here: the two-step pass (tdse_propagate_pair_kernel: segment s of step k kept in
 // registers while segment s-1 of step k+1 is solved from them; the stash form keeps 1/beta in
-// LDS between the two), and the step-parallel form for one instance alone
-// (tdse_parallel_step_kernel: every segment a workgroup of its own, halo on both sides, one
-// launch per step).
+// LDS between the two).  These kernels run where a launch shape is given; the library's own choice is
+// tdse_resident.hip, which keeps psi on the chip.
 #include "tdse_internal.h"
 #include "tdse_wave.h"
 
@@ -205,10 +204,7 @@ struct PairLds {
 //            wave-edge points published in LDS (first step of a pair);
 //   kFromRegs: psi_{k+1} from R (own chunks) and LDS (halo chunks, wave-edge neighbours),
 //            psi_{k+2} stored to HBM (second step of a pair).
-//   kParallel: one step of one segment whose window carries a halo on both sides (both
-//            recurrences truncated), so that all segments of a step are independent; psi_k
-//            from `psi`, psi_{k+1} of the own chunks to `psi_out`.
-enum SegMode { kSingle = 0, kKeep = 1, kFromRegs = 2, kParallel = 3 };
+enum SegMode { kSingle = 0, kKeep = 1, kFromRegs = 2 };
 
 // Solve one segment of one step with all waves of the workgroup.
 // observe: add the observables of the state the step starts from (psi_k, read for the
@@ -224,12 +220,10 @@ template <int MODE, bool STASH = false>
 __device__ void solve_segment(const TdseGeom &G, int seg, int own_chunks, int wave, int lane, int nw,
                               double2 *__restrict__ psi, double2 e0, double2 rot, bool observe, Acc &acc,
                               double2 (*slot_f)[2], double2 (*slot_b)[2], const double2 *edge_in, double2 *edge_out,
-                              double2 (&R)[C], PairLds *pl, double2 *__restrict__ psi_out = nullptr,
-                              double2 *stash = nullptr)
+                              double2 (&R)[C], PairLds *pl, double2 *stash = nullptr)
 {
     const int gl = wave * 64 + lane;                 // lane index in the workgroup
-    // first chunk of the window: the first own chunk, or H chunks before it (kParallel)
-    const int cs = MODE == kParallel ? seg * own_chunks - G.halo_lanes : seg * own_chunks;
+    const int cs = seg * own_chunks;  // first own chunk
     // live waves: those with a lane on the grid (chunks past the grid are zero padding and
     // carry the zero map, so dropping whole waves of them changes nothing)
     const int nwl = min(nw, (G.nchunks - cs + 63) >> 6);
@@ -265,8 +259,8 @@ __device__ void solve_segment(const TdseGeom &G, int seg, int own_chunks, int wa
     if constexpr (MODE != kFromRegs) {
 #pragma unroll
         for (int i = 0; i < C; i++) P[i] = ld2(psi, base + 64 * i);
-        if (lane == 0 && (gl > 0 || MODE == kParallel))
-            nb = ld2(psi, tdse_chunk_base(c - 1) + 64 * (C - 1));  // not yet overwritten (chunk -1..-41: zero)
+        if (lane == 0 && gl > 0)
+            nb = ld2(psi, tdse_chunk_base(c - 1) + 64 * (C - 1));  // not yet overwritten
         if (lane == 63 && gl < nl - 1) nb = ld2(psi, tdse_chunk_base(min(c + 1, G.nchunks)));
     } else {
         // own chunks: the previous stage's registers; halo chunks: its successor's first H
@@ -285,9 +279,7 @@ __device__ void solve_segment(const TdseGeom &G, int seg, int own_chunks, int wa
         }
     }
     __builtin_amdgcn_s_setprio(0);
-    const bool own = MODE == kParallel
-                         ? gl >= G.halo_lanes && gl < G.halo_lanes + own_chunks && c >= 0 && c < G.nchunks
-                         : gl < own_chunks && c < G.nchunks;
+    const bool own = gl < own_chunks && c < G.nchunks;
     const int j0 = c * C;
     // observables of the state this step starts from (psi_k)
     if (observe) observe_chunk(G, P, T.dp, base, j0, own, acc);
@@ -295,7 +287,7 @@ __device__ void solve_segment(const TdseGeom &G, int seg, int own_chunks, int wa
     const double(&Gv)[C] = T.Gv;
     const double2 Qc = T.Qc, Gc = T.Gc;
     double gL = T.gL, gR = T.gR;
-    if (MODE != kParallel && gl == own_chunks - 1) edge_out[0] = P[C - 1];  // the next segment's left neighbour
+    if (gl == own_chunks - 1) edge_out[0] = P[C - 1];  // the next segment's left neighbour
     // neighbours across the chunk edges: shuffles inside a wave, loads across waves, LDS for
     // the point left of the window, zero past the window's right end
     {
@@ -304,11 +296,10 @@ __device__ void solve_segment(const TdseGeom &G, int seg, int own_chunks, int wa
         gR = lane == 63 ? gR : gRd;
     }
     double2 left = dpp2_z<kWaveShr1>(P[C - 1]), right = dpp2_z<kWaveShl1>(P[0]);
-    if (lane == 0) left = (gl > 0 || MODE == kParallel) ? nb : (seg > 0 ? edge_in[0] : zero2);
+    if (lane == 0) left = gl > 0 ? nb : (seg > 0 ? edge_in[0] : zero2);
     if (lane == 63) right = nb;
-    // the forward recurrence enters exactly from the previous segment, or from zero H chunks
-    // before the own chunks (kParallel: truncated like the backward one)
-    const double2 z_in = (MODE != kParallel && seg > 0) ? edge_in[1] : zero2;
+    // the forward recurrence enters exactly from the previous segment
+    const double2 z_in = seg > 0 ? edge_in[1] : zero2;
 
     // r' = (M2' - i H') psi
     cn_rhs(P, Gv, left, right, gL, gR, G.k36);
@@ -334,7 +325,7 @@ __device__ void solve_segment(const TdseGeom &G, int seg, int own_chunks, int wa
             z = cmul(make_double2(tr, ti), IB[i]);
             P[i] = z;
         }
-        if (MODE != kParallel && gl == own_chunks - 1) edge_out[1] = z;  // the next segment's forward carry
+        if (gl == own_chunks - 1) edge_out[1] = z;  // the next segment's forward carry
     }
 
     // backward recurrence u_j = z_j + h_j u_{j+1},  h_j = -(1 + i g_{j+1}) ib_j
@@ -376,10 +367,9 @@ __device__ void solve_segment(const TdseGeom &G, int seg, int own_chunks, int wa
         if (lane == 0) pl->bnd[par][wave][0] = R[0];
         if (lane == 63) pl->bnd[par][wave][1] = R[C - 1];
     } else {
-        double2 *dst = MODE == kParallel ? psi_out : psi;
 #pragma unroll
         for (int i = 0; i < C; i++) {
-            st2(dst, base + 64 * i, cmul(e, P[i]));
+            st2(psi, base + 64 * i, cmul(e, P[i]));
             e = cmul(e, rot);
         }
     }
@@ -474,31 +464,6 @@ __device__ inline StepPhase step_phase(const TdseGeom &G, double F, int wave, in
 // LDS) and stored.  psi then streams through HBM once per two steps.
 // States saved for partial runs and snapshots are copied from the finished state between
 // steps (they are rare), so the segment solve carries no extra stores.
-// The XCD this wave runs on (hardware register XCC_ID, bits 3:0).
-__device__ inline int xcd_id()
-{
-    unsigned v;
-    asm volatile("s_getreg_b32 %0, hwreg(HW_REG_XCC_ID)" : "=s"(v));
-    return (int)(v & 15u);
-}
-
-// Next instance of the launch for this workgroup (thread 0 only): from the queue of this XCD
-// first, then the others in turn; tried (LDS) counts the queues found drained so far.  -1 when
-// every queue is drained: a queue is left only after its counter passed its length, so once
-// every workgroup has left every queue, each instance was taken exactly once.
-__device__ inline int next_instance(const TdseQueues &qs, int *counter, int &tried)
-{
-    const int q0 = xcd_id() % TDSE_QUEUES;
-    for (; tried < TDSE_QUEUES; tried++) {
-        const int q = (q0 + tried) % TDSE_QUEUES;
-        const int len = qs.off[q + 1] - qs.off[q];
-        if (len == 0) continue;
-        const int t = atomicAdd(counter + q, 1);
-        if (t < len) return qs.off[q] + t;
-    }
-    return -1;
-}
-
 template <bool PAIR, bool STASH = false>
 __device__ void propagate_loop(const TdseGeom *__restrict__ geoms, const TdseInst *__restrict__ insts,
                                const int *__restrict__ order, const TdseQueues &queues, int *counter, double2 *work,
@@ -570,11 +535,11 @@ __device__ void propagate_loop(const TdseGeom *__restrict__ geoms, const TdseIns
                         if (s & 1)
                             solve_segment<kKeep, STASH>(G, s, own_chunks, wave, lane, nw, buf, e0, ph0.rot, observe0,
                                                         acc0, slot_f, slot_b, edge[s & 1], edge[(s + 1) & 1], R1, pl,
-                                                        nullptr, st);
+                                                        st);
                         else
                             solve_segment<kKeep, STASH>(G, s, own_chunks, wave, lane, nw, buf, e0, ph0.rot, observe0,
                                                         acc0, slot_f, slot_b, edge[s & 1], edge[(s + 1) & 1], R0, pl,
-                                                        nullptr, st);
+                                                        st);
                         e0 = cmul(e0, ph0.r_seg);
                     }
                     lds_barrier();  // the halo and wave-edge points of segment s are in LDS
@@ -584,11 +549,11 @@ __device__ void propagate_loop(const TdseGeom *__restrict__ geoms, const TdseIns
                         if (sb & 1)
                             solve_segment<kFromRegs, STASH>(G, sb, own_chunks, wave, lane, nw, buf, e1, ph1.rot, true,
                                                             acc1, slot_f, slot_b, edge_b[sb & 1],
-                                                            edge_b[(sb + 1) & 1], R1, pl, nullptr, st);
+                                                            edge_b[(sb + 1) & 1], R1, pl, st);
                         else
                             solve_segment<kFromRegs, STASH>(G, sb, own_chunks, wave, lane, nw, buf, e1, ph1.rot, true,
                                                             acc1, slot_f, slot_b, edge_b[sb & 1],
-                                                            edge_b[(sb + 1) & 1], R0, pl, nullptr, st);
+                                                            edge_b[(sb + 1) & 1], R0, pl, st);
                         e1 = cmul(e1, ph1.r_seg);
                     }
                 }
@@ -670,25 +635,6 @@ __device__ void propagate_loop(const TdseGeom *__restrict__ geoms, const TdseIns
     }
 }
 
-// Entry idx of the outputs from the per-segment partial sums of a step-parallel run, added in
-// segment order; F is the gated field of the step that produced the state.  One thread.
-__device__ inline void store_partials(const TdseInst &I, const double *parts, int nseg, int idx, double F)
-{
-    double s0 = 0, s1 = 0, s2 = 0, s3 = 0, s4 = 0;
-    for (int q = 0; q < nseg; q++) {
-        s0 += parts[5 * q + 0];
-        s1 += parts[5 * q + 1];
-        s2 += parts[5 * q + 2];
-        s3 += parts[5 * q + 3];
-        s4 += parts[5 * q + 4];
-    }
-    I.src[idx] = -s4 + F;
-    I.ptot[idx] = s0 * s0 + s1 * s1;
-    I.pint[idx] = s2;
-    I.expv[idx] = s3;
-    if (I.efield) I.efield[idx] = F;
-}
-
 } // namespace
 
 // One time step per pass over psi (168-VGPR budget, 12 waves per CU).
@@ -719,73 +665,6 @@ tdse_propagate_pair_stash_kernel(const TdseGeom *__restrict__ geoms, const TdseI
     __shared__ PairLds pl;
     extern __shared__ double2 stash[];
     propagate_loop<true, true>(geoms, insts, order, queues, counter, work, work_stride, &pl, stash);
-}
-
-// One time step k of instance blockIdx.y, split over independent segments (blockIdx.x) whose
-// windows carry a halo on both sides: psi_k from psi_in, psi_{k+1} to psi_out (the caller
-// alternates the two).  The field is the gated one (I.field[k] = F_k).  The observables of
-// psi_k (k >= 1) go to partial[k & 1][instance][segment]; the next launch sums those of
-// entry k - 1 in segment order (tdse_parallel_finish_kernel the last).  For one instance
-// alone this runs a step in the time of one segment instead of all of them in turn.
-__global__ void __launch_bounds__(64 * TDSE_MAX_WAVES, TDSE_WAVES_PER_SIMD)
-tdse_parallel_step_kernel(const TdseGeom *__restrict__ geom, const TdseInst *__restrict__ insts, int k,
-                          const double2 *psi_in, double2 *psi_out, long long state_stride, double *partial, int nseg)
-{
-    __shared__ double part[TDSE_MAX_WAVES][5];
-    __shared__ double2 slot_f[TDSE_MAX_WAVES][2], slot_b[TDSE_MAX_WAVES][2];
-    const int nw = blockDim.x >> 6;
-    const int wave = threadIdx.x >> 6;
-    const int lane = threadIdx.x & 63;
-    const int inst = blockIdx.y, seg = blockIdx.x, n_inst = gridDim.y;
-    const TdseInst &I = insts[inst];
-    const TdseGeom &G = *geom;
-    const int own_chunks = nw * 64 - 2 * G.halo_lanes;  // host guarantees >= 64
-    if (seg == 0 && threadIdx.x == 0 && I.src) {
-        if (k == 0) {
-            I.src[0] = 0.0;
-            I.ptot[0] = 1.0;
-            I.pint[0] = G.pint0;
-            I.expv[0] = 0.0;
-            if (I.efield) I.efield[0] = 0.0;
-        } else if (k >= 2) {
-            store_partials(I, partial + ((long long)((k - 1) & 1) * n_inst + inst) * nseg * 5, nseg, k - 1,
-                           I.field[k - 2]);
-        }
-    }
-    const double F = I.field[k];
-    const double Fdt = F * G.dt;
-    double2 rot, e0;
-    sincos(Fdt * G.dx, &rot.y, &rot.x);
-    const int c = seg * own_chunks - G.halo_lanes + wave * 64 + lane;  // this lane's chunk
-    sincos(Fdt * grid_x(c * C, G.dx, G.xmax), &e0.y, &e0.x);
-    Acc acc = {0.0, 0.0, 0.0, 0.0, 0.0};
-    double2 R[C];  // unused by this mode
-    solve_segment<kParallel>(G, seg, own_chunks, wave, lane, nw,
-                             const_cast<double2 *>(psi_in) + (long long)inst * state_stride, e0, rot, k >= 1, acc,
-                             slot_f, slot_b, nullptr, nullptr, R, nullptr,
-                             psi_out + (long long)inst * state_stride);
-    wave_observables(acc, wave, lane, part);
-    __syncthreads();
-    if (threadIdx.x == 0 && k >= 1) {
-        double *dst = partial + (((long long)(k & 1) * n_inst + inst) * nseg + seg) * 5;
-        for (int q = 0; q < 5; q++) {
-            double sum = 0.0;
-            for (int w = 0; w < nw; w++) sum += part[w][q];
-            dst[q] = sum;
-        }
-    }
-}
-
-// The last observed entry (n_steps - 1) of a step-parallel run: one thread per instance.
-__global__ void tdse_parallel_finish_kernel(const TdseInst *insts, int n_inst, const double *partial, int nseg)
-{
-    const int inst = blockIdx.x * blockDim.x + threadIdx.x;
-    if (inst >= n_inst) return;
-    const TdseInst &I = insts[inst];
-    const int last = I.n_steps - 1;
-    if (!I.src || last < 1) return;
-    store_partials(I, partial + ((long long)(last & 1) * n_inst + inst) * nseg * 5, nseg, last,
-                   last >= 1 ? I.field[last - 1] : 0.0);
 }
 
 // The gated field of prop.c:125-134: F_k = 0 up to and including the first k with

@@ -286,7 +286,9 @@ __host__ __device__ void pivot_scan(TableJob &J)
     // CV = 1e-12, 5e-25 after the 6 of CV = 1e-25): a window that kept the plateau would cover
     // the whole grid and make every step read psi0 at every point.
     int lo = nx, hi = -1;
+    bool real = true;
     for (int j = 0; j < nx; j++) {
+        real = real && J.psi0_nat[2 * j + 1] == 0.0;
         const double v = J.psi0_nat[2 * j] * J.psi0_nat[2 * j] + J.psi0_nat[2 * j + 1] * J.psi0_nat[2 * j + 1];
         if (v > 1e-32 * mx) {
             if (j < lo) lo = j;
@@ -295,6 +297,7 @@ __host__ __device__ void pivot_scan(TableJob &J)
     }
     J.p0_lo = lo;
     J.p0_hi = hi;
+    J.psi0_real = real;
 }
 
 } // namespace
@@ -405,16 +408,6 @@ __global__ void tdse_xgrid_kernel(double *x, int num_r, double dx)
     if (k > num_r) return;
     const double half_span = 0.5 * num_r * dx;
     x[k] = (double)k * dx - half_span;
-}
-
-// A tiled state in natural order, interleaved re, im (a snapshot row of prop.c:248-263)
-__global__ void tdse_untile_kernel(const double2 *psi, int nx, double *row)
-{
-    const int j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= nx) return;
-    const double2 v = psi[tdse_index(j)];
-    row[2 * j] = v.x;
-    row[2 * j + 1] = v.y;
 }
 
 __global__ void tdse_fill_int_kernel(int *p, int n, int v)

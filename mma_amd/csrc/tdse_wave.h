@@ -248,4 +248,29 @@ __device__ inline double2 block_carry(double2 Qi, double2 zi, int wave, int lane
     return make_double2(ze.x + Qe.x * Z.x - Qe.y * Z.y, ze.y + Qe.x * Z.y + Qe.y * Z.x);
 }
 
+// The XCD this wave runs on (hardware register XCC_ID, bits 3:0).
+__device__ inline int xcd_id()
+{
+    unsigned v;
+    asm volatile("s_getreg_b32 %0, hwreg(HW_REG_XCC_ID)" : "=s"(v));
+    return (int)(v & 15u);
+}
+
+// Next instance of the launch for this workgroup (thread 0 only): from the queue of this XCD
+// first, then the others in turn; tried (LDS) counts the queues found drained so far.  -1 when
+// every queue is drained: a queue is left only after its counter passed its length, so once
+// every workgroup has left every queue, each instance was taken exactly once.
+__device__ inline int next_instance(const TdseQueues &qs, int *counter, int &tried)
+{
+    const int q0 = xcd_id() % TDSE_QUEUES;
+    for (; tried < TDSE_QUEUES; tried++) {
+        const int q = (q0 + tried) % TDSE_QUEUES;
+        const int len = qs.off[q + 1] - qs.off[q];
+        if (len == 0) continue;
+        const int t = atomicAdd(counter + q, 1);
+        if (t < len) return qs.off[q] + t;
+    }
+    return -1;
+}
+
 } // namespace tdse

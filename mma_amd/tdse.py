@@ -21,13 +21,17 @@ OUTPUT_ROWS = ("sourceterm", "PopTot", "PopInt", "expval", "Efield")
 
 
 class LaunchConfig(ctypes.Structure):
-    """Launch shape of the persistent propagation kernel (ctdse_launch_config): waves per
+    """Launch shape of the streaming propagation kernels (ctdse_launch_config): waves per
     workgroup (a segment of the parallel solve is 64 * waves_per_group chunks of 8 points),
-    resident workgroups per compute unit, and time steps per pass over the state (1 or 2)."""
+    resident workgroups per compute unit, and time steps per pass over the state (1 or 2).
+    library_choice: the library's own launch instead, which keeps the states on the chip where
+    it can (as a config of BatchPlan it is the same as None); its three numbers are those of
+    the streaming kernels' default."""
     _fields_ = [("waves_per_group", c_int), ("groups_per_cu", c_int), ("steps_per_pass", c_int)]
 
     def __init__(self, waves_per_group=4, groups_per_cu=3, steps_per_pass=1):
         super().__init__(int(waves_per_group), int(groups_per_cu), int(steps_per_pass))
+        self.library_choice = False
 
     def as_tuple(self):
         return (self.waves_per_group, self.groups_per_cu, self.steps_per_pass)
@@ -283,6 +287,8 @@ class BatchPlan:
         cfg = None
         if config is not None:
             cfg = config if isinstance(config, LaunchConfig) else LaunchConfig(*[int(v) for v in config])
+            if cfg.library_choice:
+                cfg = None
         self._p = c_void_p()
         _raise(_lib().ctdse_batch_plan_create(n_inst, handles, (c_int * n_inst)(*n_steps), c_void_p(fields.data_ptr()),
                                               field_off, c_void_p(out.data_ptr()), out_off, width,
@@ -290,6 +296,7 @@ class BatchPlan:
         info = LaunchConfig()
         wg = c_int()
         _raise(_lib().ctdse_batch_plan_info(self._p, byref(info), byref(wg)))
+        info.library_choice = cfg is None
         self.config, self.workgroups = info, wg.value
         self.pt_steps = sum(int(g.num_r + 1) * s for g, s in zip(geoms, n_steps))
 
@@ -317,9 +324,10 @@ class BatchPlan:
 
 
 def default_config(geometries):
-    """The launch shape ctdse_propagate_batch picks for these geometries."""
+    """The launch ctdse_propagate_batch picks for these geometries."""
     n = len(geometries)
     cfg = LaunchConfig()
+    cfg.library_choice = True
     _raise(_lib().ctdse_launch_config_default(n, (c_void_p * n)(*[g.handle.value for g in geometries]), byref(cfg)))
     return cfg
 
@@ -329,7 +337,8 @@ def propagate_stepwise(geometry, fields, out=None, stream=None):
     one kernel launch per time step over the whole batch, each instance's state held in HBM
     between launches and stepped in place (ctdse_propagate_states).  Same arguments and
     result as propagate_batch for a uniform batch (n_steps = L - 1 for every row), bit for
-    bit: the same segment solve and observable order run either way."""
+    bit up to 16384 grid points: the same solve and observable order run either way.  Larger
+    grids are solved in windows of several steps, so there the two agree to rounding."""
     from .adjoint import gate
     _check_device(fields, "fields")
     L = _lib()
@@ -361,7 +370,7 @@ def propagate_stepwise(geometry, fields, out=None, stream=None):
 
 def propagate_one(geometry, field, n_steps=None, out=None, stream=None):
     """One instance alone (ctdse_propagate_one): the propagation call1DTDSE runs, with the
-    segments of each step side by side.  field: device float64 samples (at least n_steps + 1;
+    grid's windows side by side.  field: device float64 samples (at least n_steps + 1;
     default n_steps = len(field) - 1); returns out, (5, n_steps) rows as propagate_batch's.
     Equal to propagate_batch's row to rounding, not bitwise."""
     field = field.reshape(-1)
