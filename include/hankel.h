@@ -105,6 +105,16 @@ typedef struct {
  * (Nr_FF, No) orientation of Hankel_long's results).  n_out <= 4 unless per_plane. */
 int hk_direct(const hk_planes *p, int n_out, const double *weights, int per_plane, double *out, void *stream);
 
+/* The same with a workspace: where it is the cheaper way, the sources of each frequency are first
+ * summed onto a common grid in K r / D by Lagrange interpolation of 16 points, whose error bound is 2e-16
+ * of an element, and J0 comes from one table (the sum is then a real FP64 product on the
+ * matrix cores).  With work NULL the call sets *bytes to the device bytes that this needs and runs
+ * nothing, or runs hk_direct's form and sets *bytes to 0 (few elements, radii that do not ascend from >= 0,
+ * a grid beyond LDS); a second call gives work, of *bytes or more, which is free again when it
+ * returns.  host_rho: the host copy of p->rho (NULL: copied from the device). */
+int hk_direct_work(const hk_planes *p, int n_out, const double *weights, int per_plane, const double *host_rho,
+                   double *out, void *work, long long *bytes, void *stream);
+
 /* Gridded contraction (no counterpart in the reference; same integral, reassociated):
  * J0(s r rho) = J0(q rho) with q = K r / D_k is interpolated in q from a uniform grid
  * Q_l = (l - HK_GRID_P/2) h, l < nq, by Lagrange interpolation of HK_GRID_P points, so that

@@ -38,6 +38,7 @@ SOURCES = [
     ("hankel_medium.hip", []),
     ("hankel_contract.hip", []),
     ("hankel_gemm.hip", []),
+    ("hankel_grid64.hip", []),
     ("hankel_abi.cpp", ["-x", "hip"]),
     ("stream_probe.hip", []),
 ]
@@ -45,7 +46,8 @@ SOURCES = [
 LIBS = {
     "libsingleTDSE.so": ["tdse_setup.hip", "tdse_analysis.hip", "tdse_propagate.hip", "tdse_resident.hip",
                          "tdse_adjoint.hip", "tdse_reverse.hip", "ctdse_abi.cpp"],
-    "libmmahankel.so": ["hankel_medium.hip", "hankel_contract.hip", "hankel_gemm.hip", "hankel_abi.cpp"],
+    "libmmahankel.so": ["hankel_medium.hip", "hankel_contract.hip", "hankel_gemm.hip", "hankel_grid64.hip",
+                        "hankel_abi.cpp"],
     # bandwidth probes for bench.py only (not part of the product)
     "libmmaprobe.so": ["stream_probe.hip"],
 }

@@ -56,6 +56,7 @@ HkConst make_constants()
 const double kInvC = 1.0 / 299792458.0;
 // largest q grid: its bins (16 B each) and the spread kernel's few static bytes fit the 160 KiB of LDS
 const int kMaxBins = 10176;
+const size_t kLds64 = size_t(160 * 1024) - 1024;  // bins of hk64_spread_kernel (its static LDS is some 600 bytes)
 
 int check_planes(const hk_planes *p)
 {
@@ -181,6 +182,113 @@ hipError_t enqueue_prefactor(const hk_medium *m, int nz, const double *zgrid, in
     return hipGetLastError();
 }
 
+// The contraction through one J0 table (hankel_grid64.hip): bytes 0 where hk_direct_kernel runs instead.
+struct Plan64 {
+    hk_grid64 g{};
+    int chunk = 0;  // outputs whose spread sources are held at once
+    long long bytes = 0;
+    size_t table = 0, rows = 0;  // offsets in the workspace (its start: the flag)
+};
+
+constexpr size_t kRows64 = size_t(512) << 20;  // spread sources held at once (one output at least)
+constexpr size_t kWork64 = size_t(4) << 30;    // largest workspace; beyond it the direct kernel runs
+
+int plan_grid64(const hk_planes *p, int outputs, int per_plane, const double *host_rho, Plan64 *plan)
+{
+    // The direct kernel's seconds: a thread's nz nr elements follow each other, 0.2 us each and 0.155 us for every
+    // workgroup on its CU (20 x 300 elements, 0.4 workgroups a CU: 2.1 ms; 256 x 512, 12: 246 ms).
+    const double direct = (double)p->nz * p->nr * (0.2e-6 + 0.155e-6 * p->no * ((p->nrho + 255) / 256) / 256.0);
+    if (direct < 100e-6 || p->nr > 64 * kBlocks64 || outputs > (1 << 20)) return HK_OK;
+    HostGrids hg;
+    std::vector<double> rho;
+    if (host_grids(p, hg) != HK_OK || host_grid(rho, host_rho, p->rho, p->nrho) != HK_OK) return g_status;
+    double rho_max = 0.0, o_max = 0.0, before = 0.0;
+    hk_grid64 g{};
+    g.inv_c = kInvC;
+    g.d_min = INFINITY;
+    for (double v : rho) {
+        if (!std::isfinite(v)) return HK_OK;
+        rho_max = std::max(rho_max, std::fabs(v));
+    }
+    for (double v : hg.o) {
+        if (!(v >= 0.0) || !std::isfinite(v)) return HK_OK;
+        o_max = std::max(o_max, v);
+    }
+    for (double v : hg.r) {
+        if (!(v >= before) || !std::isfinite(v)) return HK_OK;
+        before = v;
+    }
+    g.r_max = before;
+    for (double v : hg.z) {
+        const double d = p->distance - v;
+        if (!(d > 0.0) || !std::isfinite(d)) return HK_OK;
+        g.d_min = std::min(g.d_min, d);
+        g.d_max = std::max(g.d_max, d);
+    }
+    const double q_max = o_max * g.inv_c / g.d_min * g.r_max;
+    if (!(q_max * rho_max >= 1.0) || !(q_max * rho_max < 1e5)) return HK_OK;
+    // rho_max h: (rho h)^P max prod |f - d_i| / P! = 2e-16; h to 24 bits, so that l h is exact
+    double bound = 1.0;
+    for (int i = 0; i < kNodes64; i++) bound *= std::fabs(0.5 - (i - (kNodes64 / 2 - 1))) / (i + 1);
+    g.h = (double)std::nextafterf((float)(std::pow(2e-16 / bound, 1.0 / kNodes64) / rho_max), 0.0f);
+    g.inv_h = 1.0 / g.h;
+    const int need = (int)(q_max * g.inv_h) + kNodes64 + 3;
+    g.ld = (need + kStage64 - 1) / kStage64 * kStage64;
+    const int blocks = (p->nr + 63) / 64;
+    for (int b = 0; b < blocks; b++) {
+        const double k = o_max * g.inv_c, r0 = hg.r[b * 64], r1 = hg.r[std::min(b * 64 + 63, p->nr - 1)];
+        g.bins += (int)(k / g.d_min * r1 * g.inv_h) + kNodes64 + 4 - (int)(k / g.d_max * r0 * g.inv_h);
+    }
+    if ((size_t)g.bins * sizeof(double2) > kLds64) return HK_OK;
+    // This form's: 200 FP64 instructions a source and output and 0.8 us a plane in a row, 150 an entry of the table,
+    // the spread sources written and read, the product at 40 TFLOP/s or its tiles' serial sum, the launches.
+    // (64 planes x 300 frequencies x 256 radii to 512 screen points: 0.41 ms against 9.6, 256 x 768 x 512 to 1024:
+    // 1.76 against 246.)
+    const double rate = 3.9e13, rows = 2.0 * p->no * outputs, in_row = per_plane ? 1 : p->nz;
+    const double sources = (double)p->no * p->nr * in_row * outputs;
+    const double grid = sources * 200.0 / rate + in_row * ((blocks + 7) / 8) * 0.8e-6 + (double)p->nrho * g.ld * 150.0 / rate +
+                        rows * g.ld * 16.0 / 3e12 + std::max(2.0 * rows * g.ld * p->nrho / 4e13, g.ld * 27e-9) + 60e-6;
+    if (direct <= grid) return HK_OK;
+    plan->g = g;
+    const size_t tiles = (size_t)((p->nrho + kTile64 - 1) / kTile64) * ((2 * (size_t)p->no + kTile64 - 1) / kTile64);
+    const size_t one = 2 * (size_t)p->no * g.ld * sizeof(double);
+    plan->chunk = (int)std::max<size_t>(1, std::min<size_t>({(size_t)outputs, kRows64 / one, (size_t)65535, (size_t(1) << 30) / tiles}));
+    plan->table = 256;
+    plan->rows = plan->table + (size_t)p->nrho * g.ld * sizeof(double);
+    const size_t bytes = plan->rows + plan->chunk * one;
+    if (bytes <= kWork64) plan->bytes = (long long)bytes;
+    return HK_OK;
+}
+
+// finite: false where the spread met a value that is not (out is then written, but not the sum's)
+int run_grid64(const hk_planes *p, int outputs, const double *weights, const Plan64 &plan, double *out, void *work,
+               hipStream_t s, bool *finite)
+{
+    const hk_grid64 &g = plan.g;
+    char *w = static_cast<char *>(work);
+    int *flag = reinterpret_cast<int *>(w), got = 0;
+    double *table = reinterpret_cast<double *>(w + plan.table), *rows = reinterpret_cast<double *>(w + plan.rows);
+    const size_t lds = (size_t)g.bins * sizeof(double2);
+    auto spread = p->src_c64 ? hk64_spread_kernel<float2> : hk64_spread_kernel<double2>;
+    HK_HIP(hipFuncSetAttribute((const void *)spread, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLds64));
+    hipLaunchKernelGGL(hk_fill_int_kernel, dim3(1), dim3(64), 0, s, flag, 1, 0);
+    hipLaunchKernelGGL(hk64_bessel_kernel, dim3((g.ld + 255) / 256, p->nrho), dim3(256), 0, s, p->nrho, p->rho, g, table);
+    const int threads = std::min(kSpread64, 64 * ((p->nr + 63) / 64));
+    const int N = 2 * p->no, mt = (p->nrho + kTile64 - 1) / kTile64, nt = (N + kTile64 - 1) / kTile64;
+    for (int q = 0; q < outputs; q += plan.chunk) {
+        const int n = std::min(plan.chunk, outputs - q);
+        hipLaunchKernelGGL(spread, dim3(p->no, n), dim3(threads), lds, s, *p, g, outputs, weights, q, rows, flag);
+        const unsigned tiles = (unsigned)mt * nt * n;
+        hipLaunchKernelGGL(hk64_gemm_kernel, dim3((tiles + 7) / 8 * 8), dim3(512), 0, s, p->nrho, N, n, g, p->ogrid, table, rows,
+                           out + (size_t)q * p->nrho * N, (long long)N);
+    }
+    HK_HIP(hipGetLastError());
+    HK_HIP(hipMemcpyAsync(&got, flag, sizeof(int), hipMemcpyDeviceToHost, s));
+    HK_HIP(hipStreamSynchronize(s));
+    *finite = got == 0;
+    return HK_OK;
+}
+
 } // namespace
 
 extern "C" {
@@ -244,6 +352,31 @@ int hk_prefactor_status(int flag)
     if (flag == HK_FLAG_RANGE) return fail(HK_ERR_TABLE, "photon energy outside the tabulated scattering factors");
     if (flag == HK_FLAG_F1) return fail(HK_ERR_TABLE, "f1-scattering coefficient not listed for this frequency.");
     return HK_OK;
+}
+
+int hk_direct_work(const hk_planes *p, int n_out, const double *weights, int per_plane, const double *host_rho,
+                   double *out, void *work, long long *bytes, void *stream)
+{
+    clear_status();
+    if (check_planes(p) != HK_OK) return g_status;
+    if (!out || !bytes || (!per_plane && (n_out < 1 || n_out > 4 || !weights)))
+        return fail(HK_ERR_ARGUMENT, "need out, bytes and 1..4 weighted outputs (or per_plane)");
+    const int outputs = per_plane ? p->nz : n_out;
+    Plan64 plan;
+    if (plan_grid64(p, outputs, per_plane, host_rho, &plan) != HK_OK) return g_status;
+    if (plan.bytes > 0) {
+        if (!work) {
+            *bytes = plan.bytes;
+            return HK_OK;
+        }
+        if (*bytes < plan.bytes) return fail(HK_ERR_ARGUMENT, "workspace too small");
+        bool finite = true;
+        if (run_grid64(p, outputs, per_plane ? nullptr : weights, plan, out, work, (hipStream_t)stream, &finite) != HK_OK)
+            return g_status;
+        if (finite) return HK_OK;  // else the infinities and NaN of the sum itself
+    }
+    *bytes = 0;
+    return hk_direct(p, n_out, weights, per_plane, out, stream);
 }
 
 int hk_direct(const hk_planes *p, int n_out, const double *weights, int per_plane, double *out, void *stream)

@@ -34,6 +34,24 @@ template <typename S>
 __global__ void hk_direct_kernel(hk_planes p, int n_out, const double *weights, int per_plane, double2 *out,
                                  double inv_c, int uniform_r, double r0, double dr);
 
+// The FP64 contraction through one J0 table (hankel_grid64.hip): its grid Q_l = (l - kNodes64 / 2) h and what places the
+// sources on it.
+constexpr int kNodes64 = 16;    // Lagrange nodes
+constexpr int kTile64 = 64;     // rows and columns of a tile of the product
+constexpr int kStage64 = 32;    // elements of its sum per stage (the grid's length is a multiple)
+constexpr int kSpread64 = 512;  // largest workgroup of the spread
+constexpr int kBlocks64 = 64;   // blocks of 64 radii it takes
+struct hk_grid64 {
+    int ld;    // grid points, and the row stride of both operands
+    int bins;  // LDS bins of a workgroup (complex)
+    double h, inv_h, inv_c, d_min, d_max, r_max;
+};
+template <typename S>
+__global__ void hk64_spread_kernel(hk_planes p, hk_grid64 g, int outputs, const double *weights, int q0, double *out, int *nonfinite);
+__global__ void hk64_bessel_kernel(int nrho, const double *rho, hk_grid64 g, double *out);
+__global__ void hk64_gemm_kernel(int M, int N, int outputs, hk_grid64 g, const double *ogrid, const double *A, const double *B,
+                                 double *out, long long ldo);
+
 template <int TYPE>
 __global__ void hk_spread_kernel(hk_planes p, const double *weights, int nq, double h, double inv_c, void *out,
                                  long long ld, long long row0);

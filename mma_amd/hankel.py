@@ -72,6 +72,8 @@ def _L():
                                            c_void_p, c_void_p, c_void_p, c_void_p, c_void_p]
         L.hk_prefactor_status.argtypes = [c_int]
         L.hk_direct.argtypes = [POINTER(hk_planes), c_int, c_void_p, c_int, c_void_p, c_void_p]
+        L.hk_direct_work.argtypes = [POINTER(hk_planes), c_int, c_void_p, c_int, c_void_p, c_void_p, c_void_p,
+                                     POINTER(c_longlong), c_void_p]
         L.hk_grid_size.argtypes = [c_double, c_double, c_double, POINTER(c_int), POINTER(c_double)]
         L.hk_grid_spread.argtypes = [POINTER(hk_planes), c_int, c_void_p, c_int, c_double, c_int, c_void_p,
                                      c_longlong, c_longlong, c_void_p]
@@ -416,14 +418,22 @@ def direct(src, zgrid, ogrid, rgrid, rho, distance, weights=None, near_field=Tru
     keep = []
     pre_mode = 0 if pre is None else (1 if pre.dim() == 2 else 2)
     p = _planes_struct(src, zgrid, ogrid, rgrid, rho, distance, near_field, pre, pre_mode, keep)
-    nz = src.shape[0]
-    if per_plane:
-        out = torch.empty((nz, p.nrho, p.no), dtype=torch.complex128, device="cuda")
-        _check(_L().hk_direct(byref(p), 0, c_void_p(), 1, _ptr(out), _stream()))
-        return out
-    w = _dev(np.atleast_2d(weights))
-    out = torch.empty((w.shape[0], p.nrho, p.no), dtype=torch.complex128, device="cuda")
-    _check(_L().hk_direct(byref(p), w.shape[0], _ptr(w), 0, _ptr(out), _stream()))
+    w = None if per_plane else _dev(np.atleast_2d(weights))
+    n_out = 0 if per_plane else w.shape[0]
+    out = torch.empty((src.shape[0] if per_plane else n_out, p.nrho, p.no), dtype=torch.complex128, device="cuda")
+    hrho = _host(rho)
+    hrho_p = c_void_p(hrho.ctypes.data) if hrho is not None else c_void_p()
+    need = c_longlong()
+    L = _L()
+    args = (byref(p), n_out, _ptr(w), int(per_plane))
+    _check(L.hk_direct_work(*args, hrho_p, _ptr(out), c_void_p(), byref(need), _stream()))
+    if need.value > 0:
+        try:
+            work = torch.empty(need.value, dtype=torch.uint8, device="cuda")
+        except torch.cuda.OutOfMemoryError:  # the form without a workspace
+            _check(L.hk_direct(*args, _ptr(out), _stream()))
+        else:
+            _check(L.hk_direct_work(*args, hrho_p, _ptr(out), _ptr(work), byref(need), _stream()))
     return out
 
 
