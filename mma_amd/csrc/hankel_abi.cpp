@@ -182,6 +182,19 @@ hipError_t enqueue_prefactor(const hk_medium *m, int nz, const double *zgrid, in
     return hipGetLastError();
 }
 
+// Workgroups of hk_direct_kernel per frequency, its sources dealt to `parts` threads per screen radius.
+long long direct_blocks(const hk_planes *p, int parts) { return ((long long)p->nrho * parts + 255) / 256; }
+
+// parts: doubled up to 16 while there are fewer than four workgroups per CU.  64 frequencies x 200 radii to 301 screen
+// points: 86 us with 1, 57 with 2, 42 with 4 to 16; 16 x 1500 to 300: 515 with 1, 64 with 16; 200 x 300 to 600: 198
+// with 1, 143 with 2, 189 with 16.
+int direct_parts(const hk_planes *p)
+{
+    int parts = 1;
+    while (parts < 16 && p->no * direct_blocks(p, parts) < 1024) parts *= 2;
+    return parts;
+}
+
 // The contraction through one J0 table (hankel_grid64.hip): bytes 0 where hk_direct_kernel runs instead.
 struct Plan64 {
     hk_grid64 g{};
@@ -195,9 +208,11 @@ constexpr size_t kWork64 = size_t(4) << 30;    // largest workspace; beyond it t
 
 int plan_grid64(const hk_planes *p, int outputs, int per_plane, const double *host_rho, Plan64 *plan)
 {
-    // The direct kernel's seconds: a thread's nz nr elements follow each other, 0.2 us each and 0.155 us for every
-    // workgroup on its CU (20 x 300 elements, 0.4 workgroups a CU: 2.1 ms; 256 x 512, 12: 246 ms).
-    const double direct = (double)p->nz * p->nr * (0.2e-6 + 0.155e-6 * p->no * ((p->nrho + 255) / 256) / 256.0);
+    // The direct kernel's seconds: a thread's nz nr / parts elements follow each other, 0.2 us each and 0.155 us for
+    // every workgroup on its CU (16 frequencies, 1500 radii, 16 parts: 45 us; 256 x 512 elements, 12 workgroups a
+    // CU: 246 ms).
+    const int parts = direct_parts(p);
+    const double direct = (double)p->nz * p->nr / parts * (0.2e-6 + 0.155e-6 * p->no * direct_blocks(p, parts) / 256.0);
     if (direct < 100e-6 || p->nr > 64 * kBlocks64 || outputs > (1 << 20)) return HK_OK;
     HostGrids hg;
     std::vector<double> rho;
@@ -391,13 +406,14 @@ int hk_direct(const hk_planes *p, int n_out, const double *weights, int per_plan
     double dr = 0.0;
     const bool uniform = uniform_radii(r, &dr);
     hipStream_t s = (hipStream_t)stream;
-    dim3 grid(p->no, (p->nrho + 255) / 256);
+    const int parts = direct_parts(p);
+    dim3 grid((unsigned)p->no, (unsigned)direct_blocks(p, parts));
     if (p->src_c64)
         hipLaunchKernelGGL(hk_direct_kernel<float2>, grid, dim3(256), 0, s, *p, n_out, weights, per_plane,
-                           reinterpret_cast<double2 *>(out), kInvC, (int)uniform, r.front(), dr);
+                           reinterpret_cast<double2 *>(out), kInvC, (int)uniform, dr, parts);
     else
         hipLaunchKernelGGL(hk_direct_kernel<double2>, grid, dim3(256), 0, s, *p, n_out, weights, per_plane,
-                           reinterpret_cast<double2 *>(out), kInvC, (int)uniform, r.front(), dr);
+                           reinterpret_cast<double2 *>(out), kInvC, (int)uniform, dr, parts);
     HK_HIP(hipGetLastError());
     HK_HIP(hipStreamSynchronize(s));
     return HK_OK;

@@ -32,7 +32,7 @@ __global__ void hk_prefactor_finish_kernel(int nz, int no, const double *ogrid, 
 
 template <typename S>
 __global__ void hk_direct_kernel(hk_planes p, int n_out, const double *weights, int per_plane, double2 *out,
-                                 double inv_c, int uniform_r, double r0, double dr);
+                                 double inv_c, int uniform_r, double dr, int parts);
 
 // The FP64 contraction through one J0 table (hankel_grid64.hip): its grid Q_l = (l - kNodes64 / 2) h and what places the
 // sources on it.

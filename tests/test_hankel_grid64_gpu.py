@@ -98,3 +98,23 @@ def test_calls_that_keep_the_elementwise_kernel():
         assert table_bytes(src, z, o, rr, rho, D, 3, False) == 0
         assert torch.equal(H.direct(src, z, o, rr, rho, D, weights=weights),
                            elementwise(src, z, o, rr, rho, D, weights))
+
+
+# 16, 16, 8, 2 and 1 parts of the sources; 600 radii are two tiles of them
+@pytest.mark.parametrize("nz,no,nr,nrho", [(1, 3, 2, 1), (3, 5, 17, 300), (2, 60, 600, 150), (1, 130, 40, 700),
+                                           (1, 300, 40, 900)])
+def test_dealt_sources_against_fp64_sums(nz, no, nr, nrho):
+    src, z, o, r, rho, D, weights = case(nz, no, nr, nrho)
+    got = elementwise(src, z, o, r, rho, D, weights)
+    w = np.zeros(nr)
+    w[:-1] += 0.5 * np.diff(r)
+    w[1:] += 0.5 * np.diff(r)
+    K = o / H.C_LIGHT
+    ref = np.zeros((3, nrho, no), dtype=complex)
+    from scipy.special import j0
+    for k in range(nz):
+        u = src[k].cpu().numpy() * (w * r) * np.exp(-1j * K[:, None] * r ** 2 / (2 * (D - z[k])))
+        J = j0((K / (D - z[k]))[:, None, None] * (rho[:, None] * r))
+        ref += weights[:, k, None, None] * np.matmul(J, u[:, :, None])[..., 0].T
+    bound = TOL * absolute_terms(src, r, o, weights, False).cpu().numpy()[:, None, :] + 1e-300
+    assert (np.abs(got.cpu().numpy() - ref) <= bound).all()
