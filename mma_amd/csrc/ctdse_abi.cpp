@@ -516,12 +516,6 @@ bool plan_resident(int nx, int reach, TdseResident &R)
     return R.chunk > 0;
 }
 
-// Dynamic LDS of a workgroup of plan R: the lanes' share of b.
-size_t lane_lds(const TdseResident &R)
-{
-    return (size_t)R.waves * 64 * std::min(R.chunk, TDSE_RES_LDS) * sizeof(double2);
-}
-
 // Entries of a resident table of nx points in lanes of C: whole tiles, one zero chunk at least.
 long long resident_entries(int nx, int C) { return (long long)(((nx + C - 1) / C + 1 + 63) / 64) * 64 * C; }
 
@@ -583,6 +577,7 @@ int attach_tables(ctdse_geometry *G, const ctdse_geometry *src, TdseResident &R,
     const int off = (src->num_r - G->num_r) / 2;
     R.chunk0 = off / R.chunk;
     R.lead = off % R.chunk;
+    R.nx = D.nx;
     R.head = src != G ? std::min(D.nx, G->reach) : 0;
     // the chunks around the atom: rows of <psi0|psi> (p0_lo > p0_hi: psi0 is zero) and of PopInt
     const int lo = std::min(std::min(D.p0_lo, D.pint_lo), std::max(D.pint_hi, 0));
@@ -597,6 +592,7 @@ int attach_tables(ctdse_geometry *G, const ctdse_geometry *src, TdseResident &R,
     J.C = R.chunk;
     J.first = R.core_chunk0 * R.chunk - R.lead;
     J.n = R.core_chunks;
+    J.n_tiles = R.core_chunks / 64 + 1;
     J.lo = D.pint_lo;
     J.hi = D.pint_hi;
     J.head = R.head;
@@ -611,7 +607,7 @@ int add_resident(const std::vector<ctdse_geometry *> &gs)
 {
     // here and not at a launch, which may be captured
     HIP_CHECK(hipFuncSetAttribute((const void *)tdse_window_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                  TDSE_ONE_WAVES * 64 * TDSE_RES_LDS * (int)sizeof(double2)));
+                                  tdse_res_lds(TDSE_ONE_WAVES, 24)));
     std::map<const Lattice *, ctdse_geometry *> widest;
     for (ctdse_geometry *G : gs)
         if (G && G->lattice) {
@@ -634,7 +630,8 @@ int add_resident(const std::vector<ctdse_geometry *> &gs)
     if (jobs.empty()) return CTDSE_OK;
     auto pool = std::make_shared<DevMem>();
     size_t entries = 0;  // of 16 bytes
-    auto size_of = [](const ResidentJob &J) { return (size_t)(J.C * J.n + J.head + (J.C * J.n + 1) / 2); };
+    auto rows_of = [](const ResidentJob &J) { return J.C * 64 * J.n_tiles; };
+    auto size_of = [&](const ResidentJob &J) { return (size_t)(rows_of(J) + J.head + rows_of(J) / 2); };
     for (const ResidentJob &J : jobs) entries += size_of(J);
     DevMem d_jobs;
     HIP_CHECK(pool->alloc(entries * sizeof(double2)));
@@ -644,7 +641,7 @@ int add_resident(const std::vector<ctdse_geometry *> &gs)
     for (size_t k = 0; k < jobs.size(); k++) {
         ResidentJob &J = jobs[k];
         TdseResident &R = *plans[k].second;
-        const int m = J.C * J.n;
+        const int m = rows_of(J);
         J.core = at;
         J.head_b = at + m;
         J.im = reinterpret_cast<double *>(at + m + J.head);
@@ -927,11 +924,13 @@ int resident_shape(const std::vector<const ctdse_geometry *> &geoms, LaunchShape
 {
     sh.resident = true;
     sh.nw = 1;
+    size_t lanes = 0;
     for (const ctdse_geometry *g : geoms) {
         const TdseResident &R = g->dev.res;
         sh.nw = std::max(sh.nw, R.waves);
-        sh.lds = std::max(sh.lds, lane_lds(R));
+        lanes = std::max(lanes, (size_t)(tdse_res_lds(R.waves, R.chunk) - tdse_res_shared(R.waves)));
     }
+    sh.lds = tdse_res_shared(sh.nw) + lanes;
     hipFuncAttributes attr;
     int dev = 0, lds = 0;
     HIP_CHECK(hipFuncGetAttributes(&attr, (const void *)tdse_resident_kernel));
@@ -941,7 +940,7 @@ int resident_shape(const std::vector<const ctdse_geometry *> &geoms, LaunchShape
     sh.per_cu = std::max(1, std::min(4 * TDSE_RES_WAVES_PER_SIMD / sh.nw, fit));
     // the most any batch asks for, so that plans of different sizes live side by side
     HIP_CHECK(hipFuncSetAttribute((const void *)tdse_resident_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                  TDSE_MAX_WAVES * 64 * TDSE_RES_LDS * (int)sizeof(double2)));
+                                  tdse_res_lds(TDSE_MAX_WAVES, 32)));
     return CTDSE_OK;
 }
 
@@ -1023,12 +1022,13 @@ struct BatchHost {
     std::vector<int> order;
     TdseQueues queues{};
     long long stride = 0;
-    long long res_stride = 0;  // of the resident kernel: one state of its windows
+    long long res_stride = 0;  // of the resident kernel: two states of its windows, and b (tdse_res_far)
 };
 
 int describe(const std::vector<InstSpec> &spec, BatchHost &B)
 {
     const int n = (int)spec.size();
+    bool far = false;
     B.insts.assign(n, TdseInst{});
     for (int i = 0; i < n; i++) {
         const InstSpec &s = spec[i];
@@ -1065,8 +1065,10 @@ int describe(const std::vector<InstSpec> &spec, BatchHost &B)
         B.stride = std::max(B.stride, s.geom->dev.npad);
         const TdseResident &R = s.geom->dev.res;
         if (R.chunk && R.windows > 1)
-            B.res_stride = std::max(B.res_stride, (((long long)(R.windows - 1) * R.stride + 64 * R.waves + 63) / 64) * 64 * R.chunk);
+            B.res_stride = std::max(B.res_stride, (((long long)(R.windows - 1) * R.stride + 64 * R.waves + 63) / 64) * 64 * R.chunk * 2);
+        far = far || (R.chunk > 24 && R.head > 0);
     }
+    if (B.res_stride > 0 || far) B.res_stride += tdse_res_far(TDSE_MAX_WAVES, 32);
     // largest instances first (longest-processing-time order for the atomic queues)
     std::vector<int> lpt(n);
     for (int i = 0; i < n; i++) lpt[i] = i;
@@ -1129,11 +1131,11 @@ int enqueue_plan(const ctdse_batch_plan &P, double2 *work, hipStream_t stream)
     return CTDSE_OK;
 }
 
-// A launch's work buffer: one state per workgroup; the resident kernel needs two, and only for
-// grids of several windows.
+// A launch's work buffer: one state per workgroup; for the resident kernel what res_stride says, and only for
+// grids of several windows or, with 32 points a lane, of a shared lattice.
 size_t work_bytes(const ctdse_batch_plan &P)
 {
-    return (size_t)P.slots * P.stride * sizeof(double2) * (P.shape.resident ? 2 : 1);
+    return (size_t)P.slots * P.stride * sizeof(double2);
 }
 
 // Immediate path: descriptors copied on `stream`, the shared work buffer, and a wait.
@@ -1210,7 +1212,7 @@ int enqueue_steps(const InstSpec &s, const StepBufs &b, hipStream_t stream)
     inst.pregated = 1;
     hipLaunchKernelGGL(tdse_put_desc_kernel, dim3(1), dim3(64), 0, stream, g, inst, b.geom, b.inst);
     hipLaunchKernelGGL(tdse_gate_kernel, dim3(1), dim3(256), 0, stream, s.field, n_field, b.gated);
-    const size_t lds = lane_lds(R);
+    const size_t lds = tdse_res_lds(R.waves, R.chunk);
     const dim3 untile_grid((g.nx + 255) / 256);
     const int n_snap = s.snap ? s.n_snap : 0, every = std::max(1, s.snap_every);
     int i_snap = 0, launch = 0, prev = 0;

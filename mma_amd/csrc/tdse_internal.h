@@ -27,7 +27,6 @@
 #define TDSE_REV_WAVES_PER_SIMD 2  // reconstructing adjoint kernel: 256-VGPR budget, 8 waves per CU
 #define TDSE_MAX_HALO 40           // largest truncation depth in chunks
 #define TDSE_RES_WAVES_PER_SIMD 2  // resident propagation kernel: 256-VGPR budget, 8 waves per CU
-#define TDSE_RES_LDS 19            // its points per lane whose factor sits in LDS
 #define TDSE_RES_RING 16           // its steps between two writes of observables
 #define TDSE_RES_GROUP 4           // points per thread of its table builders
 #define TDSE_ONE_WAVES 4           // waves per window of one instance alone (one per SIMD)
@@ -65,13 +64,43 @@ struct TdseResident {
     int waves, windows, steps;
     int stride, halo;     // chunks: from window to window, and not owned at an inner edge
     int lead, chunk0, chunks;  // chunks: table chunks before the first zero one
-    const double2 *core;  // {Re psi0, 1 in the PopInt window}: row i of core_chunks chunks per point of a chunk
+    const double2 *core;  // {Re psi0, 1 in the PopInt window} of core_chunks chunks and one of zeros, in tiles
     const double *core_im;  // Im psi0 likewise, null where it is 0
     int core_chunk0, core_chunks;
     const double2 *head_b;  // b of the leading `head` points, which feel the geometry's own left wall
-    int head;
+    int head;             // 0: the tables are the geometry's own
+    int nx;               // its points
     int reach;            // points after which a carry is below 1e-17
 };
+
+// What neighbouring waves of the resident kernel exchange in one step.
+struct TdseWaveEdge {
+    double2 a;    // f and carry of the wave's last point, for the wave after
+    double2 nb;   // -b of that point
+    double2 f0;   // f of the wave's first point, for the wave before
+    double2 up;   // phi of the wave's first point, for the wave before
+};
+
+// Points of a lane of c whose b sits in LDS (with 32, the product nQ as well: tdse_res_lds_rows).  With 32 a CU
+// has room for one workgroup of 8 waves, whose 19 rows fill its LDS; with 24, 18 leave room for as many
+// workgroups of 1, 2 or 4 waves as make 8 waves (with 19 one of 4 waves had the CU for itself: 6001 points, 512
+// instances 4.6 ms, now 3.6).
+__host__ __device__ constexpr int tdse_res_lds_points(int c) { return c <= 16 ? c : 18; }
+__host__ __device__ constexpr int tdse_res_lds_rows(int c) { return tdse_res_lds_points(c) + (c > 24 ? 1 : 0); }
+
+// Entries of global memory for the other points' b of nw waves with 32 points a lane.
+__host__ __device__ constexpr int tdse_res_far(int nw, int c) { return c > 24 ? nw * 64 * (c - tdse_res_lds_points(c)) : 0; }
+
+// Bytes of LDS of a workgroup of nw waves: what the waves share, and the lanes' b before it.
+__host__ __device__ constexpr int tdse_res_shared(int nw)
+{
+    const int bytes = (nw + 1) * (int)sizeof(TdseWaveEdge) + (TDSE_RES_RING + 1) * nw * 5 * 8;
+    return (bytes + 15) / 16 * 16;
+}
+__host__ __device__ constexpr int tdse_res_lds(int nw, int c)
+{
+    return tdse_res_shared(nw) + nw * 64 * tdse_res_lds_rows(c) * (int)sizeof(double2);
+}
 
 // Step-independent tables of one geometry (num_r, dx, dt, a, x_int), device pointers.
 // The Crank-Nicolson system of one step, scaled by 12, is
@@ -186,7 +215,7 @@ struct ResidentJob {
     const double *g;        // tiled
     const double2 *ib;      // tiled
     const double2 *psi0;    // natural order
-    int nx, C, first, n, lo, hi, head, warm;
+    int nx, C, first, n, n_tiles, lo, hi, head, warm;
     double k36;
     double2 *core, *head_b;
     double *im;

@@ -12,22 +12,26 @@
 // i.e. for phi = G psi' a symmetric system with unit off-diagonals, tridiag(1, c_j, 1) phi = r.  Its
 // factorisation needs one number per point, b_j = (1 + i g_j) / beta_j (the pivots of phi):
 //     r_j   = (f_{j+1} - f_j) - (f_j - f_{j-1}) + (12 - i (12 g_j + K)) psi_j,   f = conj(G) psi
-//     y_j   = r_j - b_{j-1} y_{j-1}            4 FMA a point
-//     phi_j = b_j (y_j - phi_{j+1})            6
+//     y_j   = r_j - b_{j-1} y_{j-1}            4 FMA a point, or w_j = b_j y_j = b_j (r_j - w_{j-1}), 6
+//     phi_j = w_j - b_j phi_{j+1}              4
 //     psi'_j = phi_j / (1 + i g_j)             4, from a table
 // Both recurrences run twice around a scan over the lanes: once from zero for the carry that leaves
-// the lane's chunk, once from the true carry.  Carries decay by rho < 1 per point, below 1e-17 after
+// the lane's chunk (as y), once from the true carry (as w).  Carries decay by rho < 1 per point, below 1e-17 after
 // `reach` points, so a scan looks back only as far as that (3 or 4 levels within rows of 16 lanes, one
 // step from the row before), a wave takes its carry from the one wave next to it, and windows
 // overlap by `reach` points per step.
 //
-// Where the operands live: psi (r, y and phi in turn) in 4 C registers, b in LDS (up to 19 points a
-// lane: 512 lanes x 19 x 16 B = 152 KB) and the rest in registers, both for the whole run; g, V' and
-// 1/(1 + i g) come from L2, 32 B a point and step, shared by all instances of a grid.  HBM is idle:
-// the FP64 units bound the step (about 57 + 330 / C instructions a point).
+// Where the operands live: psi (r, w and psi in turn) in 4 C registers; b of up to 18 points a lane in LDS (512
+// lanes x 18 x 16 B = 144 KB), of the others in registers, with 32 points from L2 once a step (far_points); g, V' and
+// 1/(1 + i g) come from L2, 32 B a point and step, shared by all instances of a grid.  HBM is idle: the
+// FP64 units bound the step (about 46 + 300 / C of their instructions a point, 60 % of the time; the rest is
+// waits for LDS and L2 and the two barriers).  No step spills a register: with 22 reloads of spilled values a
+// step of 16001 points took 11.7 us, each reload waiting for the table rows in flight before it as well.
 //
-// Measured under load: a step of 16001 points takes 11.6 us a compute unit, of 12001 8.2, of 8001 6.0, 3.4 to 3.7e11
-// points a second on the chip, where the streaming kernels reach 1.75e11.
+// Measured under load, 512 instances: a step of 16001 points takes 9.7 us a compute unit (11.7 before the waves
+// around the atom had a loop of their own, the sine and cosine that all lanes share were evaluated once
+// for eight steps, and the spills were gone), of 12001 7.3 (7.9), of 8001 5.6 (6.0), of 6001 4.0 (5.2, one
+// workgroup a CU); 3.6 to 4.2e11 points a second on the chip, where the streaming kernels reach 1.75e11.
 //
 // r_j takes the differences of f first: they cancel exactly, where f_{j-1} + f_{j+1} + (10 - i (10 g_j + K)) psi_j
 // rounds three terms of 2 |g| |psi| each (|g| = 75 to 300) for a result of 12 |psi|.  That noise made two solves of one run with
@@ -43,20 +47,24 @@ namespace {
 
 using namespace tdse;
 
-// points of a lane whose b sits in LDS; the rest are held in registers
-constexpr int lds_points(int c) { return c < TDSE_RES_LDS ? c : TDSE_RES_LDS; }
-
-// what neighbouring waves exchange in one step
-struct WaveEdge {
-    double2 a;    // f and carry of the wave's last point, for the wave after
-    double2 nb;   // -b of that point
-    double2 f0;   // f of the wave's first point, for the wave before
-    double2 up;   // phi of the wave's first point, for the wave before
-};
-
+// What a workgroup of nw waves shares, in dynamic LDS (tdse_res_lds()).
 struct Shared {
-    WaveEdge edge[TDSE_MAX_WAVES + 1];
-    double ring[TDSE_RES_RING + 1][TDSE_MAX_WAVES][5];
+    TdseWaveEdge *edge; // nw + 1
+    double *ring;       // TDSE_RES_RING + 1 entries of the observables' sums, [nw][5]
+    double2 *b;         // the lanes' share of b
+    int nw;
+    __device__ double *sums(int t, int wave) const { return ring + (t * nw + wave) * 5; }
+};
+__device__ inline Shared shared_memory(double2 *lds)
+{
+    Shared sh;
+    sh.nw = blockDim.x >> 6;
+    sh.edge = reinterpret_cast<TdseWaveEdge *>(lds);
+    sh.ring = reinterpret_cast<double *>(sh.edge + sh.nw + 1);
+    sh.b = lds + tdse_res_shared(sh.nw) / sizeof(double2);
+    return sh;
+}
+struct Queue {
     int cur, tried, gate;
 };
 
@@ -66,6 +74,42 @@ __device__ inline double2 row(const double2 *base, unsigned lane_off, int i)
     const TDSE_GLOBAL char *p = (const TDSE_GLOBAL char *)base + i * 1024;
     const tdse_d2 v = *(const TDSE_GLOBAL tdse_d2 *)(p + lane_off);
     return make_double2(v.x, v.y);
+}
+
+// a value that all lanes agree on, in scalar registers
+__device__ inline double uniform(double v)
+{
+    const long long b = __builtin_bit_cast(long long, v);
+    const int lo = __builtin_amdgcn_readfirstlane((int)b), hi = __builtin_amdgcn_readfirstlane((int)(b >> 32));
+    return __builtin_bit_cast(double, ((long long)hi << 32) | (unsigned int)lo);
+}
+
+// r with its fields to be read again from here on, and not kept in registers across what came before
+template <typename T>
+__device__ inline const T &fresh(const T &r)
+{
+    typedef const T __attribute__((address_space(4))) const_t;
+    const unsigned long long a = reinterpret_cast<unsigned long long>(&r);
+    unsigned lo = __builtin_amdgcn_readfirstlane((int)a), hi = __builtin_amdgcn_readfirstlane((int)(a >> 32));
+    asm volatile("" : "+s"(lo), "+s"(hi));
+    return *(const T *)(const_t *)((unsigned long long)hi << 32 | lo);
+}
+
+// a value that all lanes agree on, as one that might differ: branches on it keep the registers' allocation in
+// one piece (scalar ones cut it, and b was spilled around them)
+__device__ inline int per_lane(int v)
+{
+    int l;
+    asm volatile("v_mov_b32 %0, %1" : "=v"(l) : "s"(v));
+    return l;
+}
+
+// this lane's number, formed anew: kept across a step it would be spilled, and wait for its reload
+__device__ inline int lane_id()
+{
+    int l;
+    asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=&v"(l));
+    return l;
 }
 
 // p as a value the compiler knows nothing about: the row addresses of one step are then formed in
@@ -150,17 +194,24 @@ __device__ inline StepConst step_const(const TdseGeom &G)
     return c;
 }
 
+// With 32 points a lane's registers do not hold psi, b and what the first pass works with.  That pass
+// needs no b, so those that LDS does not hold are read from the table again after it, and arrive while y runs
+// over the points before (7 B a point and step more from L2).  What is left in registers the compiler spills, and
+// each pass waits for the reloads: with the phases of one stage of this kernel a step of 16001 points took 11.1 us
+// with all 14, 11.4 with 12, 14 to 18 with 4.
+constexpr int far_points(int c) { return c > 24 ? c - tdse_res_lds_points(c) : 0; }
+
 // The state of one lane and what it needs of its grid and window.
 template <int C>
 struct Lane {
-    static constexpr int NL = lds_points(C), NR = C - NL;
-    double2 P[C];                    // psi, then r, y, phi in place
+    static constexpr int NL = tdse_res_lds_points(C), NF = far_points(C), NR = C - NL;
+    double2 P[C];                    // psi, then r, w, psi in place
     double2 br[NR > 0 ? NR : 1];     // b of points NL .. C - 1
-    double2 nQ;                      // product of -b over the chunk (both transfer maps)
-    double gl;                       // g of the last point
+    double2 nQ;                      // product of -b over the chunk (both transfer maps); with 32 points in LDS, lb[64 NL]
     unsigned off;                    // byte offset of the lane's first table row
     int j0;                          // grid index of its first point (may lie before the grid)
     bool own;                        // its points belong to this window
+    const TDSE_GLOBAL tdse_d2 *far;  // b of point NL + i at [64 i], where they are not kept all the time
 };
 
 // b of point i
@@ -182,7 +233,7 @@ __device__ inline unsigned row_offset(int c)
 // Puts a lane on its chunk of window w: chunks of C points, counted from the table chunk that holds the
 // grid's start.  core: the lane's wave holds part of the core table's chunks.
 template <int C>
-__device__ inline void place_lane(const TdseResident &R, int w, int wave, int lane, Lane<C> &L, int &chunk, bool &core)
+__device__ inline void place_lane(const TdseResident &R, int w, int wave, int lane, Lane<C> &L, int &chunk, int &core)
 {
     const int c0 = w * R.stride, w0 = c0 + wave * 64, c = w0 + lane;
     L.off = row_offset<C>(min(c + R.chunk0, R.chunks));  // (table chunk R.chunks: zeros)
@@ -192,18 +243,24 @@ __device__ inline void place_lane(const TdseResident &R, int w, int wave, int la
     core = __builtin_amdgcn_readfirstlane(w0 < R.core_chunk0 + R.core_chunks && w0 + 64 > R.core_chunk0);
 }
 
+// b of point i, where the table (of a lattice that several grids share) has `b`
+template <int C>
+__device__ inline double2 own_b(const TdseResident &R, const Lane<C> &L, int i, double2 b)
+{
+    const int j = L.j0 + i;
+    if (j < R.head && j >= 0) b = ld2(R.head_b, j);  // still feels this grid's own left wall
+    return j < 0 || j >= R.nx ? make_double2(0.0, 0.0) : b;
+}
+
 // The lane's b into LDS and registers, with what follows from it.
 template <int C>
-__device__ inline void load_b(const TdseGeom &G, const TdseResident &R, Lane<C> &L, double2 *lb)
+__device__ inline void load_b(const TdseResident &R, Lane<C> &L, double2 *lb, double2 *store)
 {
+    using LN = Lane<C>;
     double2 q = make_double2(1.0, 0.0);
-    L.gl = row(R.gv, L.off, C - 1).x;
 #pragma unroll
     for (int i = 0; i < C; i++) {
-        const int j = L.j0 + i;
-        double2 b = row(R.b, L.off, i);
-        if (j < R.head && j >= 0) b = ld2(R.head_b, j);  // still feels this grid's own left wall
-        if (j < 0 || j >= G.nx) b = make_double2(0.0, 0.0);
+        const double2 b = own_b<C>(R, L, i, row(R.b, L.off, i));
         if (i < Lane<C>::NL)
             lb[i * 64] = b;
         else
@@ -211,7 +268,36 @@ __device__ inline void load_b(const TdseGeom &G, const TdseResident &R, Lane<C> 
         q = cmul(q, make_double2(-b.x, -b.y));
         __builtin_amdgcn_sched_barrier(0);
     }
-    L.nQ = q;
+    if (C > 24)
+        lb[64 * LN::NL] = q;
+    else
+        L.nQ = q;
+    if constexpr (LN::NF > 0) {
+        // from the table, unless the lane's b are its own
+        const bool own = R.head > 0 && (L.j0 < R.head || L.j0 + C > R.nx);
+        const double2 *const p = own ? store : R.b + L.off / sizeof(double2) + 64 * LN::NL;
+        L.far = (const TDSE_GLOBAL tdse_d2 *)p;
+        if (own) {
+#pragma unroll
+            for (int i = 0; i < LN::NF; i++) st2(store, 64 * i, L.br[i]);
+        }
+    }
+}
+
+// Those of the lane's b that the first pass did not keep.
+template <int C>
+__device__ inline void fetch_far(Lane<C> &L)
+{
+    using LN = Lane<C>;
+    if constexpr (LN::NF == 0) return;
+    unsigned long long at = reinterpret_cast<unsigned long long>(L.far);
+    asm volatile("" : "+v"(at));  // the rows' addresses are formed here, not kept (and spilled) across the steps
+    const TDSE_GLOBAL tdse_d2 *const far = reinterpret_cast<const TDSE_GLOBAL tdse_d2 *>(at);
+#pragma unroll
+    for (int i = C - LN::NF; i < C; i++) {
+        const tdse_d2 v = far[64 * (i - LN::NL)];
+        L.br[i < LN::NL ? 0 : i - LN::NL] = make_double2(v.x, v.y);
+    }
 }
 
 // The lane's points of a tiled state (zero outside the grid).
@@ -233,53 +319,52 @@ __device__ inline void put_state(double *dst, long long index, double2 v)
     dst[2 * index + 1] = v.y;
 }
 
-// Rows of the tables, and of b from LDS, in flight in the first, the last and the passes between.  A
-// row costs registers that 32 points a lane do not have: there 3, 6 and 1 / 3 run a step of 16001 points in
-// 11.6 us under load, 2 and 6 in 13.4, 3 and 5 in 14, two b rows at the ends in 12.4.  With 16 points 4 rows take 6.0 us
-// for 8001 points, 5 or 6 rows 6.4.
+// Rows of the tables, of the core table, and of b from LDS in flight in the first, the last and the passes
+// between.  A row costs registers that 32 points a lane do not have; more of them gain nothing for 16 and 24
+// (6 or 8 rows in the first pass, 12 in the last, 4 and 6 of LDS: within 1 % or slower).
 constexpr int rows_first(int c) { return c > 24 ? 3 : 4; }
-constexpr int rows_last(int c) { return c > 24 ? 6 : 8; }
+constexpr int rows_last(int c) { return c > 24 ? 4 : 8; }
+constexpr int rows_core(int c) { return c > 24 ? 2 : 4; }
 constexpr int lds_ends(int c) { return c > 24 ? 1 : 2; }
-constexpr int lds_between(int c) { return c > 24 ? 3 : 4; }
+constexpr int lds_between(int c) { return c > 24 ? 2 : 4; }
 
-// Observables over the lane's points (psi in P) that only waves near the atom need: <psi0|psi> and
-// PopInt, from the core table: {Re psi0, 1 inside the PopInt window} (and Im psi0 where it is not 0)
-// of the chunks that hold either, one row of core_chunks entries per point of a chunk.
-template <int C>
-__device__ inline void observe_core(const TdseResident &R, const Lane<C> &L, int chunk, Acc &acc)
+// Sine and cosine with the coefficients from memory, into scalar registers: as literals they are moved to
+// vector registers before the loop over the steps, where no register is free, and spilled.
+__constant__ double kCoef[17] = SINCOS_COEFFICIENTS;
+__device__ inline void sincos_lean(double x, double *s, double *c)
 {
-    const int c = chunk - R.core_chunk0, n = R.core_chunks;
-    if (c < 0 || c >= n) return;
-    const double2 *q = R.core + c;
-    constexpr int A = 8;  // rows in flight
-    double2 t[A];
-#pragma unroll
-    for (int i = 0; i < A; i++) t[i] = ld2(q, i * n);
+    typedef const double __attribute__((address_space(4))) coef_t;
+    coef_t *k = (coef_t *)kCoef;
+    asm volatile("" : "+s"(k));
+    sincos_wide(x, s, c, k);
+}
+
+// Offset of the lane's rows in the core table: {Re psi0, 1 inside the PopInt window} of the chunks that hold
+// either, in tiles as the other tables, then a chunk of zeros for the other lanes of a wave.
+template <int C>
+__device__ inline unsigned core_offset(const TdseResident &R, const Lane<C> &L)
+{
+    const int c = (L.j0 + R.lead) / C - R.core_chunk0;
+    return row_offset<C>(c < 0 || c > R.core_chunks ? R.core_chunks : c);
+}
+
+// The part of Im psi0 in a lane's sums over <psi0|psi>, where there is one.
+template <int C>
+__device__ inline void core_im(const TdseResident &R, const Lane<C> &L, unsigned off, Acc &acc)
+{
+    const double *m = R.core_im + off / sizeof(double2);
 #pragma unroll
     for (int i = 0; i < C; i++) {
-        const double2 w = t[i % A], p = L.P[i];
-        if (i + A < C) t[i % A] = ld2(q, (i + A) * n);
-        acc.pr = fma(p.x, w.x, acc.pr);
-        acc.pi = fma(-p.y, w.x, acc.pi);
-        acc.pint = fma(fma(p.x, p.x, p.y * p.y), w.y, acc.pint);
-        asm volatile("" : "+v"(acc.pr), "+v"(acc.pi), "+v"(acc.pint));
+        const double v = ld1(m, 64 * i);
+        acc.pr = fma(L.P[i].y, v, acc.pr);
+        acc.pi = fma(L.P[i].x, v, acc.pi);
+        asm volatile("" : "+v"(acc.pr), "+v"(acc.pi));
         __builtin_amdgcn_sched_barrier(0);
-    }
-    if (R.core_im) {
-        const double *m = R.core_im + c;
-#pragma unroll
-        for (int i = 0; i < C; i++) {
-            const double v = ld1(m, i * n);
-            acc.pr = fma(L.P[i].y, v, acc.pr);
-            acc.pi = fma(L.P[i].x, v, acc.pi);
-            asm volatile("" : "+v"(acc.pr), "+v"(acc.pi));
-            __builtin_amdgcn_sched_barrier(0);
-        }
     }
 }
 
 // Per-wave sums into a ring entry (lane 63 writes; `add`: onto what earlier windows left there).
-__device__ inline void put_observables(Acc &acc, bool own, bool core, bool add, int lane, double *dst)
+__device__ inline void put_observables(Acc &acc, bool own, int core, bool add, int lane, double *dst)
 {
     if (!own) acc = Acc{0.0, 0.0, 0.0, 0.0, 0.0};
     const double pos = sum63(acc.pos), gp = sum63(acc.gp);
@@ -290,115 +375,158 @@ __device__ inline void put_observables(Acc &acc, bool own, bool core, bool add, 
         pint = sum63(acc.pint);
     }
     if (lane == 63) {
-        dst[0] = add ? dst[0] + pr : pr;
-        dst[1] = add ? dst[1] + pi : pi;
-        dst[2] = add ? dst[2] + pint : pint;
-        dst[3] = add ? dst[3] + pos : pos;
-        dst[4] = add ? dst[4] + gp : gp;
+        const double v[5] = {pr, pi, pint, pos, gp};
+        const int more = per_lane(add);
+#pragma unroll
+        for (int q = 0; q < 5; q++) {
+            const double old = dst[q];
+            dst[q] = more ? old + v[q] : v[q];
+        }
     }
 }
 
 // The observables of P alone (the last state of a partial run).
 template <int C>
-__device__ inline void observe_only(const TdseGeom &G, const Lane<C> &L, int chunk, const double2 *gv, bool core, bool add,
+__device__ inline void observe_only(const TdseGeom &G, const Lane<C> &L, const double2 *gv, int core, bool add,
                                     int lane, double *dst)
 {
     double s0 = 0.0, s1 = 0.0;
     const TdseResident &R = G.res;
     Acc acc = {0.0, 0.0, 0.0, 0.0, 0.0};
-    if (core) observe_core<C>(R, L, chunk, acc);
+    const unsigned off = core_offset<C>(R, L);
 #pragma unroll
     for (int i = 0; i < C; i++) {
-        const double n2 = fma(L.P[i].x, L.P[i].x, L.P[i].y * L.P[i].y);
+        const double2 p = L.P[i];
+        const double n2 = fma(p.x, p.x, p.y * p.y);
         s0 += n2;
         s1 = fma((double)i, n2, s1);
         acc.gp = fma(n2, row(gv, L.off, i).y, acc.gp);
+        if (core) {
+            const double2 w = row(R.core, off, i);
+            acc.pr = fma(p.x, w.x, acc.pr);
+            acc.pi = fma(-p.y, w.x, acc.pi);
+            acc.pint = fma(n2, w.y, acc.pint);
+        }
         __builtin_amdgcn_sched_barrier(0);
     }
+    if (core && R.core_im) core_im<C>(R, L, off, acc);
     acc.pos = fma(grid_x(L.j0, G.dx, G.xmax), s0, G.dx * s1);
     put_observables(acc, L.own, core, add, lane, dst);
 }
 
-// One time step of the window's points.  ring: this wave's ring entry for the state it starts from.
-template <int C>
-__device__ inline void step(const TdseResident &R, const StepConst &K, Lane<C> &L, int chunk, const double2 *gv,
-                            const double2 *rs, const double2 *lb, Shared &sh, int wave, int lane, double F, bool core,
-                            bool deep, bool add, double *ring)
+// Observables of the state, and the right-hand side r in its place.  CORE: the wave holds part of the atom.
+// What only the wave's edge lanes need later (f of its first and last point) goes to E at once.
+template <int C, bool CORE>
+__device__ inline void first_pass(const TdseResident &R, const StepConst &K, Lane<C> &L, const double2 *gv, Acc &acc,
+                                  TdseWaveEdge &E)
+{
+    constexpr int kRows = rows_first(C), kCore = CORE ? rows_core(C) : 1;  // rows in flight
+    const double2 *const cq = opaque(R.core);
+    const unsigned coff = CORE ? core_offset<C>(R, L) : 0;
+    double2 t[kRows], q[kCore];
+    const double gl = row(gv, L.off, C - 1).x;
+#pragma unroll
+    for (int i = 0; i < kRows; i++) t[i] = row(gv, L.off, i);
+    if (CORE) {
+#pragma unroll
+        for (int i = 0; i < kCore; i++) q[i] = row(cq, coff, i);
+        if (R.core_im) core_im<C>(R, L, coff, acc);
+    }
+    const double2 pl = L.P[C - 1];
+    const double2 f0 = make_double2(fma(t[0].x, L.P[0].y, L.P[0].x), fma(-t[0].x, L.P[0].x, L.P[0].y));
+    const double2 fl = make_double2(fma(gl, pl.y, pl.x), fma(-gl, pl.x, pl.y));
+    const int lane = lane_id();
+    if (lane == 0) E.f0 = f0;
+    if (lane == 63) E.a = fl;
+    const double2 fR = dpp2_z<kWaveShl1>(f0);
+    const double2 fL = dpp2_z<kWaveShr1>(fl);
+    double2 dm = make_double2(f0.x - fL.x, f0.y - fL.y), fc = f0;
+    double s0 = 0.0, s1 = 0.0;
+    const double twelve = 12.0;
+#pragma unroll
+    for (int i = 0; i < C; i++) {
+        const double2 p = L.P[i], tt = t[i % kRows];
+        const double n2 = fma(p.x, p.x, p.y * p.y);
+        s0 += n2;
+        s1 = fma((double)i, n2, s1);
+        acc.gp = fma(n2, tt.y, acc.gp);
+        if (CORE) {
+            const double2 w = q[i % kCore];
+            acc.pr = fma(p.x, w.x, acc.pr);
+            acc.pi = fma(-p.y, w.x, acc.pi);
+            acc.pint = fma(n2, w.y, acc.pint);
+            asm volatile("" : "+v"(acc.pr), "+v"(acc.pi), "+v"(acc.pint));
+            if (i + kCore < C) q[i % kCore] = row(cq, coff, i + kCore);
+        }
+        double2 fp = fR;
+        if (i + 1 < C) {
+            const double gn = t[(i + 1) % kRows].x;
+            fp = make_double2(fma(gn, L.P[i + 1].y, L.P[i + 1].x), fma(-gn, L.P[i + 1].x, L.P[i + 1].y));
+        }
+        const double2 dp = make_double2(fp.x - fc.x, fp.y - fc.y);
+        const double v = fma(twelve, tt.x, K.k36);
+        L.P[i] = make_double2(fma(v, p.y, fma(twelve, p.x, dp.x - dm.x)), fma(-v, p.x, fma(twelve, p.y, dp.y - dm.y)));
+        // formed here, not where they are used: that would keep every operand alive
+        asm volatile("" : "+v"(s0), "+v"(s1), "+v"(acc.gp), "+v"(L.P[i].x), "+v"(L.P[i].y));
+        dm = dp;
+        fc = fp;
+        if (i + kRows < C) t[i % kRows] = row(gv, L.off, i + kRows);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    acc.pos = fma(grid_x(L.j0, K.dx, K.xmax), s0, K.dx * s1);
+}
+
+// One time step of the window's points.  rot: exp(-i F dt dx) - 1, from a point's phase to the one before.  ring: this wave's ring entry for the state it starts from.
+template <int C, bool CORE>
+__device__ inline void step(const TdseResident &R, const StepConst &K, Lane<C> &L, const double2 *gv,
+                            const double2 *rs, const double2 *lb, const Shared &sh, int wave, double F, double2 rot, bool deep,
+                            bool add, double *ring)
 {
     using LN = Lane<C>;
-    constexpr int NL = LN::NL, kRows = rows_first(C), kRows4 = rows_last(C), kLds1 = lds_ends(C), kLds = lds_between(C);
-    double2 e, rot;  // exp(i F dt x) at the lane's last point; exp(-i F dt dx) - 1, to the point before
+    constexpr int NL = LN::NL, kRows4 = rows_last(C), kLds1 = lds_ends(C), kLds = lds_between(C);
+    double2 e;  // exp(i F dt x) at the lane's last point
     double2 carry;
+    Acc acc = {0.0, 0.0, 0.0, 0.0, 0.0};
+    TdseWaveEdge &E = sh.edge[wave];
+    first_pass<C, CORE>(R, K, L, gv, acc, E);
+    __builtin_amdgcn_sched_barrier(0);
+    fetch_far<C>(L);
+    __builtin_amdgcn_sched_barrier(0);
     {
-        // pass 1: observables, r in place, and y from zero
-        double2 t[kRows], bq[kLds1];
+        // y from zero
+        double2 bq[kLds];
 #pragma unroll
-        for (int i = 0; i < kRows && i < C; i++) t[i] = row(gv, L.off, i);
-#pragma unroll
-        for (int i = 0; i < kLds1 && i < NL; i++) bq[i] = lb[i * 64];
-        Acc acc = {0.0, 0.0, 0.0, 0.0, 0.0};
-        if (core) observe_core<C>(R, L, chunk, acc);  // a wave that holds part of the atom
-        const double2 pl = L.P[C - 1];
-        const double2 f0 = make_double2(fma(t[0].x, L.P[0].y, L.P[0].x), fma(-t[0].x, L.P[0].x, L.P[0].y));
-        const double2 fl = make_double2(fma(L.gl, pl.y, pl.x), fma(-L.gl, pl.x, pl.y));
-        const double2 fR = dpp2_z<kWaveShl1>(f0);
-        const double2 fL = dpp2_z<kWaveShr1>(fl);
-        double2 dm = make_double2(f0.x - fL.x, f0.y - fL.y), fc = f0;
-        double2 y = make_double2(0.0, 0.0), bp = make_double2(0.0, 0.0);
-        double s0 = 0.0, s1 = 0.0;
-        const double twelve = 12.0;
+        for (int i = 0; i < kLds && i < NL; i++) bq[i] = lb[i * 64];
+        double2 y = make_double2(0.0, 0.0), b = y;
 #pragma unroll
         for (int i = 0; i < C; i++) {
-            const double2 p = L.P[i], tt = t[i % kRows];
-            const double n2 = fma(p.x, p.x, p.y * p.y);
-            s0 += n2;
-            s1 = fma((double)i, n2, s1);
-            acc.gp = fma(n2, tt.y, acc.gp);
-            double2 fp = fR;
-            if (i + 1 < C) {
-                const double gn = t[(i + 1) % kRows].x;
-                fp = make_double2(fma(gn, L.P[i + 1].y, L.P[i + 1].x), fma(-gn, L.P[i + 1].x, L.P[i + 1].y));
-            }
-            const double2 dp = make_double2(fp.x - fc.x, fp.y - fc.y);
-            const double v = fma(twelve, tt.x, K.k36);
-            const double2 r = make_double2(fma(v, p.y, fma(twelve, p.x, dp.x - dm.x)), fma(-v, p.x, fma(twelve, p.y, dp.y - dm.y)));
-            L.P[i] = r;
-            y = i > 0 ? cfms(bp, y, r) : r;
-            // summed here, not where the sums are used: that would keep every operand alive
-            asm volatile("" : "+v"(y.x), "+v"(y.y), "+v"(s0), "+v"(s1), "+v"(acc.gp));
-            dm = dp;
-            fc = fp;
-            bp = i < NL ? bq[i % kLds1] : b_at<C>(L, lb, i);
-            if (i + kRows < C) t[i % kRows] = row(gv, L.off, i + kRows);
-            if (i + kLds1 < NL) bq[i % kLds1] = lb[(i + kLds1) * 64];
-            __builtin_amdgcn_sched_barrier(0);
+            y = i > 0 ? cfms(b, y, L.P[i]) : L.P[i];
+            asm volatile("" : "+v"(y.x), "+v"(y.y));
+            b = i < NL ? bq[i % kLds] : b_at<C>(L, lb, i);
+            if (i + kLds < NL) bq[i % kLds] = lb[(i + kLds) * 64];
+            if (i % 2 == 0) __builtin_amdgcn_sched_barrier(0);
         }
         // what the chunk hands to the next lane's first row: -b y of its last point
-        const double2 nb = make_double2(-bp.x, -bp.y);
-        double2 Q = L.nQ, z = cmul(nb, y);
+        const double2 nb = make_double2(-b.x, -b.y);
+        double2 Q = C > 24 ? lb[64 * NL] : L.nQ, z = cmul(nb, y);
         scan_wave<true>(Q, z, deep);
-        WaveEdge &E = sh.edge[wave];
+        const int lane = lane_id();
         if (lane == 63) {
-            E.a = make_double2(fl.x + z.x, fl.y + z.y);
+            E.a = make_double2(E.a.x + z.x, E.a.y + z.y);
             E.nb = nb;
         }
-        if (lane == 0) E.f0 = f0;
         // while the other waves arrive: the phase factors and the observables' sums
         {
-            const double Fdt = F * K.dt, th = Fdt * grid_x(L.j0 + C - 1, K.dx, K.xmax), d = Fdt * K.dx;
-            sincos_wide(th, &e.y, &e.x);
-            double hs, hc;
-            sincos_wide(-0.5 * d, &hs, &hc);
-            rot = make_double2(-2.0 * hs * hs, 2.0 * hs * hc);
+            const double th = F * K.dt * grid_x(L.j0 + C - 1, K.dx, K.xmax);
+            sincos_lean(th, &e.y, &e.x);
         }
-        acc.pos = fma(grid_x(L.j0, K.dx, K.xmax), s0, K.dx * s1);
-        put_observables(acc, L.own, core, add, lane, ring);
+        put_observables(acc, L.own, CORE, add, lane, ring);
         lds_barrier();
         // from the wave before: its last point's f, and its carry corrected for the f of this wave's
         // first point, which its last row was still missing
         double2 Z = make_double2(0.0, 0.0);
-        if (wave > 0) {
-            const WaveEdge &B = sh.edge[wave - 1];
+        if (per_lane(wave) > 0) {
+            const TdseWaveEdge &B = sh.edge[wave - 1];
             Z = cfma(B.nb, E.f0, B.a);
         }
         carry = lane_carry<true>(Q, z, Z, lane);
@@ -407,40 +535,41 @@ __device__ inline void step(const TdseResident &R, const StepConst &K, Lane<C> &
         L.P[C - 1].x += lane == 63 ? fn.x : 0.0;
         L.P[C - 1].y += lane == 63 ? fn.y : 0.0;
     }
-    // pass 2: y from the true carry, in place
+    // w from the true carry, in place
     {
         double2 bq[kLds];
 #pragma unroll
         for (int i = 0; i < kLds && i < NL; i++) bq[i] = lb[i * 64];
-        double2 y = make_double2(L.P[0].x + carry.x, L.P[0].y + carry.y);
-        L.P[0] = y;
+        double2 w = make_double2(-carry.x, -carry.y);
 #pragma unroll
-        for (int i = 1; i < C; i++) {
-            const double2 b = i - 1 < NL ? bq[(i - 1) % kLds] : b_at<C>(L, lb, i - 1);
-            y = cfms(b, y, L.P[i]);
-            asm volatile("" : "+v"(y.x), "+v"(y.y));
-            L.P[i] = y;
-            if (i - 1 + kLds < NL) bq[(i - 1) % kLds] = lb[(i - 1 + kLds) * 64];
+        for (int i = 0; i < C; i++) {
+            const double2 b = i < NL ? bq[i % kLds] : b_at<C>(L, lb, i);
+            w = cmul(b, make_double2(L.P[i].x - w.x, L.P[i].y - w.y));
+            asm volatile("" : "+v"(w.x), "+v"(w.y));
+            L.P[i] = w;
+            if (i + kLds < NL) bq[i % kLds] = lb[(i + kLds) * 64];
             if (i % 2 == 0) __builtin_amdgcn_sched_barrier(0);
         }
     }
-    // pass 3: phi from zero, for the carry to the lane before
+    // phi from zero, for the carry to the lane before
     double2 s[kRows4], bq[kLds];
     {
+        constexpr int i0 = NL < C - 1 ? NL - 1 : C - 2;  // the first b from LDS
 #pragma unroll
         for (int i = 0; i < kLds; i++)
-            if (NL - 1 - i >= 0) bq[(NL - 1 - i) % kLds] = lb[(NL - 1 - i) * 64];
-        double2 u = make_double2(0.0, 0.0);
+            if (i0 - i >= 0) bq[(i0 - i) % kLds] = lb[(i0 - i) * 64];
+        double2 u = L.P[C - 1];
 #pragma unroll
-        for (int i = C - 1; i >= 0; i--) {
+        for (int i = C - 2; i >= 0; i--) {
             const double2 b = i < NL ? bq[i % kLds] : b_at<C>(L, lb, i);
-            u = cmul(b, make_double2(L.P[i].x - u.x, L.P[i].y - u.y));
+            u = cfms(b, u, L.P[i]);
             asm volatile("" : "+v"(u.x), "+v"(u.y));
             if (i < NL && i - kLds >= 0) bq[i % kLds] = lb[(i - kLds) * 64];
             if (i % 2 == 0) __builtin_amdgcn_sched_barrier(0);
         }
-        double2 Q = L.nQ;
+        double2 Q = C > 24 ? lb[64 * NL] : L.nQ;
         scan_wave<false>(Q, u, deep);
+        const int lane = lane_id();
         if (lane == 0) sh.edge[wave].up = u;
         // the rows of the last pass, in flight across the barrier
 #pragma unroll
@@ -452,13 +581,13 @@ __device__ inline void step(const TdseResident &R, const StepConst &K, Lane<C> &
         lds_barrier();
         carry = lane_carry<false>(Q, u, sh.edge[wave + 1].up, lane);
     }
-    // pass 4: phi from the true carry, psi' = phi / (1 + i g), the phase
+    // phi from the true carry, psi' = phi / (1 + i g), the phase
     {
         double2 u = carry;
 #pragma unroll
         for (int i = C - 1; i >= 0; i--) {
             const double2 b = i < NL ? bq[i % kLds1] : b_at<C>(L, lb, i);
-            u = cmul(b, make_double2(L.P[i].x - u.x, L.P[i].y - u.y));
+            u = cfms(b, u, L.P[i]);
             L.P[i] = cmul(e, cmul(s[i % kRows4], u));
             asm volatile("" : "+v"(u.x), "+v"(u.y), "+v"(L.P[i].x), "+v"(L.P[i].y));
             if (i > 0) e = cfma(e, rot, e);  // e + e rot: the rotation's own rounding would change |e| by C steps of it
@@ -469,118 +598,179 @@ __device__ inline void step(const TdseResident &R, const StepConst &K, Lane<C> &
     }
 }
 
+// What a run of steps does with its observables: entry t of the ring is sample k + t.
+struct Entries {
+    const TdseInst *inst;
+    int k, k_start, gate, waves;
+    bool flush;  // while the steps run (one window)
+};
+
+// Samples e.k + t, t0 <= t < t1, from the waves' sums, one per lane of this wave.
+__device__ inline void write_entries(const Entries &e, const Shared &sh, int t0, int t1, int mask)
+{
+    const TdseInst &I = fresh(*e.inst);
+    const int t = t0 + lane_id(), idx = e.k + t;
+    if (!I.src || t >= t1 || idx <= e.k_start) return;
+    double sum[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+    for (int w = 0; w < e.waves; w++)
+        for (int q = 0; q < 5; q++) sum[q] += sh.sums(t & mask, w)[q];
+    const double F = idx - 1 <= e.gate ? 0.0 : I.field[idx - 1];  // the step that produced the state
+    I.src[idx] = -sum[4] + F;
+    I.ptot[idx] = sum[0] * sum[0] + sum[1] * sum[1];
+    I.pint[idx] = sum[2];
+    I.expv[idx] = sum[3];
+    if (I.efield) I.efield[idx] = F;
+}
+
+// nb steps of the window's points.  The ring's halves are written out by the first wave in turn, while the others go
+// on: they come back to a half after more barriers than that takes.  The waves that hold part of the atom
+// run a loop of their own: with both in one, either the registers or the loads in flight of the others pay for
+// what only those need.
+template <int C, bool CORE>
+__device__ inline void run_steps(const TdseResident &R, const StepConst &K, Lane<C> &L, const double2 *lb, const Shared &sh,
+                                 int wave, const Entries &e, int nb, bool deep, bool add)
+{
+    constexpr int kHalf = TDSE_RES_RING / 2;
+    for (int t0 = 0; t0 < nb; t0 += kHalf) {
+        const int m = t0 + lane_id(), t1 = min(nb, t0 + kHalf);
+        const double fields = m < t1 && e.k + m > e.gate ? fresh(*e.inst).field[e.k + m] : 0.0;
+        double hs, hc;
+        sincos_lean(-0.5 * (fields * K.dt * K.dx), &hs, &hc);
+        const double2 rots = make_double2(-2.0 * hs * hs, 2.0 * hs * hc);
+        for (int t = t0; t < t1; t++)
+            step<C, CORE>(R, K, L, opaque(R.gv), opaque(R.s), lb, sh, wave, readlane(fields, t - t0), readlane2(rots, t - t0), deep,
+                          add, sh.sums(t % TDSE_RES_RING, wave));
+        if (e.flush && t1 - t0 == kHalf && per_lane(wave) == 0) write_entries(e, sh, t0, t1, TDSE_RES_RING - 1);
+    }
+}
+
 // The whole run of one instance by the waves of a workgroup.
 template <int C>
-__device__ inline void run_instance(const TdseGeom &G, const TdseInst &I, double2 *work, long long work_stride, double2 *lds,
-                                    Shared &sh)
+__device__ inline void run_instance(const TdseGeom &geom, const TdseInst &inst, double2 *work, long long work_stride, double2 *far,
+                                    const Shared &sh, Queue &queue)
 {
     using LN = Lane<C>;
-    const TdseResident &R = G.res;
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int nw = R.waves;
-    const bool live = wave < nw;
-    const bool deep = R.reach > 8 * C;
-    const bool windows = R.windows > 1;
-    const int k_start = I.k0, k_stop = I.n_run > 0 ? I.k0 + I.n_run : I.n_steps;
-    const bool final_obs = I.src && k_stop < I.n_steps;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int nw = geom.res.waves;
+    const bool live = per_lane(wave) < nw;
+    const bool deep = geom.res.reach > 8 * C;
+    const bool windows = geom.res.windows > 1;
+    const int k_start = inst.k0, k_stop = inst.n_run > 0 ? inst.k0 + inst.n_run : inst.n_steps;
     int i_snap = 0;
     int cur = 0;  // multi-window states: the buffer that holds the current state
-    // the field is 0 up to and including the first sign change of in_field (prop.c:125-134)
-    if (threadIdx.x == 0) sh.gate = I.pregated ? -1 : I.n_steps;
-    __syncthreads();
-    for (int m0 = 0; !I.pregated && m0 < k_stop; m0 += blockDim.x) {
-        const int m = m0 + (int)threadIdx.x;
-        if (m < k_stop && I.field[m] * I.field[m + 1] <= 0.0) atomicMin(&sh.gate, m);
+    {
+        const TdseGeom &G = geom;
+        const TdseInst &I = inst;
+        // the field is 0 up to and including the first sign change of in_field (prop.c:125-134)
+        if (threadIdx.x == 0) queue.gate = I.pregated ? -1 : I.n_steps;
         __syncthreads();
-        const bool found = sh.gate < I.n_steps;
-        __syncthreads();
-        if (found) break;
-    }
-    const int gate = __builtin_amdgcn_readfirstlane(sh.gate);
-    auto field = [&](int m) { return m <= gate ? 0.0 : I.field[m]; };
-    if (threadIdx.x == 0) {
-        const double2 zero = make_double2(0.0, 0.0);
-        sh.edge[nw].f0 = zero;  // past the last wave: the wall, or a window's end
-        sh.edge[nw].up = zero;
-        if (I.src && k_start == 0) {
-            I.src[0] = 0.0;
-            I.ptot[0] = 1.0;
-            I.pint[0] = G.pint0;
-            I.expv[0] = 0.0;
-            if (I.efield) I.efield[0] = 0.0;
+        for (int m0 = 0; !I.pregated && m0 < k_stop; m0 += blockDim.x) {
+            const int m = m0 + (int)threadIdx.x;
+            if (m < k_stop && I.field[m] * I.field[m + 1] <= 0.0) atomicMin(&queue.gate, m);
+            __syncthreads();
+            const bool found = queue.gate < I.n_steps;
+            __syncthreads();
+            if (found) break;
         }
+        if (threadIdx.x == 0) {
+            const double2 zero = make_double2(0.0, 0.0);
+            sh.edge[nw].f0 = zero;  // past the last wave: the wall, or a window's end
+            sh.edge[nw].up = zero;
+            if (I.src && k_start == 0) {
+                I.src[0] = 0.0;
+                I.ptot[0] = 1.0;
+                I.pint[0] = G.pint0;
+                I.expv[0] = 0.0;
+                if (I.efield) I.efield[0] = 0.0;
+            }
+        }
+        __syncthreads();
     }
-    __syncthreads();
-    double2 *const lb = lds + wave * (64 * LN::NL) + lane;  // this lane's b: point i at lb[i * 64]
+    const int gate = __builtin_amdgcn_readfirstlane(queue.gate);
+    double2 *const lb = sh.b + wave * (64 * tdse_res_lds_rows(C)) + lane;  // this lane's b: point i at lb[i * 64]
     LN L;
-    const StepConst K = step_const(G);
-    const double2 *const gv = R.gv, *const rs = R.s;
-    bool core = false;
+    const StepConst K = step_const(fresh(geom));
+    int core = 0;
     int chunk = 0;
-    auto place = [&](int w) { place_lane<C>(R, w, wave, lane, L, chunk, core); };
-    // chunk c's rows in a window buffer
-    auto buf_off = [&](int w) { return row_offset<C>(w * R.stride + wave * 64 + lane); };
+    // prop.c:248-255: snapshot row i_snap gets psi after step m when m % every == 0; the next such step
+    auto snap_step = [&](const TdseInst &I, int k) {
+        return I.snap && i_snap < I.n_snap - 1 ? (k + I.snap_every - 1) / I.snap_every * I.snap_every : 0x7ffffffe;
+    };
 
     for (int k = k_start; k < k_stop;) {
-        int nb = min(R.steps, k_stop - k);
-        if (I.save) nb = min(nb, I.save_every - (k - k_start) % I.save_every);
-        // prop.c:248-255: snapshot row i_snap gets psi after step m when m % every == 0
-        const int snap_step = (k + I.snap_every - 1) / I.snap_every * I.snap_every;
-        const bool snaps = I.snap && i_snap < I.n_snap - 1;
-        if (snaps) nb = min(nb, snap_step + 1 - k);
+        int nb;
+        {
+            const TdseInst &I = fresh(inst);
+            nb = windows ? min(fresh(geom).res.steps, k_stop - k) : k_stop - k;
+            if (I.save) nb = min(nb, I.save_every - (k - k_start) % I.save_every);
+            nb = min(nb, snap_step(I, k) + 1 - k);
+        }
         // who gets the state the block ends with: a save (tiled), a snapshot, and after the last step (prop.c:256-262) the
         // last row, if every earlier one was used, and the final state
-        double2 *const save = I.save && (k + nb - k_start) % I.save_every == 0
-                                  ? I.save + (long long)((k + nb - k_start) / I.save_every - 1) * G.npad
-                                  : nullptr;
-        double *row_to[3] = {nullptr, nullptr, nullptr};
-        if (snaps && k + nb == snap_step + 1) row_to[0] = I.snap + 2ll * G.nx * i_snap++;
-        if (k + nb == k_stop) {
-            if (I.snap && i_snap == I.n_snap - 1) row_to[1] = I.snap + 2ll * G.nx * i_snap;
-            row_to[2] = I.psi_final;
-        }
-        for (int w = 0; w < R.windows; w++) {
+        double *to[4];
+        auto receivers = [&] {
+            const TdseInst &I = fresh(inst);
+            const TdseGeom &G = fresh(geom);
+            to[0] = I.save && (k + nb - k_start) % I.save_every == 0
+                        ? reinterpret_cast<double *>(I.save + (long long)((k + nb - k_start) / I.save_every - 1) * G.npad)
+                        : nullptr;
+            const bool at_snap = k + nb == snap_step(I, k) + 1;
+            to[1] = at_snap ? I.snap + 2ll * G.nx * i_snap : nullptr;
+            to[2] = k + nb == k_stop && I.snap && i_snap + at_snap == I.n_snap - 1 ? I.snap + 2ll * G.nx * (i_snap + at_snap)
+                                                                               : nullptr;
+            to[3] = k + nb == k_stop ? I.psi_final : nullptr;
+            return at_snap;
+        };
+        bool at_snap = false;
+        for (int w = 0; w == 0 || w < fresh(geom).res.windows; w++) {
             const bool add = w > 0;
             if (live && (windows || k == k_start)) {
-                place(w);
-                load_b<C>(G, R, L, lb);
+                const TdseGeom &G = fresh(geom);
+                const TdseInst &I = fresh(inst);
+                place_lane<C>(G.res, w, wave, lane, L, chunk, core);
+                load_b<C>(G.res, L, lb, far + wave * tdse_res_far(1, C) + lane);
                 if (k == k_start) {
                     load_tiled<C>(G, L, I.psi_init ? I.psi_init : G.psi0);
                 } else {
                     const double2 *src = work + cur * work_stride;
-                    const unsigned o = buf_off(w);
+                    const unsigned o = row_offset<C>(chunk);  // (a window's chunks lie in its buffer as in the grid)
 #pragma unroll
                     for (int i = 0; i < C; i++) L.P[i] = row(src, o, i);
                 }
             }
-            // the block's fields, one per lane
-            const double fields = lane < nb ? field(k + lane) : 0.0;
-            for (int t = 0; t < nb; t++) {
-                if (live) {
-                    step<C>(R, K, L, chunk, opaque(gv), opaque(rs), lb, sh, wave, lane, readlane(fields, t), core, deep, add,
-                            sh.ring[t][wave]);
-                } else {
+            const Entries entries = {&inst, k, k_start, gate, nw, !windows};
+            if (!live) {
+                for (int t = 0; t < nb; t++) {
                     lds_barrier();
                     lds_barrier();
                 }
+            } else if (per_lane(core)) {
+                run_steps<C, true>(fresh(geom).res, K, L, lb, sh, wave, entries, nb, deep, add);
+            } else {
+                run_steps<C, false>(fresh(geom).res, K, L, lb, sh, wave, entries, nb, deep, add);
             }
+            at_snap = receivers();
             if (live) {
-                if (final_obs && k + nb == k_stop) observe_only<C>(G, L, chunk, gv, core, add, lane, sh.ring[nb][wave]);
+                const TdseGeom &G = fresh(geom);
+                const TdseInst &I = fresh(inst);
+                if (I.src && k_stop < I.n_steps && k + nb == k_stop)
+                    observe_only<C>(G, L, G.res.gv, core, add, lane,
+                                    sh.sums(windows ? nb : nb % TDSE_RES_RING, wave));
                 if (windows) {
                     double2 *dst = work + (cur ^ 1) * work_stride;
-                    const unsigned o = buf_off(w);
+                    const unsigned o = row_offset<C>(chunk);
                     if (L.own) {
 #pragma unroll
                         for (int i = 0; i < C; i++) st2((double2 *)((char *)dst + o), 64 * i, L.P[i]);
                     }
-                } else {
+                } else if (to[0] || to[1] || to[2] || to[3]) {
                     for (int m = 0; m < 4; m++) {
-                        double *dst = m < 3 ? row_to[m] : reinterpret_cast<double *>(save);
+                        double *dst = to[m];
                         if (!dst) continue;
 #pragma unroll
                         for (int i = 0; i < C; i++) {
                             const int j = L.j0 + i;
-                            if (j >= 0 && j < G.nx) put_state(dst, m < 3 ? j : tdse_index(j), L.P[i]);
+                            if (j >= 0 && j < G.nx) put_state(dst, m > 0 ? j : tdse_index(j), L.P[i]);
                             __builtin_amdgcn_sched_barrier(0);
                         }
                     }
@@ -589,33 +779,27 @@ __device__ inline void run_instance(const TdseGeom &G, const TdseInst &I, double
         }
         __syncthreads();  // the ring is complete, a window buffer is in memory
         if (windows) {
+            const TdseGeom &G = fresh(geom);
             cur ^= 1;
             const double2 *src = work + cur * work_stride;
             for (int m = 0; m < 4; m++) {
-                double *dst = m < 3 ? row_to[m] : reinterpret_cast<double *>(save);
+                double *dst = to[m];
                 if (!dst) continue;
                 for (int j = threadIdx.x; j < G.nx; j += blockDim.x) {
-                    const int q = j + R.lead, c = q / C;
-                    put_state(dst, m < 3 ? j : tdse_index(j), src[(long long)(c >> 6) * (C * 64) + (q % C) * 64 + (c & 63)]);
+                    const int q = j + G.res.lead, c = q / C;
+                    put_state(dst, m > 0 ? j : tdse_index(j), src[(long long)(c >> 6) * (C * 64) + (q % C) * 64 + (c & 63)]);
                 }
             }
         }
-        // entries k .. k + nb - 1 of the outputs (and k + nb, the last state of a partial run)
-        if (I.src && threadIdx.x <= (unsigned)nb) {
-            const int t = threadIdx.x, idx = k + t;
-            if (idx > k_start && (t < nb || (final_obs && idx == k_stop))) {
-                double sum[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
-                for (int w = 0; w < nw; w++)
-                    for (int q = 0; q < 5; q++) sum[q] += sh.ring[t][w][q];
-                const double F = field(idx - 1);  // the step that produced the state
-                I.src[idx] = -sum[4] + F;
-                I.ptot[idx] = sum[0] * sum[0] + sum[1] * sum[1];
-                I.pint[idx] = sum[2];
-                I.expv[idx] = sum[3];
-                if (I.efield) I.efield[idx] = F;
-            }
+        // what is left in the ring, and the last state of a partial run
+        if (wave == 0) {
+            const Entries entries = {&inst, k, k_start, gate, nw, false};
+            const int from = windows ? 0 : nb / (TDSE_RES_RING / 2) * (TDSE_RES_RING / 2);
+            const bool last = k + nb == k_stop && k_stop < fresh(inst).n_steps;
+            write_entries(entries, sh, from, nb + last, windows ? 31 : TDSE_RES_RING - 1);
         }
         __syncthreads();  // the ring has been read
+        i_snap += at_snap;
         k += nb;
     }
 }
@@ -623,27 +807,30 @@ __device__ inline void run_instance(const TdseGeom &G, const TdseInst &I, double
 } // namespace
 
 // Persistent workgroups: instances from the per-XCD queues as in tdse_propagate_kernel, each by
-// the chunk length of its geometry.  Dynamic LDS: lds_points(C) complex doubles per lane.
+// the chunk length of its geometry.  Dynamic LDS: tdse_res_lds().
 __global__ void __launch_bounds__(64 * TDSE_MAX_WAVES, TDSE_RES_WAVES_PER_SIMD)
 tdse_resident_kernel(const TdseGeom *__restrict__ geoms, const TdseInst *__restrict__ insts, const int *__restrict__ order,
                      TdseQueues queues, int *counter, double2 *work, long long work_stride)
 {
-    __shared__ Shared sh;
+    __shared__ Queue queue;
     extern __shared__ double2 lds[];
-    if (threadIdx.x == 0) sh.tried = 0;
+    const Shared sh = shared_memory(lds);
+    if (threadIdx.x == 0) queue.tried = 0;
     for (;;) {
-        if (threadIdx.x == 0) sh.cur = next_instance(queues, counter, sh.tried);
+        if (threadIdx.x == 0) queue.cur = next_instance(queues, counter, queue.tried);
         __syncthreads();
-        const int t = __builtin_amdgcn_readfirstlane(sh.cur);
+        const int t = __builtin_amdgcn_readfirstlane(queue.cur);
         __syncthreads();
         if (t < 0) break;
-        const TdseInst &I = insts[order[t]];
-        const TdseGeom &G = geoms[I.geom];
-        double2 *const buf = work + 2 * (long long)blockIdx.x * work_stride;
+        const TdseInst &I = insts[__builtin_amdgcn_readfirstlane(order[t])];
+        const TdseGeom &G = geoms[__builtin_amdgcn_readfirstlane(I.geom)];
+        // two states of the windows, and the lanes' own b that registers do not hold
+        double2 *const buf = work + (long long)blockIdx.x * work_stride;
+        const long long states = (work_stride - tdse_res_far(TDSE_MAX_WAVES, 32)) / 2;
         switch (G.res.chunk) {
-        case 16: run_instance<16>(G, I, buf, work_stride, lds, sh); break;
-        case 24: run_instance<24>(G, I, buf, work_stride, lds, sh); break;
-        case 32: run_instance<32>(G, I, buf, work_stride, lds, sh); break;
+        case 16: run_instance<16>(G, I, buf, states, buf + 2 * states, sh, queue); break;
+        case 24: run_instance<24>(G, I, buf, states, buf + 2 * states, sh, queue); break;
+        case 32: run_instance<32>(G, I, buf, states, buf + 2 * states, sh, queue); break;
         default: break;
         }
     }
@@ -674,22 +861,22 @@ __device__ inline void store_entries(const TdseInst &I, const double *part, int 
 
 template <int C>
 __device__ inline void run_window(const TdseGeom &G, const TdseInst &I, const TdseResident &R, int k, int nb,
-                                  const double2 *src, double2 *dst, double *part, double2 *lds, Shared &sh)
+                                  const double2 *src, double2 *dst, double *part, const Shared &sh)
 {
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, w = blockIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6), lane = threadIdx.x & 63, w = blockIdx.x;
     const bool deep = R.reach > 8 * C;
-    double2 *const lb = lds + wave * (64 * Lane<C>::NL) + lane;
+    double2 *const lb = sh.b + wave * (64 * tdse_res_lds_rows(C)) + lane;
     Lane<C> L;
     const StepConst K = step_const(G);
-    const double2 *const gv = R.gv, *const rs = R.s;
-    bool core = false;
+    const double2 *const gv = R.gv;
+    int core = 0;
     int chunk = 0;
     if (threadIdx.x == 0) {
         sh.edge[R.waves].f0 = make_double2(0.0, 0.0);
         sh.edge[R.waves].up = make_double2(0.0, 0.0);
     }
     place_lane<C>(R, w, wave, lane, L, chunk, core);
-    load_b<C>(G, R, L, lb);
+    load_b<C>(R, L, lb, nullptr);
     const bool on_grid = L.j0 < G.nx;
     if (src) {
         const unsigned o = row_offset<C>(on_grid ? chunk : 0);
@@ -701,11 +888,12 @@ __device__ inline void run_window(const TdseGeom &G, const TdseInst &I, const Td
     } else {
         load_tiled<C>(G, L, G.psi0);
     }
-    const double fields = lane < nb ? I.field[k + lane] : 0.0;
+    const Entries entries = {&I, k, 0, -1, R.waves, false};
     __syncthreads();
-    for (int t = 0; t < nb; t++)
-        step<C>(R, K, L, chunk, opaque(gv), opaque(rs), lb, sh, wave, lane, readlane(fields, t), core, deep, false,
-                sh.ring[t][wave]);
+    if (per_lane(core))
+        run_steps<C, true>(R, K, L, lb, sh, wave, entries, nb, deep, false);
+    else
+        run_steps<C, false>(R, K, L, lb, sh, wave, entries, nb, deep, false);
     if (L.own && on_grid) {
         const unsigned o = row_offset<C>(chunk);
 #pragma unroll
@@ -714,7 +902,7 @@ __device__ inline void run_window(const TdseGeom &G, const TdseInst &I, const Td
     __syncthreads();
     for (int e = threadIdx.x; e < 5 * nb; e += blockDim.x) {
         double sum = 0.0;
-        for (int v = 0; v < R.waves; v++) sum += sh.ring[e / 5][v][e % 5];
+        for (int v = 0; v < R.waves; v++) sum += sh.sums(e / 5, v)[e % 5];
         part[((e / 5) * R.windows + w) * 5 + e % 5] = sum;
     }
 }
@@ -729,8 +917,8 @@ __global__ void __launch_bounds__(64 * TDSE_ONE_WAVES)
 tdse_window_kernel(const TdseGeom *__restrict__ geom, const TdseInst *__restrict__ inst, TdseResident R, int k, int nb, int nb_prev,
                    int launch, const double2 *src, double2 *dst, double *part)
 {
-    __shared__ Shared sh;
     extern __shared__ double2 lds[];
+    const Shared sh = shared_memory(lds);
     const TdseGeom &G = *geom;
     const TdseInst &I = *inst;
     const long long half = (long long)TDSE_RES_RING * R.windows * 5;
@@ -747,9 +935,9 @@ tdse_window_kernel(const TdseGeom *__restrict__ geom, const TdseInst *__restrict
     }
     double *const mine = part + (launch & 1) * half;
     if (R.chunk == 16)
-        run_window<16>(G, I, R, k, nb, src, dst, mine, lds, sh);
+        run_window<16>(G, I, R, k, nb, src, dst, mine, sh);
     else
-        run_window<24>(G, I, R, k, nb, src, dst, mine, lds, sh);
+        run_window<24>(G, I, R, k, nb, src, dst, mine, sh);
 }
 
 // The entries of the run's last launch.
@@ -876,16 +1064,16 @@ __global__ void tdse_resident_tables_kernel(const double *g, const double *dpot,
     }
 }
 
-// Per geometry (job blockIdx.y), the core table: entry (i, c) is point (core_chunk0 + c) C + i - lead, {Re psi0,
-// 1 in the PopInt window [lo, hi]} and Im psi0, zero outside the grid; and b of its first `head` points,
-// which feel its own left wall where the lattice's do not.
+// Per geometry (job blockIdx.y), the core table: chunk c of n (n_tiles tiles of 64; zeros from n on), row i, is
+// point (core_chunk0 + c) C + i - lead, {Re psi0, 1 in the PopInt window [lo, hi]} and Im psi0, zero outside
+// the grid; and b of its first `head` points, which feel its own left wall where the lattice's do not.
 __global__ void tdse_resident_core_kernel(const ResidentJob *jobs)
 {
     const ResidentJob J = jobs[blockIdx.y];
-    const int m = J.C * J.n;
+    const int m = J.C * 64 * J.n_tiles;
     for (int q = blockIdx.x * blockDim.x + threadIdx.x; q < m; q += gridDim.x * blockDim.x) {
-        const int j = J.first + (q % J.n) * J.C + q / J.n;
-        const bool on = j >= 0 && j < J.nx;
+        const int c = q / (64 * J.C) * 64 + q % 64, j = J.first + c * J.C + q / 64 % J.C;
+        const bool on = c < J.n && j >= 0 && j < J.nx;
         J.core[q] = make_double2(on ? J.psi0[j].x : 0.0, on && j >= J.lo && j <= J.hi ? 1.0 : 0.0);
         J.im[q] = on ? J.psi0[j].y : 0.0;
     }

@@ -55,6 +55,23 @@ def test_shared_lattice_offsets():
         agree(tdse.propagate_one(geo, dev[i].contiguous()), got[i])
 
 
+# 32 points a lane read part of the factor from the lattice's table again in every step, and near a grid's own
+# left wall and past its end, where the table is another grid's, from a copy of their own
+@pytest.mark.parametrize("sizes", [[16382, 16380, 15000, 14222, 12990], [16001, 13001, 12289], [16382, 20000, 402, 16000]])
+def test_shared_lattice_with_32_points(sizes):
+    geos = tdse.Geometry.create_many(sizes, 0.1, 0.25, W.GRID["a"], W.GRID["e_guess"], W.UNEVEN_CV, 2.0)
+    dev = fields(len(sizes))
+    agree(tdse.propagate_batch(geos, dev), tdse.BatchPlan(geos, dev, config=SHAPE).enqueue())
+
+
+# the ring of observables is written out in halves of 8 steps
+@pytest.mark.parametrize("nx", [2001, 9001, 13001, 17001])
+@pytest.mark.parametrize("steps", [1, 2, 7, 8, 9, 16, 17, 24, 31])
+def test_run_lengths(nx, steps):
+    geo, dev = geometry(nx - 1), fields()[:, :steps + 1].contiguous()
+    agree(tdse.propagate_batch(geo, dev), tdse.BatchPlan(geo, dev, config=SHAPE).enqueue())
+
+
 @pytest.mark.parametrize("nx", [2001, 17001])
 def test_complex_start_state(nx):
     x, psi = geometry(nx - 1).ground_state()
@@ -81,6 +98,18 @@ def test_partial_runs_equal_the_whole(nx, every):
     adjoint.run_states(geo, F, n, start * every, 0, save, None, 1, part, init_slot=start - 1)
     k = start * every + 1
     agree(part[:, :, k:], whole[:, :, k:])
+
+
+# the same with 16, 24 and 32 points a lane and one window, where a run goes on between saves
+@pytest.mark.parametrize("nx,every", [(4001, 9), (9001, 8), (13001, 7)])
+def test_saves_leave_the_run_alone(nx, every):
+    geo, dev = geometry(nx - 1), fields()
+    n = dev.shape[1] - 1
+    F = adjoint.gate(dev)[0].contiguous()
+    save = torch.zeros((2, n // every, adjoint.state_length(geo), 2), dtype=torch.float64, device="cuda")
+    out = torch.zeros((2, 5, n), dtype=torch.float64, device="cuda")
+    adjoint.run_states(geo, F, n, 0, 0, None, save, every, out)
+    assert torch.equal(out[:, :4], tdse.propagate_batch(geo, dev)[:, :4])
 
 
 def test_given_shape_is_kept_and_the_library_choice_returns():
