@@ -258,14 +258,25 @@ __device__ inline void load_b(const TdseResident &R, Lane<C> &L, double2 *lb, do
 {
     using LN = Lane<C>;
     double2 q = make_double2(1.0, 0.0);
+    // rows in flight: one at a time, a window's factors took longer to arrive than one of its steps (256
+    // instances of 32001 points, two windows, 445 steps: 17.7 ms, with 8 16.2)
+    constexpr int kGroup = 8;
 #pragma unroll
-    for (int i = 0; i < C; i++) {
-        const double2 b = own_b<C>(R, L, i, row(R.b, L.off, i));
-        if (i < Lane<C>::NL)
-            lb[i * 64] = b;
-        else
-            L.br[i < Lane<C>::NL ? 0 : i - Lane<C>::NL] = b;
-        q = cmul(q, make_double2(-b.x, -b.y));
+    for (int i0 = 0; i0 < C; i0 += kGroup) {
+        double2 t[kGroup];
+#pragma unroll
+        for (int m = 0; m < kGroup; m++) t[m] = row(R.b, L.off, i0 + m);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int m = 0; m < kGroup; m++) {
+            const int i = i0 + m;
+            const double2 b = own_b<C>(R, L, i, t[m]);
+            if (i < LN::NL)
+                lb[i * 64] = b;
+            else
+                L.br[i < LN::NL ? 0 : i - LN::NL] = b;
+            q = cmul(q, make_double2(-b.x, -b.y));
+        }
         __builtin_amdgcn_sched_barrier(0);
     }
     if (C > 24)
