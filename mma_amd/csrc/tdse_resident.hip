@@ -24,7 +24,7 @@
 // Where the operands live: psi (r, w and psi in turn) in 4 C registers; b of up to 18 points a lane in LDS (512
 // lanes x 18 x 16 B = 144 KB), of the others in registers, with 32 points from L2 once a step (far_points); g, V' and
 // 1/(1 + i g) come from L2, 32 B a point and step, shared by all instances of a grid.  HBM is idle: the
-// FP64 units bound the step (about 46 + 300 / C of their instructions a point, 60 % of the time; the rest is
+// FP64 units bound the step (about 46 + 300 / C of their instructions a point, 72 % of the time; the rest is
 // waits for LDS and L2 and the two barriers).  No step spills a register: with 22 reloads of spilled values a
 // step of 16001 points took 11.7 us, each reload waiting for the table rows in flight before it as well.
 //
@@ -212,6 +212,14 @@ struct Lane {
     int j0;                          // grid index of its first point (may lie before the grid)
     bool own;                        // its points belong to this window
     const TDSE_GLOBAL tdse_d2 *far;  // b of point NL + i at [64 i], where they are not kept all the time
+};
+
+// The lane's table rows in registers, for a kernel with one wave per SIMD, which has twice the registers
+// and no other wave that computes while it waits: they are the same in every step (one instance of 16001
+// points, 4416 steps: 20.1 -> 18.0 ms).  Empty otherwise.
+template <int C, bool HOLD>
+struct Held {
+    double2 gv[HOLD ? C : 1], s[HOLD ? C : 1], b[HOLD ? C : 1];
 };
 
 // b of point i
@@ -427,17 +435,24 @@ __device__ inline void observe_only(const TdseGeom &G, const Lane<C> &L, const d
 
 // Observables of the state, and the right-hand side r in its place.  CORE: the wave holds part of the atom.
 // What only the wave's edge lanes need later (f of its first and last point) goes to E at once.
-template <int C, bool CORE>
-__device__ inline void first_pass(const TdseResident &R, const StepConst &K, Lane<C> &L, const double2 *gv, Acc &acc,
+template <int C, bool CORE, bool HOLD>
+__device__ inline void first_pass(const TdseResident &R, const StepConst &K, Lane<C> &L, const double2 *gv,
+                                  const Held<C, HOLD> &H, Acc &acc,
                                   TdseWaveEdge &E)
 {
     constexpr int kRows = rows_first(C), kCore = CORE ? rows_core(C) : 1;  // rows in flight
     const double2 *const cq = opaque(R.core);
+    auto g_row = [&](int i) {
+        if constexpr (HOLD)
+            return H.gv[i];
+        else
+            return row(gv, L.off, i);
+    };
     const unsigned coff = CORE ? core_offset<C>(R, L) : 0;
     double2 t[kRows], q[kCore];
-    const double gl = row(gv, L.off, C - 1).x;
+    const double gl = g_row(C - 1).x;
 #pragma unroll
-    for (int i = 0; i < kRows; i++) t[i] = row(gv, L.off, i);
+    for (int i = 0; i < kRows; i++) t[i] = g_row(i);
     if (CORE) {
 #pragma unroll
         for (int i = 0; i < kCore; i++) q[i] = row(cq, coff, i);
@@ -481,25 +496,38 @@ __device__ inline void first_pass(const TdseResident &R, const StepConst &K, Lan
         asm volatile("" : "+v"(s0), "+v"(s1), "+v"(acc.gp), "+v"(L.P[i].x), "+v"(L.P[i].y));
         dm = dp;
         fc = fp;
-        if (i + kRows < C) t[i % kRows] = row(gv, L.off, i + kRows);
+        if (i + kRows < C) t[i % kRows] = g_row(i + kRows);
         __builtin_amdgcn_sched_barrier(0);
     }
     acc.pos = fma(grid_x(L.j0, K.dx, K.xmax), s0, K.dx * s1);
 }
 
-// One time step of the window's points.  rot: exp(-i F dt dx) - 1, from a point's phase to the one before.  ring: this wave's ring entry for the state it starts from.
-template <int C, bool CORE>
+// One time step of the window's points.  rot: exp(-i F dt dx) - 1, from a point's phase to the one before.
+// ring: this wave's ring entry for the state it starts from.
+template <int C, bool CORE, bool HOLD>
 __device__ inline void step(const TdseResident &R, const StepConst &K, Lane<C> &L, const double2 *gv,
-                            const double2 *rs, const double2 *lb, const Shared &sh, int wave, double F, double2 rot, bool deep,
+                            const double2 *rs, const double2 *lb, const Held<C, HOLD> &H, const Shared &sh, int wave, double F, double2 rot, bool deep,
                             bool add, double *ring)
 {
     using LN = Lane<C>;
     constexpr int NL = LN::NL, kRows4 = rows_last(C), kLds1 = lds_ends(C), kLds = lds_between(C);
+    auto b_row = [&](int i) {
+        if constexpr (HOLD)
+            return H.b[i];
+        else
+            return b_at<C>(L, lb, i);
+    };
+    auto s_row = [&](int i) {
+        if constexpr (HOLD)
+            return H.s[i];
+        else
+            return row(rs, L.off, i);
+    };
     double2 e;  // exp(i F dt x) at the lane's last point
     double2 carry;
     Acc acc = {0.0, 0.0, 0.0, 0.0, 0.0};
     TdseWaveEdge &E = sh.edge[wave];
-    first_pass<C, CORE>(R, K, L, gv, acc, E);
+    first_pass<C, CORE, HOLD>(R, K, L, gv, H, acc, E);
     __builtin_amdgcn_sched_barrier(0);
     fetch_far<C>(L);
     __builtin_amdgcn_sched_barrier(0);
@@ -507,14 +535,14 @@ __device__ inline void step(const TdseResident &R, const StepConst &K, Lane<C> &
         // y from zero
         double2 bq[kLds];
 #pragma unroll
-        for (int i = 0; i < kLds && i < NL; i++) bq[i] = lb[i * 64];
+        for (int i = 0; i < kLds && i < NL; i++) bq[i] = b_row(i);
         double2 y = make_double2(0.0, 0.0), b = y;
 #pragma unroll
         for (int i = 0; i < C; i++) {
             y = i > 0 ? cfms(b, y, L.P[i]) : L.P[i];
             asm volatile("" : "+v"(y.x), "+v"(y.y));
-            b = i < NL ? bq[i % kLds] : b_at<C>(L, lb, i);
-            if (i + kLds < NL) bq[i % kLds] = lb[(i + kLds) * 64];
+            b = i < NL ? bq[i % kLds] : b_row(i);
+            if (i + kLds < NL) bq[i % kLds] = b_row(i + kLds);
             if (i % 2 == 0) __builtin_amdgcn_sched_barrier(0);
         }
         // what the chunk hands to the next lane's first row: -b y of its last point
@@ -550,15 +578,15 @@ __device__ inline void step(const TdseResident &R, const StepConst &K, Lane<C> &
     {
         double2 bq[kLds];
 #pragma unroll
-        for (int i = 0; i < kLds && i < NL; i++) bq[i] = lb[i * 64];
+        for (int i = 0; i < kLds && i < NL; i++) bq[i] = b_row(i);
         double2 w = make_double2(-carry.x, -carry.y);
 #pragma unroll
         for (int i = 0; i < C; i++) {
-            const double2 b = i < NL ? bq[i % kLds] : b_at<C>(L, lb, i);
+            const double2 b = i < NL ? bq[i % kLds] : b_row(i);
             w = cmul(b, make_double2(L.P[i].x - w.x, L.P[i].y - w.y));
             asm volatile("" : "+v"(w.x), "+v"(w.y));
             L.P[i] = w;
-            if (i + kLds < NL) bq[i % kLds] = lb[(i + kLds) * 64];
+            if (i + kLds < NL) bq[i % kLds] = b_row(i + kLds);
             if (i % 2 == 0) __builtin_amdgcn_sched_barrier(0);
         }
     }
@@ -568,14 +596,14 @@ __device__ inline void step(const TdseResident &R, const StepConst &K, Lane<C> &
         constexpr int i0 = NL < C - 1 ? NL - 1 : C - 2;  // the first b from LDS
 #pragma unroll
         for (int i = 0; i < kLds; i++)
-            if (i0 - i >= 0) bq[(i0 - i) % kLds] = lb[(i0 - i) * 64];
+            if (i0 - i >= 0) bq[(i0 - i) % kLds] = b_row(i0 - i);
         double2 u = L.P[C - 1];
 #pragma unroll
         for (int i = C - 2; i >= 0; i--) {
-            const double2 b = i < NL ? bq[i % kLds] : b_at<C>(L, lb, i);
+            const double2 b = i < NL ? bq[i % kLds] : b_row(i);
             u = cfms(b, u, L.P[i]);
             asm volatile("" : "+v"(u.x), "+v"(u.y));
-            if (i < NL && i - kLds >= 0) bq[i % kLds] = lb[(i - kLds) * 64];
+            if (i < NL && i - kLds >= 0) bq[i % kLds] = b_row(i - kLds);
             if (i % 2 == 0) __builtin_amdgcn_sched_barrier(0);
         }
         double2 Q = C > 24 ? lb[64 * NL] : L.nQ;
@@ -585,10 +613,10 @@ __device__ inline void step(const TdseResident &R, const StepConst &K, Lane<C> &
         // the rows of the last pass, in flight across the barrier
 #pragma unroll
         for (int i = 0; i < kRows4; i++)
-            if (C - 1 - i >= 0) s[(C - 1 - i) % kRows4] = row(rs, L.off, C - 1 - i);
+            if (C - 1 - i >= 0) s[(C - 1 - i) % kRows4] = s_row(C - 1 - i);
 #pragma unroll
         for (int i = 0; i < kLds1; i++)
-            if (NL - 1 - i >= 0) bq[(NL - 1 - i) % kLds1] = lb[(NL - 1 - i) * 64];
+            if (NL - 1 - i >= 0) bq[(NL - 1 - i) % kLds1] = b_row(NL - 1 - i);
         lds_barrier();
         carry = lane_carry<false>(Q, u, sh.edge[wave + 1].up, lane);
     }
@@ -597,13 +625,13 @@ __device__ inline void step(const TdseResident &R, const StepConst &K, Lane<C> &
         double2 u = carry;
 #pragma unroll
         for (int i = C - 1; i >= 0; i--) {
-            const double2 b = i < NL ? bq[i % kLds1] : b_at<C>(L, lb, i);
+            const double2 b = i < NL ? bq[i % kLds1] : b_row(i);
             u = cfms(b, u, L.P[i]);
             L.P[i] = cmul(e, cmul(s[i % kRows4], u));
             asm volatile("" : "+v"(u.x), "+v"(u.y), "+v"(L.P[i].x), "+v"(L.P[i].y));
             if (i > 0) e = cfma(e, rot, e);  // e + e rot: the rotation's own rounding would change |e| by C steps of it
-            if (i < NL && i - kLds1 >= 0) bq[i % kLds1] = lb[(i - kLds1) * 64];
-            if (i - kRows4 >= 0) s[i % kRows4] = row(rs, L.off, i - kRows4);
+            if (i < NL && i - kLds1 >= 0) bq[i % kLds1] = b_row(i - kLds1);
+            if (i - kRows4 >= 0) s[i % kRows4] = s_row(i - kRows4);
             if (i % 2 == 0) __builtin_amdgcn_sched_barrier(0);
         }
     }
@@ -637,8 +665,9 @@ __device__ inline void write_entries(const Entries &e, const Shared &sh, int t0,
 // on: they come back to a half after more barriers than that takes.  The waves that hold part of the atom
 // run a loop of their own: with both in one, either the registers or the loads in flight of the others pay for
 // what only those need.
-template <int C, bool CORE>
-__device__ inline void run_steps(const TdseResident &R, const StepConst &K, Lane<C> &L, const double2 *lb, const Shared &sh,
+template <int C, bool CORE, bool HOLD>
+__device__ inline void run_steps(const TdseResident &R, const StepConst &K, Lane<C> &L, const double2 *lb,
+                                 const Held<C, HOLD> &H, const Shared &sh,
                                  int wave, const Entries &e, int nb, bool deep, bool add)
 {
     constexpr int kHalf = TDSE_RES_RING / 2;
@@ -649,7 +678,7 @@ __device__ inline void run_steps(const TdseResident &R, const StepConst &K, Lane
         sincos_lean(-0.5 * (fields * K.dt * K.dx), &hs, &hc);
         const double2 rots = make_double2(-2.0 * hs * hs, 2.0 * hs * hc);
         for (int t = t0; t < t1; t++)
-            step<C, CORE>(R, K, L, opaque(R.gv), opaque(R.s), lb, sh, wave, readlane(fields, t - t0), readlane2(rots, t - t0), deep,
+            step<C, CORE, HOLD>(R, K, L, opaque(R.gv), opaque(R.s), lb, H, sh, wave, readlane(fields, t - t0), readlane2(rots, t - t0), deep,
                           add, sh.sums(t % TDSE_RES_RING, wave));
         if (e.flush && t1 - t0 == kHalf && per_lane(wave) == 0) write_entries(e, sh, t0, t1, TDSE_RES_RING - 1);
     }
@@ -756,9 +785,9 @@ __device__ inline void run_instance(const TdseGeom &geom, const TdseInst &inst, 
                     lds_barrier();
                 }
             } else if (per_lane(core)) {
-                run_steps<C, true>(fresh(geom).res, K, L, lb, sh, wave, entries, nb, deep, add);
+                run_steps<C, true, false>(fresh(geom).res, K, L, lb, {}, sh, wave, entries, nb, deep, add);
             } else {
-                run_steps<C, false>(fresh(geom).res, K, L, lb, sh, wave, entries, nb, deep, add);
+                run_steps<C, false, false>(fresh(geom).res, K, L, lb, {}, sh, wave, entries, nb, deep, add);
             }
             at_snap = receivers();
             if (live) {
@@ -899,12 +928,20 @@ __device__ inline void run_window(const TdseGeom &G, const TdseInst &I, const Td
     } else {
         load_tiled<C>(G, L, G.psi0);
     }
+    constexpr bool kHold = C <= 16;  // 24 points' rows do not fit 512 registers
+    Held<C, kHold> H;
+#pragma unroll
+    for (int i = 0; kHold && i < C; i++) {
+        H.gv[i] = row(R.gv, L.off, i);
+        H.s[i] = row(R.s, L.off, i);
+        H.b[i] = b_at<C>(L, lb, i);
+    }
     const Entries entries = {&I, k, 0, -1, R.waves, false};
     __syncthreads();
     if (per_lane(core))
-        run_steps<C, true>(R, K, L, lb, sh, wave, entries, nb, deep, false);
+        run_steps<C, true, kHold>(R, K, L, lb, H, sh, wave, entries, nb, deep, false);
     else
-        run_steps<C, false>(R, K, L, lb, sh, wave, entries, nb, deep, false);
+        run_steps<C, false, kHold>(R, K, L, lb, H, sh, wave, entries, nb, deep, false);
     if (L.own && on_grid) {
         const unsigned o = row_offset<C>(chunk);
 #pragma unroll
