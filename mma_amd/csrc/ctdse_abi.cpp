@@ -457,8 +457,8 @@ int share_lattices(const std::vector<ctdse_geometry *> &gs)
 
 // How the resident kernel covers nx points whose carries reach `reach` points: lanes of C points,
 // waves and windows (TdseResident).  A function of the geometry alone, so an instance's results do
-// not depend on the batch around it.  Costs in instructions per lane and step, from the kernel's
-// listing: 55 per point and 330 for the scans, the phase and the sums.
+// not depend on the batch around it.  Costs in units of an instruction per lane and step: 55 per
+// point and 330 for the scans, the phase and the sums (1210, 1650, 2090; a step of 8 full waves takes 5.6, 7.3 and 9.7 us).
 //   One window: (C, waves) by the work of a CU per instance and step (8 waves fit one, so a CU holds
 //   8 / waves workgroups), and within a quarter of the least by a step's latency: 16 points x 8 waves
 //   rather than 32 x 4 for 8001 points, 18 % more work in half the time per step.
@@ -945,8 +945,8 @@ int resident_shape(const std::vector<const ctdse_geometry *> &geoms, LaunchShape
 }
 
 // The launch of a batch.  Without a launch shape from the caller or the environment: the resident
-// kernel, 2 to 3 x the streaming kernels' rate from 48 instances of 6001 points (24.8 ms against 71.2) to
-// 2048 of 16001 (500 steps: 409 ms against 838).  With one: the streaming kernels in that shape.
+// kernel, 2.3 to 3.5 x the streaming kernels' rate from 48 instances of 16001 points (2213 steps: 20.3 ms
+// against 71.1) to 2048 (4416 steps: 352 ms against 826).  With one: the streaming kernels in that shape.
 int shape_for(const std::vector<const ctdse_geometry *> &geoms, const ctdse_launch_config *cfg, LaunchShape *out)
 {
     int min_nw = 1, max_h = 0;
