@@ -39,6 +39,8 @@
 //
 // Observables (prop.c:293-347) of the state a step starts from are summed in its first pass, per
 // wave in a fixed order, and collected in LDS for up to TDSE_RES_RING steps.
+#include <type_traits>
+
 #include "sincos_reduced.h"
 #include "tdse_internal.h"
 #include "tdse_wave.h"
@@ -102,6 +104,13 @@ __device__ inline int per_lane(int v)
     int l;
     asm volatile("v_mov_b32 %0, %1" : "=v"(l) : "s"(v));
     return l;
+}
+
+// v as a value the compiler knows nothing about: what follows from it is formed where it is used
+__device__ inline int opaque_lane(int v)
+{
+    asm volatile("" : "+v"(v));
+    return v;
 }
 
 // this lane's number, formed anew: kept across a step it would be spilled, and wait for its reload
@@ -260,9 +269,9 @@ __device__ inline double2 own_b(const TdseResident &R, const Lane<C> &L, int i, 
     return j < 0 || j >= R.nx ? make_double2(0.0, 0.0) : b;
 }
 
-// The lane's b into LDS and registers, with what follows from it.
-template <int C>
-__device__ inline void load_b(const TdseResident &R, Lane<C> &L, double2 *lb, double2 *store)
+// The lane's b into LDS and registers, and the product of -b.  OWN: some differ from the table's.
+template <int C, bool OWN>
+__device__ inline double2 load_rows_b(const TdseResident &R, Lane<C> &L, double2 *lb)
 {
     using LN = Lane<C>;
     double2 q = make_double2(1.0, 0.0);
@@ -278,7 +287,7 @@ __device__ inline void load_b(const TdseResident &R, Lane<C> &L, double2 *lb, do
 #pragma unroll
         for (int m = 0; m < kGroup; m++) {
             const int i = i0 + m;
-            const double2 b = own_b<C>(R, L, i, t[m]);
+            const double2 b = OWN ? own_b<C>(R, L, i, t[m]) : t[m];
             if (i < LN::NL)
                 lb[i * 64] = b;
             else
@@ -287,13 +296,23 @@ __device__ inline void load_b(const TdseResident &R, Lane<C> &L, double2 *lb, do
         }
         __builtin_amdgcn_sched_barrier(0);
     }
+    return q;
+}
+
+// The lane's b with what follows from it.  Only the waves at the ends of a grid that reads another one's table
+// have points whose b is not the table's.
+template <int C>
+__device__ inline void load_b(const TdseResident &R, Lane<C> &L, double2 *lb, double2 *store)
+{
+    using LN = Lane<C>;
+    const bool own = R.head > 0 && (L.j0 < R.head || L.j0 + C > R.nx);
+    const double2 q = __any(own) ? load_rows_b<C, true>(R, L, lb) : load_rows_b<C, false>(R, L, lb);
     if (C > 24)
         lb[64 * LN::NL] = q;
     else
         L.nQ = q;
     if constexpr (LN::NF > 0) {
         // from the table, unless the lane's b are its own
-        const bool own = R.head > 0 && (L.j0 < R.head || L.j0 + C > R.nx);
         const double2 *const p = own ? store : R.b + L.off / sizeof(double2) + 64 * LN::NL;
         L.far = (const TDSE_GLOBAL tdse_d2 *)p;
         if (own) {
@@ -319,15 +338,186 @@ __device__ inline void fetch_far(Lane<C> &L)
     }
 }
 
-// The lane's points of a tiled state (zero outside the grid).
+// v[q] of lane t of each four to v[t] of its lane q.
+__device__ inline void transpose_quad(double2 (&v)[4])
+{
+    const int lane = lane_id();
+    const bool odd = lane & 1, high = lane & 2;
+#pragma unroll
+    for (int q = 0; q < 4; q += 2) {
+        const double2 got = dpp2_z<kQuadXor1>(make_double2(odd ? v[q].x : v[q + 1].x, odd ? v[q].y : v[q + 1].y));
+        v[q] = make_double2(odd ? got.x : v[q].x, odd ? got.y : v[q].y);
+        v[q + 1] = make_double2(odd ? v[q + 1].x : got.x, odd ? v[q + 1].y : got.y);
+    }
+#pragma unroll
+    for (int q = 0; q < 2; q++) {
+        const double2 got = dpp2_z<kQuadXor2>(make_double2(high ? v[q].x : v[q + 2].x, high ? v[q].y : v[q + 2].y));
+        v[q] = make_double2(high ? got.x : v[q].x, high ? got.y : v[q].y);
+        v[q + 2] = make_double2(high ? v[q + 2].x : got.x, high ? v[q + 2].y : got.y);
+    }
+}
+
+// A lane's points in a tiled state.  Where the grid starts on one of the lane's chunks of 8 points (always, but for
+// members of a lattice), a row of 8-point chunks costs one instruction: from one offset per chunk, the rows
+// lie at immediate offsets.  A launch of one step executes each path once, so what counts is that all of them
+// stay in the instruction cache that two compute units share (64 KiB, the two loops over the steps take 34 of it).
+// Rows in turn, and within a row the lane's C / 8 chunks, which are neighbours: a line is done with
+// before the next.  With four of them, four lanes take 64 bytes each time, and then exchange them: as 16 bytes
+// apiece a state of 16001 points took 18.7 us to leave a compute unit (4096 instances), so 7.6.
+template <int C>
+struct TiledLane {
+    static constexpr int K = C / TDSE_CHUNK;
+    static constexpr bool kQuads = K == 4;
+    unsigned at[K];        // byte offset of row 4 of each chunk
+    int chunk[K];          // which these are
+    int j0;                // as in Lane
+    bool aligned, inside;  // for the whole wave: as above; all points on the grid
+};
+template <int C>
+__device__ inline TiledLane<C> tiled_lane(const TdseGeom &G, const Lane<C> &L)
+{
+    typedef TiledLane<C> T;
+    T t;
+    t.j0 = opaque_lane(L.j0);
+    t.aligned = __builtin_amdgcn_readfirstlane(t.j0) % TDSE_CHUNK == 0;  // (the same for every lane)
+    t.inside = __all(t.j0 >= 0 && t.j0 + C <= G.nx);
+    const int of4 = lane_id() & 3;
+#pragma unroll
+    for (int q = 0; q < T::K; q++) {
+        t.chunk[q] = (t.j0 >> 3) + (T::kQuads ? 4 * (q - of4) + of4 : q);
+        // (chunks past the grid: the first of those, which exists)
+        t.at[q] = (unsigned)tdse_chunk_base(min(t.chunk[q], G.nchunks)) * (unsigned)sizeof(double2) + 4 * 1024;
+    }
+    return t;
+}
+template <typename T>
+__device__ inline T *tiled_row(T *base, unsigned at, int r)
+{
+    typedef typename std::conditional<std::is_const<T>::value, const TDSE_GLOBAL char, TDSE_GLOBAL char>::type byte;
+    return (T *)((byte *)base + at + (r - 4) * 1024);
+}
+
+// The lane's points of a tiled state (zero outside the grid), all in flight together.
 template <int C>
 __device__ inline void load_tiled(const TdseGeom &G, Lane<C> &L, const double2 *src)
 {
+    typedef TiledLane<C> T;
+    const T t = tiled_lane<C>(G, L);
+    if (t.aligned) {
+#pragma unroll
+        for (int r = 0; r < TDSE_CHUNK; r++)
+#pragma unroll
+            for (int q = 0; q < T::K; q++) L.P[TDSE_CHUNK * q + r] = ld2(tiled_row(src, t.at[q], r), 0);
+        if constexpr (T::kQuads) {
+#pragma unroll
+            for (int r = 0; r < TDSE_CHUNK; r++) {
+                double2 v[4];
+#pragma unroll
+                for (int q = 0; q < 4; q++) v[q] = L.P[TDSE_CHUNK * q + r];
+                transpose_quad(v);
+#pragma unroll
+                for (int q = 0; q < 4; q++) L.P[TDSE_CHUNK * q + r] = v[q];
+            }
+        }
+    } else {
+        const int last = G.nx - 1;
+#pragma unroll
+        for (int i = 0; i < C; i++) {
+            L.P[i] = ld2(src, tdse_index((unsigned)min(max(t.j0 + i, 0), last)));
+            if (i % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+    if (t.inside) return;
 #pragma unroll
     for (int i = 0; i < C; i++) {
-        const int j = L.j0 + i;
-        L.P[i] = j >= 0 && j < G.nx ? ld2(src, tdse_index(j)) : make_double2(0.0, 0.0);
-        __builtin_amdgcn_sched_barrier(0);
+        const bool on = (unsigned)(t.j0 + i) < (unsigned)G.nx;
+        L.P[i] = make_double2(on ? L.P[i].x : 0.0, on ? L.P[i].y : 0.0);
+    }
+}
+
+// The points of the lanes with `own` into a tiled state (those on the grid).
+template <int C>
+__device__ inline void store_tiled(const TdseGeom &G, const Lane<C> &L, double2 *dst, bool own)
+{
+    typedef TiledLane<C> T;
+    T t = tiled_lane<C>(G, L);
+    const unsigned long long owners = __ballot(own);
+    t.inside = t.inside && owners == ~0ull;
+    bool mine[T::K];  // whether the lane's entries of chunk[q] are its own, or those of lane q of its four
+#pragma unroll
+    for (int q = 0; q < T::K; q++) mine[q] = T::kQuads ? owners >> ((lane_id() & ~3) + q) & 1 : own;
+    if (t.aligned) {
+#pragma unroll
+        for (int r = 0; r < TDSE_CHUNK; r++) {
+            double2 v[T::K];
+#pragma unroll
+            for (int q = 0; q < T::K; q++) v[q] = L.P[TDSE_CHUNK * q + r];
+            if constexpr (T::kQuads) transpose_quad(v);
+#pragma unroll
+            for (int q = 0; q < T::K; q++)
+                if (t.inside || (mine[q] && (unsigned)(TDSE_CHUNK * t.chunk[q] + r) < (unsigned)G.nx))
+                    st2(tiled_row(dst, t.at[q], r), 0, v[q]);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < C; i++) {
+            const int j = t.j0 + i;
+            if (own && (unsigned)j < (unsigned)G.nx) st2(dst, tdse_index((unsigned)j), L.P[i]);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+}
+
+// Where point j of the grid lies in the windows' buffer.
+template <int C>
+__device__ inline long long window_index(const TdseResident &R, int j)
+{
+    const int q = j + R.lead, c = q / C;
+    return (long long)(c >> 6) * (C * 64) + (q % C) * 64 + (c & 63);
+}
+
+// A state from the windows' buffer into a tiled one, by the workgroup: neighbouring threads write neighbouring
+// entries, each several of them, all in flight (in the grid's order, one entry of 8 bytes twice at a time, a state of
+// 32001 points took 50 us).
+template <int C>
+__device__ inline void copy_tiled(const TdseGeom &G, const double2 *src, double2 *dst)
+{
+    constexpr int kGroup = 8;
+    const int n = (G.nchunks + 63) / 64 * TDSE_TILE;
+    for (int e0 = threadIdx.x; e0 < n; e0 += kGroup * blockDim.x) {
+        double2 v[kGroup];
+#pragma unroll
+        for (int m = 0; m < kGroup; m++) {
+            const int e = e0 + m * blockDim.x, j = ((e >> 9) * 64 + (e & 63)) * TDSE_CHUNK + (e >> 6) % TDSE_CHUNK;
+            v[m] = ld2(src, window_index<C>(G.res, min(j, G.nx - 1)));
+        }
+#pragma unroll
+        for (int m = 0; m < kGroup; m++) {
+            const int e = e0 + m * blockDim.x, j = ((e >> 9) * 64 + (e & 63)) * TDSE_CHUNK + (e >> 6) % TDSE_CHUNK;
+            if (j < G.nx) st2(dst, TDSE_TILE + e, v[m]);
+        }
+    }
+}
+
+// Likewise those of each window's points that it left out of a tiled state.
+template <int C>
+__device__ inline void copy_left_out(const TdseGeom &G, const double2 *src, double2 *dst)
+{
+    constexpr int kGroup = 8;
+    const TdseResident &R = G.res;
+    const int each = R.halo * C, n = (R.windows - 1) * each;
+    for (int e0 = threadIdx.x; e0 < n; e0 += kGroup * blockDim.x) {
+        double2 v[kGroup];
+        int j[kGroup];
+#pragma unroll
+        for (int m = 0; m < kGroup; m++) {
+            const int e = min(e0 + m * (int)blockDim.x, n - 1), w = 1 + e / each, i = e % each;
+            j[m] = min((w * R.stride + i % R.halo) * C - R.lead + i / R.halo, G.nx - 1);
+            v[m] = ld2(src, window_index<C>(R, j[m]));
+        }
+#pragma unroll
+        for (int m = 0; m < kGroup; m++) st2(dst, tdse_index((unsigned)j[m]), v[m]);
     }
 }
 
@@ -404,29 +594,47 @@ __device__ inline void put_observables(Acc &acc, bool own, int core, bool add, i
     }
 }
 
-// The observables of P alone (the last state of a partial run).
+// The observables of P alone (the last state of a partial run), its rows eight at a time.
 template <int C>
 __device__ inline void observe_only(const TdseGeom &G, const Lane<C> &L, const double2 *gv, int core, bool add,
                                     int lane, double *dst)
 {
+    constexpr int kGroup = 8;
     double s0 = 0.0, s1 = 0.0;
     const TdseResident &R = G.res;
     Acc acc = {0.0, 0.0, 0.0, 0.0, 0.0};
     const unsigned off = core_offset<C>(R, L);
 #pragma unroll
-    for (int i = 0; i < C; i++) {
-        const double2 p = L.P[i];
-        const double n2 = fma(p.x, p.x, p.y * p.y);
-        s0 += n2;
-        s1 = fma((double)i, n2, s1);
-        acc.gp = fma(n2, row(gv, L.off, i).y, acc.gp);
-        if (core) {
-            const double2 w = row(R.core, off, i);
-            acc.pr = fma(p.x, w.x, acc.pr);
-            acc.pi = fma(-p.y, w.x, acc.pi);
-            acc.pint = fma(n2, w.y, acc.pint);
-        }
+    for (int i0 = 0; i0 < C; i0 += kGroup) {
+        double2 t[kGroup];
+#pragma unroll
+        for (int m = 0; m < kGroup; m++) t[m] = row(gv, L.off, i0 + m);
         __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int m = 0; m < kGroup; m++) {
+            const double2 p = L.P[i0 + m];
+            const double n2 = fma(p.x, p.x, p.y * p.y);
+            s0 += n2;
+            s1 = fma((double)(i0 + m), n2, s1);
+            acc.gp = fma(n2, t[m].y, acc.gp);
+        }
+        // formed here: put off to the end, the sums would keep every row (in scratch memory)
+        asm volatile("" : "+v"(s0), "+v"(s1), "+v"(acc.gp));
+        __builtin_amdgcn_sched_barrier(0);
+        if (core) {
+#pragma unroll
+            for (int m = 0; m < kGroup; m++) t[m] = row(R.core, off, i0 + m);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int m = 0; m < kGroup; m++) {
+                const double2 p = L.P[i0 + m];
+                acc.pr = fma(p.x, t[m].x, acc.pr);
+                acc.pi = fma(-p.y, t[m].x, acc.pi);
+                acc.pint = fma(fma(p.x, p.x, p.y * p.y), t[m].y, acc.pint);
+            }
+            asm volatile("" : "+v"(acc.pr), "+v"(acc.pi), "+v"(acc.pint));
+            __builtin_amdgcn_sched_barrier(0);
+        }
     }
     if (core && R.core_im) core_im<C>(R, L, off, acc);
     acc.pos = fma(grid_x(L.j0, G.dx, G.xmax), s0, G.dx * s1);
@@ -684,8 +892,10 @@ __device__ inline void run_steps(const TdseResident &R, const StepConst &K, Lane
     }
 }
 
-// The whole run of one instance by the waves of a workgroup.
-template <int C>
+// The whole run of one instance by the waves of a workgroup.  WINDOWS: over several windows, whose states are loaded
+// and stored for every block of steps; else the state stays in registers.  With both in one loop the state was a value that may
+// come from either, and went through scratch memory (more than its own 256 KB, each way) in every block.
+template <int C, bool WINDOWS>
 __device__ inline void run_instance(const TdseGeom &geom, const TdseInst &inst, double2 *work, long long work_stride, double2 *far,
                                     const Shared &sh, Queue &queue)
 {
@@ -694,7 +904,6 @@ __device__ inline void run_instance(const TdseGeom &geom, const TdseInst &inst, 
     const int nw = geom.res.waves;
     const bool live = per_lane(wave) < nw;
     const bool deep = geom.res.reach > 8 * C;
-    const bool windows = geom.res.windows > 1;
     const int k_start = inst.k0, k_stop = inst.n_run > 0 ? inst.k0 + inst.n_run : inst.n_steps;
     int i_snap = 0;
     int cur = 0;  // multi-window states: the buffer that holds the current state
@@ -728,20 +937,53 @@ __device__ inline void run_instance(const TdseGeom &geom, const TdseInst &inst, 
     }
     const int gate = __builtin_amdgcn_readfirstlane(queue.gate);
     double2 *const lb = sh.b + wave * (64 * tdse_res_lds_rows(C)) + lane;  // this lane's b: point i at lb[i * 64]
-    LN L;
     const StepConst K = step_const(fresh(geom));
-    int core = 0;
-    int chunk = 0;
     // prop.c:248-255: snapshot row i_snap gets psi after step m when m % every == 0; the next such step
     auto snap_step = [&](const TdseInst &I, int k) {
         return I.snap && i_snap < I.n_snap - 1 ? (k + I.snap_every - 1) / I.snap_every * I.snap_every : 0x7ffffffe;
     };
 
+    // the lane's chunk of window w, its b and its points: of the start state (src null) or of the windows' buffer
+    auto load_window = [&](LN &L, int &chunk, int &core, int w, const double2 *src) {
+        const TdseGeom &G = fresh(geom);
+        place_lane<C>(G.res, w, wave, lane, L, chunk, core);
+        load_b<C>(G.res, L, lb, far + wave * tdse_res_far(1, C) + lane);
+        if (!src) {
+            const TdseInst &I = fresh(inst);
+            load_tiled<C>(G, L, I.psi_init ? I.psi_init : G.psi0);
+        } else {
+            const unsigned o = row_offset<C>(chunk);  // (a window's chunks lie in its buffer as in the grid)
+#pragma unroll
+            for (int i = 0; i < C; i++) L.P[i] = row(src, o, i);
+        }
+    };
+    // nb steps from k of a window's points, and the observables of the last state of a partial run
+    auto run_window = [&](LN &L, int core, bool add, int k, int nb) {
+        const Entries entries = {&inst, k, k_start, gate, nw, !WINDOWS};
+        if (per_lane(core))
+            run_steps<C, true, false>(fresh(geom).res, K, L, lb, {}, sh, wave, entries, nb, deep, add);
+        else
+            run_steps<C, false, false>(fresh(geom).res, K, L, lb, {}, sh, wave, entries, nb, deep, add);
+        const TdseGeom &G = fresh(geom);
+        const TdseInst &I = fresh(inst);
+        if (I.src && k_stop < I.n_steps && k + nb == k_stop)
+            observe_only<C>(G, L, G.res.gv, core, add, lane, sh.sums(WINDOWS ? nb : nb % TDSE_RES_RING, wave));
+    };
+    auto other_waves_steps = [&](int nb) {
+        for (int t = 0; t < nb; t++) {
+            lds_barrier();
+            lds_barrier();
+        }
+    };
+    LN one;
+    int one_chunk = 0, one_core = 0;
+    if (!WINDOWS && live) load_window(one, one_chunk, one_core, 0, nullptr);
+
     for (int k = k_start; k < k_stop;) {
         int nb;
         {
             const TdseInst &I = fresh(inst);
-            nb = windows ? min(fresh(geom).res.steps, k_stop - k) : k_stop - k;
+            nb = WINDOWS ? min(fresh(geom).res.steps, k_stop - k) : k_stop - k;
             if (I.save) nb = min(nb, I.save_every - (k - k_start) % I.save_every);
             nb = min(nb, snap_step(I, k) + 1 - k);
         }
@@ -762,81 +1004,72 @@ __device__ inline void run_instance(const TdseGeom &geom, const TdseInst &inst, 
             return at_snap;
         };
         bool at_snap = false;
-        for (int w = 0; w == 0 || w < fresh(geom).res.windows; w++) {
-            const bool add = w > 0;
-            if (live && (windows || k == k_start)) {
-                const TdseGeom &G = fresh(geom);
-                const TdseInst &I = fresh(inst);
-                place_lane<C>(G.res, w, wave, lane, L, chunk, core);
-                load_b<C>(G.res, L, lb, far + wave * tdse_res_far(1, C) + lane);
-                if (k == k_start) {
-                    load_tiled<C>(G, L, I.psi_init ? I.psi_init : G.psi0);
-                } else {
-                    const double2 *src = work + cur * work_stride;
-                    const unsigned o = row_offset<C>(chunk);  // (a window's chunks lie in its buffer as in the grid)
-#pragma unroll
-                    for (int i = 0; i < C; i++) L.P[i] = row(src, o, i);
+        if constexpr (WINDOWS) {
+            // A run's last block goes to its save at once, and not through the windows' buffer.  The save may be the
+            // state the run starts from: in its only block a window leaves out what the next has yet to load, the `halo`
+            // chunks past the next one's first.
+            receivers();
+            double2 *const direct = k + nb == k_stop && !to[1] && !to[2] && !to[3] ? reinterpret_cast<double2 *>(to[0]) : nullptr;
+            for (int w = 0; w < fresh(geom).res.windows; w++) {
+                if (!live) {
+                    other_waves_steps(nb);
+                    continue;
                 }
-            }
-            const Entries entries = {&inst, k, k_start, gate, nw, !windows};
-            if (!live) {
-                for (int t = 0; t < nb; t++) {
-                    lds_barrier();
-                    lds_barrier();
-                }
-            } else if (per_lane(core)) {
-                run_steps<C, true, false>(fresh(geom).res, K, L, lb, {}, sh, wave, entries, nb, deep, add);
-            } else {
-                run_steps<C, false, false>(fresh(geom).res, K, L, lb, {}, sh, wave, entries, nb, deep, add);
-            }
-            at_snap = receivers();
-            if (live) {
+                LN L;
+                int chunk, core;
+                load_window(L, chunk, core, w, k == k_start ? nullptr : work + cur * work_stride);
+                run_window(L, core, w > 0, k, nb);
                 const TdseGeom &G = fresh(geom);
-                const TdseInst &I = fresh(inst);
-                if (I.src && k_stop < I.n_steps && k + nb == k_stop)
-                    observe_only<C>(G, L, G.res.gv, core, add, lane,
-                                    sh.sums(windows ? nb : nb % TDSE_RES_RING, wave));
-                if (windows) {
+                const bool later = k == k_start && w < G.res.windows - 1 && chunk >= (w + 1) * G.res.stride;
+                if (direct) store_tiled<C>(G, L, direct, L.own && !later);
+                if (L.own && (later || !direct)) {
                     double2 *dst = work + (cur ^ 1) * work_stride;
                     const unsigned o = row_offset<C>(chunk);
-                    if (L.own) {
 #pragma unroll
-                        for (int i = 0; i < C; i++) st2((double2 *)((char *)dst + o), 64 * i, L.P[i]);
-                    }
-                } else if (to[0] || to[1] || to[2] || to[3]) {
-                    for (int m = 0; m < 4; m++) {
-                        double *dst = to[m];
-                        if (!dst) continue;
-#pragma unroll
-                        for (int i = 0; i < C; i++) {
-                            const int j = L.j0 + i;
-                            if (j >= 0 && j < G.nx) put_state(dst, m > 0 ? j : tdse_index(j), L.P[i]);
-                            __builtin_amdgcn_sched_barrier(0);
-                        }
-                    }
+                    for (int i = 0; i < C; i++) st2((double2 *)((char *)dst + o), 64 * i, L.P[i]);
                 }
             }
-        }
-        __syncthreads();  // the ring is complete, a window buffer is in memory
-        if (windows) {
+            __syncthreads();  // the ring is complete, the windows' buffer is in memory
             const TdseGeom &G = fresh(geom);
             cur ^= 1;
             const double2 *src = work + cur * work_stride;
-            for (int m = 0; m < 4; m++) {
+            if (direct && k == k_start) copy_left_out<C>(G, src, direct);
+            if (!direct) at_snap = receivers();
+            if (!direct && to[0]) copy_tiled<C>(G, src, reinterpret_cast<double2 *>(to[0]));
+            for (int m = 1; m < 4 && !direct; m++) {
                 double *dst = to[m];
                 if (!dst) continue;
-                for (int j = threadIdx.x; j < G.nx; j += blockDim.x) {
-                    const int q = j + G.res.lead, c = q / C;
-                    put_state(dst, m > 0 ? j : tdse_index(j), src[(long long)(c >> 6) * (C * 64) + (q % C) * 64 + (c & 63)]);
+                for (int j = threadIdx.x; j < G.nx; j += blockDim.x) put_state(dst, j, src[window_index<C>(G.res, j)]);
+            }
+        } else {
+            if (live)
+                run_window(one, one_core, false, k, nb);
+            else
+                other_waves_steps(nb);
+            at_snap = receivers();
+            if (live) {
+                const TdseGeom &G = fresh(geom);
+                if (to[0]) store_tiled<C>(G, one, reinterpret_cast<double2 *>(to[0]), true);
+                for (int m = 1; m < 4; m++) {
+                    double *dst = to[m];
+                    if (!dst) continue;
+                    const int j0 = opaque_lane(one.j0);
+#pragma unroll
+                    for (int i = 0; i < C; i++) {
+                        const int j = j0 + i;
+                        if (j >= 0 && j < G.nx) put_state(dst, j, one.P[i]);
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
                 }
             }
+            __syncthreads();  // the ring is complete
         }
         // what is left in the ring, and the last state of a partial run
         if (wave == 0) {
             const Entries entries = {&inst, k, k_start, gate, nw, false};
-            const int from = windows ? 0 : nb / (TDSE_RES_RING / 2) * (TDSE_RES_RING / 2);
+            const int from = WINDOWS ? 0 : nb / (TDSE_RES_RING / 2) * (TDSE_RES_RING / 2);
             const bool last = k + nb == k_stop && k_stop < fresh(inst).n_steps;
-            write_entries(entries, sh, from, nb + last, windows ? 31 : TDSE_RES_RING - 1);
+            write_entries(entries, sh, from, nb + last, WINDOWS ? 31 : TDSE_RES_RING - 1);
         }
         __syncthreads();  // the ring has been read
         i_snap += at_snap;
@@ -867,10 +1100,18 @@ tdse_resident_kernel(const TdseGeom *__restrict__ geoms, const TdseInst *__restr
         // two states of the windows, and the lanes' own b that registers do not hold
         double2 *const buf = work + (long long)blockIdx.x * work_stride;
         const long long states = (work_stride - tdse_res_far(TDSE_MAX_WAVES, 32)) / 2;
-        switch (G.res.chunk) {
-        case 16: run_instance<16>(G, I, buf, states, buf + 2 * states, sh, queue); break;
-        case 24: run_instance<24>(G, I, buf, states, buf + 2 * states, sh, queue); break;
-        case 32: run_instance<32>(G, I, buf, states, buf + 2 * states, sh, queue); break;
+        auto run = [&](auto c, auto windows) {
+            run_instance<decltype(c)::value, decltype(windows)::value>(G, I, buf, states, buf + 2 * states, sh, queue);
+        };
+        const std::true_type several{};
+        const std::false_type one{};
+        switch (G.res.chunk * 2 + (G.res.windows > 1)) {
+        case 32: run(std::integral_constant<int, 16>{}, one); break;
+        case 33: run(std::integral_constant<int, 16>{}, several); break;
+        case 48: run(std::integral_constant<int, 24>{}, one); break;
+        case 49: run(std::integral_constant<int, 24>{}, several); break;
+        case 64: run(std::integral_constant<int, 32>{}, one); break;
+        case 65: run(std::integral_constant<int, 32>{}, several); break;
         default: break;
         }
     }

@@ -65,6 +65,7 @@ __device__ inline double2 cmul(double2 a, double2 b)
 
 // ---- cross-lane moves in the VALU (DPP), 64-bit values as two 32-bit halves ----
 // Lanes without a source keep `old` (bound_ctrl off), so scans pad with the identity map.
+constexpr int kQuadXor1 = 0xb1, kQuadXor2 = 0x4e;  // the lane's neighbour, and the one after that, in each four
 constexpr int kRowShr = 0x110, kRowShl = 0x100, kWaveShr1 = 0x138, kWaveShl1 = 0x130;
 // lane 15 of each row to the next row, lane 31 to rows 2 and 3 (with the row masks below)
 constexpr int kRowBcast15 = 0x142, kRowBcast31 = 0x143;
