@@ -1113,7 +1113,7 @@ int grid_slots(int n, const LaunchShape &sh, int *slots)
 // Enqueues the queue reset and the persistent kernel (no allocation, copy or wait).
 int enqueue_plan(const ctdse_batch_plan &P, double2 *work, hipStream_t stream)
 {
-    hipLaunchKernelGGL(tdse_fill_int_kernel, dim3(1), dim3(64), 0, stream, P.d_counter.as<int>(), TDSE_QUEUES, 0);
+    hipLaunchKernelGGL(tdse_fill_int_kernel, dim3(1), dim3(TDSE_COUNTERS), 0, stream, P.d_counter.as<int>(), TDSE_COUNTERS, 0);
     if (P.shape.resident) {
         hipLaunchKernelGGL(tdse_resident_kernel, dim3(P.slots), dim3(64 * P.shape.nw), P.shape.lds, stream,
                            P.d_geom.as<TdseGeom>(), P.d_inst.as<TdseInst>(), P.d_order.as<int>(), P.queues,
@@ -1161,7 +1161,7 @@ int propagate(const std::vector<InstSpec> &spec, hipStream_t stream, const ctdse
     HIP_CHECK(P.d_geom.alloc(B.gdev.size() * sizeof(TdseGeom)));
     HIP_CHECK(P.d_inst.alloc(B.insts.size() * sizeof(TdseInst)));
     HIP_CHECK(P.d_order.alloc(B.order.size() * sizeof(int)));
-    HIP_CHECK(P.d_counter.alloc(TDSE_QUEUES * sizeof(int)));
+    HIP_CHECK(P.d_counter.alloc(TDSE_COUNTERS * sizeof(int)));
     HIP_CHECK(hipMemcpyAsync(P.d_geom.p, B.gdev.data(), B.gdev.size() * sizeof(TdseGeom), hipMemcpyHostToDevice, stream));
     HIP_CHECK(hipMemcpyAsync(P.d_inst.p, B.insts.data(), B.insts.size() * sizeof(TdseInst), hipMemcpyHostToDevice, stream));
     HIP_CHECK(hipMemcpyAsync(P.d_order.p, B.order.data(), B.order.size() * sizeof(int), hipMemcpyHostToDevice, stream));
@@ -1309,7 +1309,7 @@ int make_plan(const std::vector<InstSpec> &spec, const ctdse_launch_config *cfg,
     HIP_CHECK(P.d_geom.alloc(B.gdev.size() * sizeof(TdseGeom)));
     HIP_CHECK(P.d_inst.alloc(B.insts.size() * sizeof(TdseInst)));
     HIP_CHECK(P.d_order.alloc(B.order.size() * sizeof(int)));
-    HIP_CHECK(P.d_counter.alloc(TDSE_QUEUES * sizeof(int)));
+    HIP_CHECK(P.d_counter.alloc(TDSE_COUNTERS * sizeof(int)));
     HIP_CHECK(hipMemcpy(P.d_geom.p, B.gdev.data(), B.gdev.size() * sizeof(TdseGeom), hipMemcpyHostToDevice));
     HIP_CHECK(hipMemcpy(P.d_inst.p, B.insts.data(), B.insts.size() * sizeof(TdseInst), hipMemcpyHostToDevice));
     HIP_CHECK(hipMemcpy(P.d_order.p, B.order.data(), B.order.size() * sizeof(int), hipMemcpyHostToDevice));

@@ -36,6 +36,8 @@
 // on first, then from the others in turn, so each XCD's L2 mostly serves the tables of its own
 // queue's instances.
 #define TDSE_QUEUES 8
+#define TDSE_QUEUE_STRIDE 32  // ints from one queue's counter to the next: a cache line of its own each
+#define TDSE_COUNTERS (TDSE_QUEUES * TDSE_QUEUE_STRIDE)
 struct TdseQueues {
     int off[TDSE_QUEUES + 1];
 };
@@ -234,7 +236,7 @@ __global__ void tdse_tables_ib_kernel(TableJob *jobs);
 // host forms of the serial setup steps (tdse_setup.hip), bit-identical to the kernels
 void tdse_ground_state_host(GsJob &J);
 void tdse_tables_pivot_host(TableJob &J);
-// counter: TDSE_QUEUES ints, zero at launch
+// counter: TDSE_COUNTERS ints, zero at launch
 __global__ void tdse_propagate_kernel(const TdseGeom *geoms, const TdseInst *insts, const int *order,
                                       TdseQueues queues, int *counter, double2 *work, long long work_stride);
 __global__ void tdse_propagate_pair_kernel(const TdseGeom *geoms, const TdseInst *insts, const int *order,

@@ -260,7 +260,9 @@ __device__ inline int xcd_id()
 // Next instance of the launch for this workgroup (thread 0 only): from the queue of this XCD
 // first, then the others in turn; tried (LDS) counts the queues found drained so far.  -1 when
 // every queue is drained: a queue is left only after its counter passed its length, so once
-// every workgroup has left every queue, each instance was taken exactly once.
+// every workgroup has left every queue, each instance was taken exactly once.  A workgroup looks before it
+// adds: additions to one line follow each other, 12 ns apart (4096 instances of 201 points, one step, 2048 workgroups
+// that each left eight queues whose counters shared a line: 255 us, now 62).
 __device__ inline int next_instance(const TdseQueues &qs, int *counter, int &tried)
 {
     const int q0 = xcd_id() % TDSE_QUEUES;
@@ -268,7 +270,9 @@ __device__ inline int next_instance(const TdseQueues &qs, int *counter, int &tri
         const int q = (q0 + tried) % TDSE_QUEUES;
         const int len = qs.off[q + 1] - qs.off[q];
         if (len == 0) continue;
-        const int t = atomicAdd(counter + q, 1);
+        int *const c = counter + q * TDSE_QUEUE_STRIDE;
+        if (__hip_atomic_load(c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= len) continue;
+        const int t = atomicAdd(c, 1);
         if (t < len) return qs.off[q] + t;
     }
     return -1;
