@@ -605,9 +605,11 @@ int attach_tables(ctdse_geometry *G, const ctdse_geometry *src, TdseResident &R,
 // allocation and one launch: two of each per geometry took 0.2 ms a geometry).
 int add_resident(const std::vector<ctdse_geometry *> &gs)
 {
-    // here and not at a launch, which may be captured
+    // here and not at a launch, which may be captured; the most any asks for
     HIP_CHECK(hipFuncSetAttribute((const void *)tdse_window_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
                                   tdse_res_lds(TDSE_ONE_WAVES, 24)));
+    HIP_CHECK(hipFuncSetAttribute((const void *)tdse_resident_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                  tdse_res_lds(TDSE_MAX_WAVES, 32)));
     std::map<const Lattice *, ctdse_geometry *> widest;
     for (ctdse_geometry *G : gs)
         if (G && G->lattice) {
@@ -938,9 +940,6 @@ int resident_shape(const std::vector<const ctdse_geometry *> &geoms, LaunchShape
     HIP_CHECK(hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerMultiprocessor, dev));
     const int fit = (int)((size_t)lds / (attr.sharedSizeBytes + sh.lds));
     sh.per_cu = std::max(1, std::min(4 * TDSE_RES_WAVES_PER_SIMD / sh.nw, fit));
-    // the most any batch asks for, so that plans of different sizes live side by side
-    HIP_CHECK(hipFuncSetAttribute((const void *)tdse_resident_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                  tdse_res_lds(TDSE_MAX_WAVES, 32)));
     return CTDSE_OK;
 }
 
@@ -994,7 +993,10 @@ struct ctdse_batch_plan {
     int n = 0, slots = 0;
     LaunchShape shape;
     long long stride = 0;
-    DevMem work, d_geom, d_inst, d_order, d_counter;
+    DevMem work, desc;  // desc: geoms, insts, order and counters, one allocation and one copy (upload)
+    TdseGeom *geoms = nullptr;
+    TdseInst *insts = nullptr;
+    int *order = nullptr, *counters = nullptr;
     TdseQueues queues{};
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
@@ -1072,10 +1074,11 @@ int describe(const std::vector<InstSpec> &spec, BatchHost &B)
     // largest instances first (longest-processing-time order for the atomic queues)
     std::vector<int> lpt(n);
     for (int i = 0; i < n; i++) lpt[i] = i;
-    auto steps_of = [&](int p) { return (double)(spec[p].n_run > 0 ? spec[p].n_run : spec[p].n_steps - spec[p].k0); };
-    std::stable_sort(lpt.begin(), lpt.end(), [&](int p, int q) {
-        return (double)spec[p].geom->dev.nx * steps_of(p) > (double)spec[q].geom->dev.nx * steps_of(q);
-    });
+    std::vector<double> cost(n);
+    for (int p = 0; p < n; p++)
+        cost[p] = (double)spec[p].geom->dev.nx * (spec[p].n_run > 0 ? spec[p].n_run : spec[p].n_steps - spec[p].k0);
+    auto longer = [&](int p, int q) { return cost[p] > cost[q]; };
+    if (!std::is_sorted(lpt.begin(), lpt.end(), longer)) std::stable_sort(lpt.begin(), lpt.end(), longer);
     // one queue per XCD: an instance whose geometry reads shared lattice tables goes to the
     // queue of its alignment (the 8 alignments of a lattice are 8 sets of lines; an XCD's 4 MB
     // L2 then holds one of them), the others are dealt round-robin
@@ -1113,11 +1116,11 @@ int grid_slots(int n, const LaunchShape &sh, int *slots)
 // Enqueues the queue reset and the persistent kernel (no allocation, copy or wait).
 int enqueue_plan(const ctdse_batch_plan &P, double2 *work, hipStream_t stream)
 {
-    hipLaunchKernelGGL(tdse_fill_int_kernel, dim3(1), dim3(TDSE_COUNTERS), 0, stream, P.d_counter.as<int>(), TDSE_COUNTERS, 0);
+    hipLaunchKernelGGL(tdse_fill_int_kernel, dim3(1), dim3(TDSE_COUNTERS), 0, stream, P.counters, TDSE_COUNTERS, 0);
     if (P.shape.resident) {
         hipLaunchKernelGGL(tdse_resident_kernel, dim3(P.slots), dim3(64 * P.shape.nw), P.shape.lds, stream,
-                           P.d_geom.as<TdseGeom>(), P.d_inst.as<TdseInst>(), P.d_order.as<int>(), P.queues,
-                           P.d_counter.as<int>(), work, P.stride);
+                           P.geoms, P.insts, P.order, P.queues,
+                           P.counters, work, P.stride);
         HIP_CHECK(hipGetLastError());
         return CTDSE_OK;
     }
@@ -1125,8 +1128,8 @@ int enqueue_plan(const ctdse_batch_plan &P, double2 *work, hipStream_t stream)
     hipLaunchKernelGGL(stash ? tdse_propagate_pair_stash_kernel
                              : (P.shape.steps == 2 ? tdse_propagate_pair_kernel : tdse_propagate_kernel),
                        dim3(P.slots), dim3(64 * P.shape.nw), stash ? stash_bytes(P.shape.nw) : 0, stream,
-                       P.d_geom.as<TdseGeom>(), P.d_inst.as<TdseInst>(), P.d_order.as<int>(), P.queues,
-                       P.d_counter.as<int>(), work, P.stride);
+                       P.geoms, P.insts, P.order, P.queues,
+                       P.counters, work, P.stride);
     HIP_CHECK(hipGetLastError());
     return CTDSE_OK;
 }
@@ -1136,6 +1139,29 @@ int enqueue_plan(const ctdse_batch_plan &P, double2 *work, hipStream_t stream)
 size_t work_bytes(const ctdse_batch_plan &P)
 {
     return (size_t)P.slots * P.stride * sizeof(double2);
+}
+
+// The descriptors of a batch onto the device: one allocation, one copy on `stream` from `staged`, which the caller
+// keeps until that is done.  (An allocation and a copy each, and the sort of a list in order, took 0.29 ms of a
+// call of 4096 instances.)
+int upload(ctdse_batch_plan &P, const BatchHost &B, std::vector<char> &staged, hipStream_t stream)
+{
+    auto whole = [](size_t bytes) { return (bytes + 255) / 256 * 256; };
+    const size_t n_geom = B.gdev.size() * sizeof(TdseGeom), n_inst = B.insts.size() * sizeof(TdseInst);
+    const size_t n_order = B.order.size() * sizeof(int);
+    const size_t o_inst = whole(n_geom), o_order = o_inst + whole(n_inst), o_counters = o_order + whole(n_order);
+    HIP_CHECK(P.desc.alloc(o_counters + TDSE_COUNTERS * sizeof(int)));
+    staged.resize(o_counters);
+    std::copy_n(reinterpret_cast<const char *>(B.gdev.data()), n_geom, staged.data());
+    std::copy_n(reinterpret_cast<const char *>(B.insts.data()), n_inst, staged.data() + o_inst);
+    std::copy_n(reinterpret_cast<const char *>(B.order.data()), n_order, staged.data() + o_order);
+    char *p = P.desc.as<char>();
+    P.geoms = reinterpret_cast<TdseGeom *>(p);
+    P.insts = reinterpret_cast<TdseInst *>(p + o_inst);
+    P.order = reinterpret_cast<int *>(p + o_order);
+    P.counters = reinterpret_cast<int *>(p + o_counters);
+    HIP_CHECK(hipMemcpyAsync(p, staged.data(), staged.size(), hipMemcpyHostToDevice, stream));
+    return CTDSE_OK;
 }
 
 // Immediate path: descriptors copied on `stream`, the shared work buffer, and a wait.
@@ -1158,13 +1184,8 @@ int propagate(const std::vector<InstSpec> &spec, hipStream_t stream, const ctdse
         HIP_CHECK(g_work.alloc(need));
         g_work_bytes = need;
     }
-    HIP_CHECK(P.d_geom.alloc(B.gdev.size() * sizeof(TdseGeom)));
-    HIP_CHECK(P.d_inst.alloc(B.insts.size() * sizeof(TdseInst)));
-    HIP_CHECK(P.d_order.alloc(B.order.size() * sizeof(int)));
-    HIP_CHECK(P.d_counter.alloc(TDSE_COUNTERS * sizeof(int)));
-    HIP_CHECK(hipMemcpyAsync(P.d_geom.p, B.gdev.data(), B.gdev.size() * sizeof(TdseGeom), hipMemcpyHostToDevice, stream));
-    HIP_CHECK(hipMemcpyAsync(P.d_inst.p, B.insts.data(), B.insts.size() * sizeof(TdseInst), hipMemcpyHostToDevice, stream));
-    HIP_CHECK(hipMemcpyAsync(P.d_order.p, B.order.data(), B.order.size() * sizeof(int), hipMemcpyHostToDevice, stream));
+    std::vector<char> staged;  // until the wait below
+    if (upload(P, B, staged, stream) != CTDSE_OK) return g_status;
     const int queued = enqueue_plan(P, g_work.as<double2>(), stream);
     HIP_CHECK(hipStreamSynchronize(stream));  // the descriptors are freed on return
     return queued;
@@ -1197,6 +1218,22 @@ struct StepBufs {
     double *gated;
     double2 *psi[2];
 };
+
+size_t align256(size_t n) { return (n + 255) & ~size_t(255); }
+
+// Bytes of the buffers of a run one after the other, and (with base) where they are.
+size_t step_buffers(const TdseGeom &g, int n_steps, char *base, StepBufs *b)
+{
+    const size_t o_inst = align256(sizeof(TdseGeom)), o_part = o_inst + align256(sizeof(TdseInst));
+    const size_t o_gated = o_part + align256(window_sums(g.one) * sizeof(double));
+    const size_t o_psi = o_gated + align256((size_t)(n_steps + 1) * sizeof(double));
+    const size_t state = (size_t)window_state(g.one, g.nx) * sizeof(double2);
+    if (base)
+        *b = StepBufs{reinterpret_cast<TdseGeom *>(base), reinterpret_cast<TdseInst *>(base + o_inst),
+                      reinterpret_cast<double *>(base + o_part), reinterpret_cast<double *>(base + o_gated),
+                      {reinterpret_cast<double2 *>(base + o_psi), reinterpret_cast<double2 *>(base + o_psi + state)}};
+    return o_psi + 2 * state;
+}
 
 // Queues a window run into the given buffers: no allocation and no wait.  Every buffer is written
 // here before it is read, so buffers left over from an earlier run may be reused.
@@ -1252,15 +1289,10 @@ int enqueue_steps(const InstSpec &s, const StepBufs &b, hipStream_t stream)
 int propagate_steps(const InstSpec &s, hipStream_t stream)
 {
     const TdseGeom &g = s.geom->dev;
-    const long long state = window_state(g.one, g.nx);
-    DevMem states, partial, gated, d_geom, d_inst;
-    HIP_CHECK(states.alloc(2 * (size_t)state * sizeof(double2)));
-    HIP_CHECK(partial.alloc(window_sums(g.one) * sizeof(double)));
-    HIP_CHECK(gated.alloc((size_t)(s.n_steps + 1) * sizeof(double)));
-    HIP_CHECK(d_geom.alloc(sizeof(TdseGeom)));
-    HIP_CHECK(d_inst.alloc(sizeof(TdseInst)));
-    const StepBufs b{d_geom.as<TdseGeom>(), d_inst.as<TdseInst>(), partial.as<double>(), gated.as<double>(),
-                     {states.as<double2>(), states.as<double2>() + state}};
+    DevMem mem;  // (an allocation for each buffer: 38 us for one step of 201 points, so 34)
+    StepBufs b;
+    HIP_CHECK(mem.alloc(step_buffers(g, s.n_steps, nullptr, nullptr)));
+    step_buffers(g, s.n_steps, mem.as<char>(), &b);
     std::lock_guard<std::mutex> lock(g_launch_mutex);
     const int queued = enqueue_steps(s, b, stream);
     // wait before returning (also after a launch error): the buffers freed on return may
@@ -1292,8 +1324,6 @@ int scratch_address(void **out)
     return CTDSE_OK;
 }
 
-size_t align256(size_t n) { return (n + 255) & ~size_t(255); }
-
 // Plan path: everything allocated and uploaded here, once.
 int make_plan(const std::vector<InstSpec> &spec, const ctdse_launch_config *cfg, ctdse_batch_plan &P)
 {
@@ -1306,13 +1336,9 @@ int make_plan(const std::vector<InstSpec> &spec, const ctdse_launch_config *cfg,
     if (grid_slots(std::max(n, 1), P.shape, &P.slots) != CTDSE_OK) return g_status;
     P.stride = P.shape.resident ? B.res_stride : B.stride;
     HIP_CHECK(P.work.alloc(work_bytes(P)));
-    HIP_CHECK(P.d_geom.alloc(B.gdev.size() * sizeof(TdseGeom)));
-    HIP_CHECK(P.d_inst.alloc(B.insts.size() * sizeof(TdseInst)));
-    HIP_CHECK(P.d_order.alloc(B.order.size() * sizeof(int)));
-    HIP_CHECK(P.d_counter.alloc(TDSE_COUNTERS * sizeof(int)));
-    HIP_CHECK(hipMemcpy(P.d_geom.p, B.gdev.data(), B.gdev.size() * sizeof(TdseGeom), hipMemcpyHostToDevice));
-    HIP_CHECK(hipMemcpy(P.d_inst.p, B.insts.data(), B.insts.size() * sizeof(TdseInst), hipMemcpyHostToDevice));
-    HIP_CHECK(hipMemcpy(P.d_order.p, B.order.data(), B.order.size() * sizeof(int), hipMemcpyHostToDevice));
+    std::vector<char> staged;
+    if (upload(P, B, staged, nullptr) != CTDSE_OK) return g_status;
+    HIP_CHECK(hipStreamSynchronize(nullptr));
     HIP_CHECK(hipEventCreateWithFlags(&P.done, hipEventDisableTiming));
     return CTDSE_OK;
 }
@@ -1541,19 +1567,7 @@ int ctdse_propagate_one_noalloc(const ctdse_geometry *geom, int n_steps, const d
     s.field = field;
     s.out = out;
     const TdseGeom &g = geom->dev;
-    const long long state = window_state(g.one, g.nx);
-    // layout of the scratch array: descriptors, partial sums, gated field, two states
-    size_t off = 0;
-    const size_t o_geom = off;
-    off += align256(sizeof(TdseGeom));
-    const size_t o_inst = off;
-    off += align256(sizeof(TdseInst));
-    const size_t o_part = off;
-    off += align256(window_sums(g.one) * sizeof(double));
-    const size_t o_gated = off;
-    off += align256((size_t)(n_steps + 1) * sizeof(double));
-    const size_t o_psi = off;
-    off += 2 * (size_t)state * sizeof(double2);
+    const size_t off = step_buffers(g, n_steps, nullptr, nullptr);
     // counted: two state vectors, the field, 512 bytes and 80 for every 256 chunks less a halo on each side
     const int segment = 4 * TDSE_WAVE - 2 * g.halo_lanes;
     const size_t counted = 512 + align256(80 * (size_t)((g.nchunks + segment - 1) / segment)) +
@@ -1566,11 +1580,8 @@ int ctdse_propagate_one_noalloc(const ctdse_geometry *geom, int n_steps, const d
                                                   std::to_string((size_t)CTDSE_NOALLOC_SCRATCH_BYTES) + " it holds");
     void *base = nullptr;
     if (scratch_address(&base) != CTDSE_OK) return g_status;
-    char *p = static_cast<char *>(base);
-    double2 *psi = reinterpret_cast<double2 *>(p + o_psi);
-    const StepBufs b{reinterpret_cast<TdseGeom *>(p + o_geom), reinterpret_cast<TdseInst *>(p + o_inst),
-                     reinterpret_cast<double *>(p + o_part), reinterpret_cast<double *>(p + o_gated),
-                     {psi, psi + state}};
+    StepBufs b;
+    step_buffers(g, n_steps, static_cast<char *>(base), &b);
     std::lock_guard<std::mutex> lock(g_launch_mutex);
     return enqueue_steps(s, b, (hipStream_t)stream);
 }

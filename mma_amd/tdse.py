@@ -359,8 +359,10 @@ def propagate_stepwise(geometry, fields, out=None, stream=None):
     s_off = (c_longlong * n_inst)(*[i * 2 * S for i in range(n_inst)])
     o_off = (c_longlong * n_inst)(*[i * 5 * n_steps for i in range(n_inst)])
     st = c_void_p(states.data_ptr())
+    k0 = (c_int * n_inst)()
+    step = np.frombuffer(k0, dtype=np.intc)
     for k in range(n_steps):
-        k0 = (c_int * n_inst)(*([k] * n_inst))
+        step[:] = k
         init = st if k > 0 else c_void_p()  # step 0 starts from psi0 and writes the state vector
         _raise(L.ctdse_propagate_states(n_inst, handles, steps, k0, ones, c_void_p(F.data_ptr()), f_off, init,
                                         s_off, st, s_off, 1, c_void_p(out.data_ptr()), o_off,
