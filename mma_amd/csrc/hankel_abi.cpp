@@ -185,9 +185,11 @@ hipError_t enqueue_prefactor(const hk_medium *m, int nz, const double *zgrid, in
 // Workgroups of hk_direct_kernel per frequency, its sources dealt to `parts` threads per screen radius.
 long long direct_blocks(const hk_planes *p, int parts) { return ((long long)p->nrho * parts + 255) / 256; }
 
-// parts: doubled up to 16 while there are fewer than four workgroups per CU.  64 frequencies x 200 radii to 301 screen
-// points: 86 us with 1, 57 with 2, 42 with 4 to 16; 16 x 1500 to 300: 515 with 1, 64 with 16; 200 x 300 to 600: 198
-// with 1, 143 with 2, 189 with 16.
+// parts: doubled up to 16 while there are fewer than four workgroups per CU.  Calls with 1, 2, 4, 8 and 16 parts, in us:
+// 64 frequencies x 200 radii to 301 screen points 174, 93, 74, 77, 75 (the rule takes 16); 16 x 1500 to 300 567, 331, 198,
+// 125, 104 (16); 200 x 300 to 600 215, 181, 184, 201, 230 (4: 2000 workgroups, 2 would be 1000); 300 x 300 to 300
+// 202, 172, 151, 166, 187 (4); 400 x 100 to 300 105, 106, 102, 119, 148 (2); 512 x 300 to 600 358, 338, 353, 405, 493 (1).
+// A line at 2000 workgroups would take 2 there, but 4 for 700 x 64 to 200 (95, 98, 105).
 int direct_parts(const hk_planes *p)
 {
     int parts = 1;
@@ -215,16 +217,11 @@ int plan_grid64(const hk_planes *p, int outputs, int per_plane, const double *ho
     const double direct = (double)p->nz * p->nr / parts * (0.2e-6 + 0.155e-6 * p->no * direct_blocks(p, parts) / 256.0);
     if (direct < 100e-6 || p->nr > 64 * kBlocks64 || outputs > (1 << 20)) return HK_OK;
     HostGrids hg;
-    std::vector<double> rho;
-    if (host_grids(p, hg) != HK_OK || host_grid(rho, host_rho, p->rho, p->nrho) != HK_OK) return g_status;
-    double rho_max = 0.0, o_max = 0.0, before = 0.0;
+    if (host_grids(p, hg) != HK_OK) return g_status;
+    double o_max = 0.0, before = 0.0;
     hk_grid64 g{};
     g.inv_c = kInvC;
     g.d_min = INFINITY;
-    for (double v : rho) {
-        if (!std::isfinite(v)) return HK_OK;
-        rho_max = std::max(rho_max, std::fabs(v));
-    }
     for (double v : hg.o) {
         if (!(v >= 0.0) || !std::isfinite(v)) return HK_OK;
         o_max = std::max(o_max, v);
@@ -241,29 +238,45 @@ int plan_grid64(const hk_planes *p, int outputs, int per_plane, const double *ho
         g.d_max = std::max(g.d_max, d);
     }
     const double q_max = o_max * g.inv_c / g.d_min * g.r_max;
-    if (!(q_max * rho_max >= 1.0) || !(q_max * rho_max < 1e5)) return HK_OK;
-    // rho_max h: (rho h)^P max prod |f - d_i| / P! = 2e-16; h to 24 bits, so that l h is exact
-    double bound = 1.0;
-    for (int i = 0; i < kNodes64; i++) bound *= std::fabs(0.5 - (i - (kNodes64 / 2 - 1))) / (i + 1);
-    g.h = (double)std::nextafterf((float)(std::pow(2e-16 / bound, 1.0 / kNodes64) / rho_max), 0.0f);
-    g.inv_h = 1.0 / g.h;
-    const int need = (int)(q_max * g.inv_h) + kNodes64 + 3;
-    g.ld = (need + kStage64 - 1) / kStage64 * kStage64;
     const int blocks = (p->nr + 63) / 64;
+    // the grid for screen radii up to rho_max, and this form's seconds on it: 200 FP64 instructions a source and output
+    // and 0.8 us a plane in a row, 150 an entry of the table, the spread sources written and read, the product
+    // at 40 TFLOP/s or its tiles' serial sum, the launches.  (64 planes x 300 frequencies x 256 radii to 512 screen
+    // points: 0.41 ms against 9.6, 256 x 768 x 512 to 1024: 1.76 against 246.)
+    auto grid_for = [&](double rho_max) {
+        // rho_max h: (rho h)^P max prod |f - d_i| / P! = 2e-16; h to 24 bits, so that l h is exact
+        double bound = 1.0;
+        for (int i = 0; i < kNodes64; i++) bound *= std::fabs(0.5 - (i - (kNodes64 / 2 - 1))) / (i + 1);
+        g.h = (double)std::nextafterf((float)(std::pow(2e-16 / bound, 1.0 / kNodes64) / rho_max), 0.0f);
+        g.inv_h = 1.0 / g.h;
+        const int need = (int)(q_max * g.inv_h) + kNodes64 + 3;
+        g.ld = (need + kStage64 - 1) / kStage64 * kStage64;
+        const double rate = 3.9e13, rows = 2.0 * p->no * outputs, in_row = per_plane ? 1 : p->nz;
+        const double sources = (double)p->no * p->nr * in_row * outputs;
+        return sources * 200.0 / rate + in_row * ((blocks + 7) / 8) * 0.8e-6 + (double)p->nrho * g.ld * 150.0 / rate +
+               rows * g.ld * 16.0 / 3e12 + std::max(2.0 * rows * g.ld * p->nrho / 4e13, g.ld * 27e-9) + 60e-6;
+    };
+    auto in_range = [&](double rho_max) { return q_max * rho_max >= 1.0 && q_max * rho_max < 1e5; };
+    // The seconds grow with rho_max, which is one of a screen's two ends as a rule: with those first, a call that keeps the
+    // direct kernel does not go through the screen (60000 radii: 58 us of a call of 506).
+    std::vector<double> copy;
+    if (!host_rho) {
+        if (host_grid(copy, nullptr, p->rho, p->nrho) != HK_OK) return g_status;
+        host_rho = copy.data();
+    }
+    const double ends = std::max(std::fabs(host_rho[0]), std::fabs(host_rho[p->nrho - 1]));
+    if (!(q_max * ends < 1e5) || (in_range(ends) && direct <= grid_for(ends))) return HK_OK;
+    double rho_max = 0.0;
+    for (int m = 0; m < p->nrho; m++) {
+        if (!std::isfinite(host_rho[m])) return HK_OK;
+        rho_max = std::max(rho_max, std::fabs(host_rho[m]));
+    }
+    if (!in_range(rho_max) || direct <= grid_for(rho_max)) return HK_OK;
     for (int b = 0; b < blocks; b++) {
         const double k = o_max * g.inv_c, r0 = hg.r[b * 64], r1 = hg.r[std::min(b * 64 + 63, p->nr - 1)];
         g.bins += (int)(k / g.d_min * r1 * g.inv_h) + kNodes64 + 4 - (int)(k / g.d_max * r0 * g.inv_h);
     }
     if ((size_t)g.bins * sizeof(double2) > kLds64) return HK_OK;
-    // This form's: 200 FP64 instructions a source and output and 0.8 us a plane in a row, 150 an entry of the table,
-    // the spread sources written and read, the product at 40 TFLOP/s or its tiles' serial sum, the launches.
-    // (64 planes x 300 frequencies x 256 radii to 512 screen points: 0.41 ms against 9.6, 256 x 768 x 512 to 1024:
-    // 1.76 against 246.)
-    const double rate = 3.9e13, rows = 2.0 * p->no * outputs, in_row = per_plane ? 1 : p->nz;
-    const double sources = (double)p->no * p->nr * in_row * outputs;
-    const double grid = sources * 200.0 / rate + in_row * ((blocks + 7) / 8) * 0.8e-6 + (double)p->nrho * g.ld * 150.0 / rate +
-                        rows * g.ld * 16.0 / 3e12 + std::max(2.0 * rows * g.ld * p->nrho / 4e13, g.ld * 27e-9) + 60e-6;
-    if (direct <= grid) return HK_OK;
     plan->g = g;
     const size_t tiles = (size_t)((p->nrho + kTile64 - 1) / kTile64) * ((2 * (size_t)p->no + kTile64 - 1) / kTile64);
     const size_t one = 2 * (size_t)p->no * g.ld * sizeof(double);
@@ -408,12 +421,10 @@ int hk_direct(const hk_planes *p, int n_out, const double *weights, int per_plan
     hipStream_t s = (hipStream_t)stream;
     const int parts = direct_parts(p);
     dim3 grid((unsigned)p->no, (unsigned)direct_blocks(p, parts));
-    if (p->src_c64)
-        hipLaunchKernelGGL(hk_direct_kernel<float2>, grid, dim3(256), 0, s, *p, n_out, weights, per_plane,
-                           reinterpret_cast<double2 *>(out), kInvC, (int)uniform, dr, parts);
-    else
-        hipLaunchKernelGGL(hk_direct_kernel<double2>, grid, dim3(256), 0, s, *p, n_out, weights, per_plane,
-                           reinterpret_cast<double2 *>(out), kInvC, (int)uniform, dr, parts);
+    auto kernel = p->src_c64 ? (parts > 1 ? hk_direct_kernel<float2, true> : hk_direct_kernel<float2, false>)
+                             : (parts > 1 ? hk_direct_kernel<double2, true> : hk_direct_kernel<double2, false>);
+    hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, *p, n_out, weights, per_plane, reinterpret_cast<double2 *>(out), kInvC,
+                       (int)uniform, dr, parts);
     HK_HIP(hipGetLastError());
     HK_HIP(hipStreamSynchronize(s));
     return HK_OK;

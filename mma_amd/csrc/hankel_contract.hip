@@ -52,18 +52,20 @@ constexpr int kAnchor = 32;     // exact sincos every kAnchor rotated steps
 // grid (no, ceil(nrho / (256 / parts))): one workgroup per frequency and 256 / parts screen radii, all
 // planes.  parts: the sources of a tile are dealt to that many threads per screen radius, whose sums are added
 // in their order (a small call leaves most of the chip idle, and a thread's elements follow each other, 0.28 us
-// apiece).
-template <typename S>
+// apiece).  DEALT: parts > 1; a kernel of its own, since a loop whose ends each thread has for itself keeps its count
+// and its LDS addresses in vector registers (2048 frequencies x 100 radii to 700 screen points, where parts is 1:
+// 497 us with that loop, 445 without).
+template <typename S, bool DEALT>
 __global__ void __launch_bounds__(kThreads)
 hk_direct_kernel(hk_planes p, int n_out, const double *weights, int per_plane, double2 *out, double inv_c,
                  int uniform_r, double dr, int parts)
 {
     __shared__ double2 u[kJTile];
     __shared__ double rr[kJTile];
-    __shared__ double2 sums[kThreads];
+    __shared__ double2 sums[DEALT ? kThreads : 1];
     const int o = blockIdx.x;
-    const int width = kThreads / parts, part = threadIdx.x / width;
-    const int m = blockIdx.y * width + threadIdx.x % width;
+    const int width = DEALT ? kThreads / parts : kThreads, part = DEALT ? threadIdx.x / width : 0;
+    const int m = blockIdx.y * width + (DEALT ? threadIdx.x % width : threadIdx.x);
     const bool live = m < p.nrho;
     const double rho = live ? p.rho[m] : 0.0;
     const double K = p.ogrid[o] * inv_c;
@@ -85,7 +87,7 @@ hk_direct_kernel(hk_planes p, int n_out, const double *weights, int per_plane, d
             }
             __syncthreads();
             if (!live) continue;
-            const int j_lo = nj * part / parts, j_hi = nj * (part + 1) / parts;
+            const int j_lo = DEALT ? nj * part / parts : 0, j_hi = DEALT ? nj * (part + 1) / parts : nj;
             if (uniform_r) {
                 // cos, sin of x_j by rotation through the angle a dr, re-anchored every kAnchor steps
                 double ct, st;
@@ -114,7 +116,7 @@ hk_direct_kernel(hk_planes p, int n_out, const double *weights, int per_plane, d
                 }
             }
         }
-        if (parts > 1) {
+        if (DEALT) {
             sums[threadIdx.x] = acc;
             __syncthreads();
             if (part == 0)
@@ -144,10 +146,14 @@ hk_direct_kernel(hk_planes p, int n_out, const double *weights, int per_plane, d
         if (q < n_out) out[((long long)q * p.nrho + m) * p.no + o] = acc_out[q];
 }
 
-template __global__ void hk_direct_kernel<double2>(hk_planes, int, const double *, int, double2 *, double, int,
-                                                   double, int);
-template __global__ void hk_direct_kernel<float2>(hk_planes, int, const double *, int, double2 *, double, int,
-                                                  double, int);
+template __global__ void hk_direct_kernel<double2, false>(hk_planes, int, const double *, int, double2 *, double, int,
+                                                          double, int);
+template __global__ void hk_direct_kernel<double2, true>(hk_planes, int, const double *, int, double2 *, double, int,
+                                                         double, int);
+template __global__ void hk_direct_kernel<float2, false>(hk_planes, int, const double *, int, double2 *, double, int,
+                                                         double, int);
+template __global__ void hk_direct_kernel<float2, true>(hk_planes, int, const double *, int, double2 *, double, int,
+                                                        double, int);
 
 namespace {
 

@@ -30,7 +30,7 @@ constexpr int kWalkParallelMax = 4096;  // pressure tables up to this length: on
 __global__ void hk_prefactor_finish_kernel(int nz, int no, const double *ogrid, const double *exit_abs, double2 *pre,
                                            double *renorm);
 
-template <typename S>
+template <typename S, bool DEALT>
 __global__ void hk_direct_kernel(hk_planes p, int n_out, const double *weights, int per_plane, double2 *out,
                                  double inv_c, int uniform_r, double dr, int parts);
 
