@@ -300,7 +300,8 @@ int run_grid64(const hk_planes *p, int outputs, const double *weights, const Pla
     auto spread = p->src_c64 ? hk64_spread_kernel<float2> : hk64_spread_kernel<double2>;
     HK_HIP(hipFuncSetAttribute((const void *)spread, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLds64));
     hipLaunchKernelGGL(hk_fill_int_kernel, dim3(1), dim3(64), 0, s, flag, 1, 0);
-    hipLaunchKernelGGL(hk64_bessel_kernel, dim3((g.ld + 255) / 256, p->nrho), dim3(256), 0, s, p->nrho, p->rho, g, table);
+    hipLaunchKernelGGL(hk64_bessel_kernel, dim3((g.ld + 255) / 256, (unsigned)std::min(p->nrho, 65535)), dim3(256), 0, s, p->nrho, p->rho,
+                       g, table);
     const int threads = std::min(kSpread64, 64 * ((p->nr + 63) / 64));
     const int N = 2 * p->no, mt = (p->nrho + kTile64 - 1) / kTile64, nt = (N + kTile64 - 1) / kTile64;
     for (int q = 0; q < outputs; q += plan.chunk) {

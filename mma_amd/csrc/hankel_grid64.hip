@@ -267,13 +267,15 @@ template __global__ void hk64_spread_kernel<float2>(hk_planes, hk_grid64, int, c
 // rho Q_l, which every source near that bin would share, is put back: cos and sin of the exact product.
 __global__ void hk64_bessel_kernel(int nrho, const double *rho, hk_grid64 g, double *out)
 {
-    const int l = blockIdx.x * blockDim.x + threadIdx.x, m = blockIdx.y;
+    const int l = blockIdx.x * blockDim.x + threadIdx.x;
     if (l >= g.ld) return;
-    const double q = (double)(l - P / 2) * g.h, a = rho[m];
-    const double x = a * q, e = fma(a, q, -x);
-    double s, c;
-    sincos_wide(x, &s, &c);
-    out[(long long)m * g.ld + l] = hk::j0(x, fma(-e, s, c), fma(e, c, s));
+    for (int m = blockIdx.y; m < nrho; m += gridDim.y) {  // (a grid has 65535 rows at most)
+        const double q = (double)(l - P / 2) * g.h, a = rho[m];
+        const double x = a * q, e = fma(a, q, -x);
+        double s, c;
+        sincos_wide(x, &s, &c);
+        out[(long long)m * g.ld + l] = hk::j0(x, fma(-e, s, c), fma(e, c, s));
+    }
 }
 
 // out[m][n] = sum_l A[m][l] B[n][l] in FP64: A the J0 table (M rows), B the spread sources (N rows per output).

@@ -49,3 +49,12 @@ def test_one_radius_beyond_the_grid_keeps_the_elementwise_kernel():
         far = rho.copy()
         far[at] = 400 * rho.max()
         assert table_bytes(src, z, o, r, far, D, 3, False) == 0
+
+
+# a launch has 65535 rows of blocks at most
+@pytest.mark.parametrize("nrho", [65535, 65536, 70001])
+def test_more_screen_radii_than_rows_of_a_launch(nrho):
+    src, z, o, r, rho, D, weights = case(20, 3, 64, 2)
+    rho = np.linspace(0.0, rho.max() / 20, nrho)
+    assert table_bytes(src, z, o, r, rho, D, 3, False) > 0
+    check(src, z, o, r, rho, D, weights)
