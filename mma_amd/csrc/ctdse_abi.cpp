@@ -4,6 +4,7 @@
 // data across the boundary and owns the reference's malloc/calloc output arrays.
 #include "ctdse.h"
 #include "tdse_internal.h"
+#include "tdse_plan.h"
 
 #include <algorithm>
 #include <cmath>
@@ -455,74 +456,6 @@ int share_lattices(const std::vector<ctdse_geometry *> &gs)
     return CTDSE_OK;
 }
 
-// How the resident kernel covers nx points whose carries reach `reach` points: lanes of C points,
-// waves and windows (TdseResident).  A function of the geometry alone, so an instance's results do
-// not depend on the batch around it.  Costs in units of an instruction per lane and step: 55 per
-// point and 330 for the scans, the phase and the sums (1210, 1650, 2090; a step of 8 full waves takes 5.6, 7.3 and 9.7 us).
-//   One window: (C, waves) by the work of a CU per instance and step (8 waves fit one, so a CU holds
-//   8 / waves workgroups), and within a quarter of the least by a step's latency: 16 points x 8 waves
-//   rather than 32 x 4 for 8001 points, 18 % more work in half the time per step.
-//   Several (the grid is larger than 8 waves x 32 lanes' points): `steps` steps between a window's load
-//   and store cost a halo of steps x reach points at each inner edge; loading, b included, and
-//   storing cost about 60 per point.
-bool plan_resident(int nx, int reach, TdseResident &R)
-{
-    static const int kChunks[3] = {16, 24, 32};
-    const int margin = reach + 2;  // per step: both recurrences, and the right-hand side's neighbours
-    R.chunk = 0;
-    auto per_step = [](int C) { return 55.0 * C + 330.0; };
-    double least = INFINITY;
-    for (int pass = 0; pass < 2; pass++) {
-        double best = INFINITY;
-        for (int C : kChunks) {
-            if (reach > 16 * C) continue;
-            const int waves = (nx + C - 1 + 64 * C - 1) / (64 * C);
-            if (waves > TDSE_MAX_WAVES) continue;
-            const double cost = per_step(C) / (TDSE_MAX_WAVES / waves);
-            if (pass == 0) {
-                least = std::min(least, cost);
-            } else if (cost <= 1.25 * least && per_step(C) < best) {
-                best = per_step(C);
-                R.chunk = C;
-                R.waves = waves;
-            }
-        }
-    }
-    R.reach = reach;
-    R.windows = 1;
-    R.steps = TDSE_RES_RING;
-    R.stride = R.halo = 0;
-    if (R.chunk) return true;
-    double best = INFINITY;
-    for (int C : kChunks) {
-        if (reach > 16 * C) continue;
-        const int lanes = 64 * TDSE_MAX_WAVES, total = (nx + C - 1 + C - 1) / C;
-        for (int T = TDSE_RES_RING; T >= 1; T--) {
-            const int halo = (T * margin + C - 1) / C, stride = lanes - 2 * halo;
-            if (stride < 64) continue;
-            const int n = 1 + (total - lanes + stride - 1) / stride;
-            const double cost = n * (T * per_step(C) + 60.0 * C) / T;
-            if (cost < best) {
-                best = cost;
-                R.chunk = C;
-                R.waves = TDSE_MAX_WAVES;
-                R.windows = n;
-                R.steps = T;
-                R.stride = stride;
-                R.halo = halo;
-            }
-        }
-    }
-    return R.chunk > 0;
-}
-
-// Entries of a resident table of nx points in lanes of C: whole tiles, one zero chunk at least.
-long long resident_entries(int nx, int C) { return (long long)(((nx + C - 1) / C + 1 + 63) / 64) * 64 * C; }
-
-// Points before a run of pivots from the double ones, whose error of 1e-16 decays by rho^2 a point: to
-// below 1e-20 (rho^reach = 1e-17).
-int resident_warm(int reach) { return reach / 8 + 4; }
-
 int build_resident(const ctdse_geometry *G, int C, DevMem &mem)
 {
     const long long n = resident_entries(G->dev.nx, C);
@@ -534,32 +467,6 @@ int build_resident(const ctdse_geometry *G, int C, DevMem &mem)
                        G->dev.ib, G->dev.nx, G->dev.k36, C, chunks, resident_warm(G->reach), t, t + n, t + 2 * n);
     HIP_CHECK(hipGetLastError());
     return CTDSE_OK;
-}
-
-// The windows of one instance alone: lanes of 16 points (24 where carries reach further), four waves, one
-// per SIMD, a window; as many steps per launch as leave at most kOneWindows windows.  With 16001
-// points: 39 windows of 4096 points, 13 steps a launch.
-constexpr int kOneWindows = 64;
-void plan_one(int nx, int reach, TdseResident &R)
-{
-    const int C = reach <= 16 * 16 ? 16 : 24, total = (nx + C - 1 + C - 1) / C, margin = reach + 2;
-    R.chunk = C;
-    R.reach = reach;
-    R.windows = 1;
-    R.steps = TDSE_RES_RING;
-    R.stride = R.halo = 0;
-    R.waves = std::min(TDSE_ONE_WAVES, (total + 63) / 64);
-    const int lanes = 64 * TDSE_ONE_WAVES;
-    if (total <= lanes) return;
-    for (int T = TDSE_RES_RING; T >= 1; T--) {
-        const int halo = (T * margin + C - 1) / C, stride = lanes - 2 * halo;
-        if (stride < 1) continue;
-        R.windows = 1 + (total - lanes + stride - 1) / stride;
-        R.steps = T;
-        R.stride = stride;
-        R.halo = halo;
-        if (R.windows <= kOneWindows || T == 1) return;
-    }
 }
 
 // The lane-tile tables that a plan R of geometry G reads: its own, or those of its lattice (the widest
@@ -621,9 +528,10 @@ int add_resident(const std::vector<ctdse_geometry *> &gs)
     for (ctdse_geometry *G : gs) {
         if (!G || !G->dev.g) continue;
         const ctdse_geometry *src = G->lattice ? widest[G->lattice.get()] : G;
-        plan_one(G->dev.nx, G->reach, G->dev.one);
-        if (plan_resident(G->dev.nx, G->reach, G->dev.res)) plans.push_back({G, &G->dev.res});
-        plans.push_back({G, &G->dev.one});
+        if (src->dev.nx <= kResidentPoints) {
+            if (plan_one(G->dev.nx, G->reach, G->dev.one)) plans.push_back({G, &G->dev.one});
+            if (plan_resident(G->dev.nx, G->reach, G->dev.res)) plans.push_back({G, &G->dev.res});
+        }
         while (jobs.size() < plans.size()) {
             jobs.emplace_back();
             if (attach_tables(G, src, *plans[jobs.size() - 1].second, jobs.back()) != CTDSE_OK) return g_status;
@@ -1289,6 +1197,7 @@ int enqueue_steps(const InstSpec &s, const StepBufs &b, hipStream_t stream)
 int propagate_steps(const InstSpec &s, hipStream_t stream)
 {
     const TdseGeom &g = s.geom->dev;
+    if (g.one.chunk == 0) return propagate({s}, stream);
     DevMem mem;  // (an allocation for each buffer: 38 us for one step of 201 points, so 34)
     StepBufs b;
     HIP_CHECK(mem.alloc(step_buffers(g, s.n_steps, nullptr, nullptr)));
@@ -1567,7 +1476,7 @@ int ctdse_propagate_one_noalloc(const ctdse_geometry *geom, int n_steps, const d
     s.field = field;
     s.out = out;
     const TdseGeom &g = geom->dev;
-    const size_t off = step_buffers(g, n_steps, nullptr, nullptr);
+    const size_t off = g.one.chunk > 0 ? step_buffers(g, n_steps, nullptr, nullptr) : SIZE_MAX;
     // counted: two state vectors, the field, 512 bytes and 80 for every 256 chunks less a halo on each side
     const int segment = 4 * TDSE_WAVE - 2 * g.halo_lanes;
     const size_t counted = 512 + align256(80 * (size_t)((g.nchunks + segment - 1) / segment)) +
