@@ -1,7 +1,7 @@
 // Crank-Nicolson propagation with the wavefunction resident on the chip (1DTDSE/sources/prop.c:24-347).
 //
 // tdse_propagate.hip streams psi through HBM once per step (or two): it runs at the memory's rate
-// and, per point, spends more instructions on scans than on the solve.  A grid of up to 16384
+// and, per point, spends more instructions on scans than on the solve.  A grid of up to 16353
 // points fits the registers of one compute unit, so here a workgroup of NW waves keeps the whole
 // state of its instance in registers for the whole run: every lane owns C consecutive points
 // (C = 16, 24 or 32).  Larger grids are covered by overlapping windows of that size, each
@@ -76,14 +76,6 @@ __device__ inline double2 row(const double2 *base, unsigned lane_off, int i)
     const TDSE_GLOBAL char *p = (const TDSE_GLOBAL char *)base + i * 1024;
     const tdse_d2 v = *(const TDSE_GLOBAL tdse_d2 *)(p + lane_off);
     return make_double2(v.x, v.y);
-}
-
-// a value that all lanes agree on, in scalar registers
-__device__ inline double uniform(double v)
-{
-    const long long b = __builtin_bit_cast(long long, v);
-    const int lo = __builtin_amdgcn_readfirstlane((int)b), hi = __builtin_amdgcn_readfirstlane((int)(b >> 32));
-    return __builtin_bit_cast(double, ((long long)hi << 32) | (unsigned int)lo);
 }
 
 // r with its fields to be read again from here on, and not kept in registers across what came before

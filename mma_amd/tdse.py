@@ -337,8 +337,9 @@ def propagate_stepwise(geometry, fields, out=None, stream=None):
     one kernel launch per time step over the whole batch, each instance's state held in HBM
     between launches and stepped in place (ctdse_propagate_states).  Same arguments and
     result as propagate_batch for a uniform batch (n_steps = L - 1 for every row), bit for
-    bit up to 16384 grid points: the same solve and observable order run either way.  Larger
-    grids are solved in windows of several steps, so there the two agree to rounding."""
+    bit up to 16353 grid points: the same solve and observable order run either way.  Larger
+    grids are solved in windows of several steps, which a run of one step cuts differently, so there
+    the two agree to rounding."""
     from .adjoint import gate
     _check_device(fields, "fields")
     L = _lib()
