@@ -49,6 +49,17 @@ def log(*a):
     print(*a, file=sys.stderr, flush=True)
 
 
+def propagation_rate(pt_steps, seconds, on_chip):
+    """What bounds a propagation of pt_steps grid points and steps, and its rate against that: the vector units' FP64
+    rate where the states stay on the chip, else the memory's, which carries psi in and out every step."""
+    if on_chip:
+        rate = FLOP_PER_PT_STEP * pt_steps / seconds / 1e12
+        return {"bound": "fp64", "achieved": rate, "peak": FP64_PEAK_TFLOPS, "unit": "TFLOP/s",
+                "frac": rate / FP64_PEAK_TFLOPS}
+    rate = BYTES_PER_PT_STEP * pt_steps / seconds / 1e9
+    return {"bound": "hbm", "achieved": rate, "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": rate / HBM_PEAK_GBS}
+
+
 class stdout_to_stderr:
     """Sends file descriptor 1 to stderr for the duration (the reference's C code prints its
     progress with printf; stdout carries only the result line)."""
@@ -315,7 +326,9 @@ def hankel_measure(cpu=True):
     Henke f2) x 2048 frequencies (harmonics 11-61 of 800 nm) x 512 radii (0-200 um) onto 1024
     screen radii (0-7 mm) at 1 m.  Times the device work of each contraction (pre-factor tables
     included) on complex128 sources, and the matrix-core ones on complex64 sources too, and states
-    every result's error against the FP64 direct contraction."""
+    every result's error against the FP64 contraction that evaluates J0 for every element
+    ('fp64-direct', hk_direct; 'fp64' takes J0 from one table here)."""
+    from ctypes import byref
     import torch
     from mma_amd import hankel as H, workloads as W
     zall, rg, og, rho, src, distance = W.hankel_workload()
@@ -336,6 +349,13 @@ def hankel_measure(cpu=True):
         # after the pass (check_tables), as Hankel_long does before it hands results over
         tab = H._PreFactor(zg, rg, og, "Ar", pressure, "Henke", True, "NIST", True, 1.0, defer=True)
         tabs.append(tab)
+        if kind == "fp64-direct":
+            keep = []
+            p = H._planes_struct(sources, zg, og, rg, rho, distance, True, tab.pre, 1, keep)
+            w3 = H._dev(Wt)
+            far = torch.empty((len(Wt), p.nrho, p.no), dtype=torch.complex128, device="cuda")
+            H._check(H._L().hk_direct(byref(p), len(Wt), H._ptr(w3), 0, H._ptr(far), H._stream()))
+            return far
         if kind == "fp64":
             return H.direct(sources, zg, og, rg, rho, distance, weights=Wt, pre=tab.pre)
         return H.gridded(sources, zg, og, rg, rho, distance, Wt, pre=tab.pre, kind=kind)
@@ -346,10 +366,10 @@ def hankel_measure(cpu=True):
         tabs.clear()
 
     out, res = {}, {}
-    for kind in ("fp64", "fp64-grid", "fp32-mfma", "bf16x3-mfma", "bf16x6-mfma", "fp16x3-mfma"):
+    for kind in ("fp64-direct", "fp64", "fp64-grid", "fp32-mfma", "bf16x3-mfma", "bf16x6-mfma", "fp16x3-mfma"):
         run(kind)  # warm-up (code objects, allocations)
         torch.cuda.synchronize()
-        reps = 1 if kind == "fp64" else 5
+        reps = 1 if kind == "fp64-direct" else 5
         check_tables()
         t0 = time.perf_counter()
         for _ in range(reps):
@@ -375,11 +395,11 @@ def hankel_measure(cpu=True):
         res64[kind] = r
         log("hankel %s, complex64 sources: %.2f ms" % (kind, out64[kind] * 1e3))
     del src64
-    ref = res["fp64"]
+    ref = res["fp64-direct"]
     errors = {}
     # each output against its own scale: the integrated field (a sum over planes weighted by the
     # plane spacing) is ~1/Nz of a plane's magnitude, so a max over all three would hide its error
-    for kind in ("fp64-grid", "fp32-mfma", "bf16x3-mfma", "bf16x6-mfma", "fp16x3-mfma"):
+    for kind in ("fp64", "fp64-grid", "fp32-mfma", "bf16x3-mfma", "bf16x6-mfma", "fp16x3-mfma"):
         errors[kind] = {}
         for i, name in enumerate(("FF_integrated", "entry_plane_transform", "exit_plane_transform")):
             d = res[kind][i] - ref[i]
@@ -399,11 +419,11 @@ def hankel_measure(cpu=True):
         "elements": elems,
         "seconds": out,
         "errors_vs_fp64_direct": errors,
-        "speedup_vs_fp64_direct": {k: out["fp64"] / out[k] for k in out if k != "fp64"},
+        "speedup_vs_fp64_direct": {k: out["fp64-direct"] / out[k] for k in out if k != "fp64-direct"},
         "seconds_complex64_sources": out64,
         "errors_complex64_sources_vs_fp64_direct": errors64,
-        "fp64_direct_j0_per_s": elems / out["fp64"],
-        "fp64_direct_algorithmic_tflops": 4.0 * elems / out["fp64"] / 1e12,
+        "fp64_direct_j0_per_s": elems / out["fp64-direct"],
+        "fp64_direct_algorithmic_tflops": 4.0 * elems / out["fp64-direct"] / 1e12,
         "grid_points_q": nq,
         "gemm_flops": gemm_flops,
     }
@@ -464,7 +484,8 @@ def uneven_measure(steps=2, config=None):
             "steps_range": [int(min(n_steps)), int(max(n_steps))], "pt_steps": pt,
             "max_over_min_instance_work": float(work.max() / work.min()),
             "value": pt / wall, "unit": "grid-pt-steps/s", "seconds": wall, "kernel_s": kern,
-            "hbm_frac_psi_only": BYTES_PER_PT_STEP * pt / kern / 1e9 / HBM_PEAK_GBS,
+            "roofline": propagation_rate(pt, kern, res.config.library_choice),
+            "library_choice": res.config.library_choice,
             "setup_s": t_setup, "gs_cv": W.UNEVEN_CV,
             "gs_iterations_max": max(g.gs_iterations for g in geoms), "tune_s": t_tune, "launch_config": list(res.config.as_tuple()),
             "default_config": list(default.as_tuple()), "tune_table": [list(r) for r in res.table[:6]],
@@ -644,7 +665,6 @@ def main():
     kern_ms = float(np.mean([a.elapsed_time(b) for a, b in ev]))
     ms_per_step = wall / args.steps * 1e3
     value = pt_steps / (wall / args.steps)
-    achieved = BYTES_PER_PT_STEP * pt_steps / (kern_ms * 1e-3) / 1e9
     gpu_rows = out[:, :4, :].cpu().numpy()  # for the parity check against the CPU reference members
     finite = bool(np.all(np.isfinite(gpu_rows)))
 
@@ -682,7 +702,7 @@ def main():
         hk = hankel_measure(cpu=not args.no_cpu)
         torch.cuda.empty_cache()
 
-    # the box's practical ceilings, same units as achieved: read + write (the propagation's
+    # the box's practical memory ceilings in GB/s: read + write (the streaming propagation's
     # traffic mix), read only and write only
     copy_gbs, read_gbs, write_gbs = (1e3 * stream_rate(kind, 16, 32) for kind in ("copy", "read", "write"))
     torch.cuda.empty_cache()
@@ -693,6 +713,16 @@ def main():
         with stdout_to_stderr():
             cpu, parity = cpu_baseline(gpu_rows=gpu_rows)
 
+    on_chip = tuned.config.library_choice
+    roofline = propagation_rate(pt_steps, kern_ms * 1e-3, on_chip)
+    roofline.update(copy_ceiling=copy_gbs, read_only_ceiling=read_gbs, write_only_ceiling=write_gbs)
+    if on_chip:
+        roofline["kernel"] = "tdse_resident_kernel"
+    else:
+        steps_per_pass = tuned.config.as_tuple()[2]
+        roofline.update(frac_of_copy_ceiling=roofline["achieved"] / copy_gbs if copy_gbs else None,
+                        traffic=MEASURED_TRAFFIC_BYTES.get(steps_per_pass) if (args.n_r, args.n_z) == (64, 64) else None,
+                        kernel="tdse_propagate_pair_stash_kernel" if steps_per_pass == 2 else "tdse_propagate_kernel")
     line = {
         "metric": METRIC, "value": value, "unit": "grid-pt-steps/s", "n_gpus": 1, "steps": args.steps,
         "warmup": args.warmup, "ms_per_step": ms_per_step, "higher_is_better": True, "scaling": "weak",
@@ -700,19 +730,7 @@ def main():
         "config": {"workload": "tdse-batch-gaussian-beam", "instances": n_inst, "grid_r_x_z": [args.n_r, args.n_z],
                    "Nx": nx, "dx": g["dx"], "dt": 0.25, "time_steps": n_steps, "atom": "Ar (a=1.1893)",
                    "field": "800nm 10-cycle sin2, 1.5e14 W/cm2 peak, w0=100um", "precision": "complex128"},
-        "roofline": {"bound": "fp64", "achieved": FLOP_PER_PT_STEP * pt_steps / (kern_ms * 1e-3) / 1e12,
-                     "peak": FP64_PEAK_TFLOPS, "unit": "TFLOP/s",
-                     "frac": FLOP_PER_PT_STEP * pt_steps / (kern_ms * 1e-3) / 1e12 / FP64_PEAK_TFLOPS,
-                     "copy_ceiling": copy_gbs, "read_only_ceiling": read_gbs, "write_only_ceiling": write_gbs,
-                     "kernel": "tdse_resident_kernel"} if tuned.config.library_choice else
-                    {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                     "frac": achieved / HBM_PEAK_GBS,
-                     "copy_ceiling": copy_gbs, "frac_of_copy_ceiling": achieved / copy_gbs if copy_gbs else None,
-                     "read_only_ceiling": read_gbs, "write_only_ceiling": write_gbs,
-                     "traffic": MEASURED_TRAFFIC_BYTES.get(tuned.config.as_tuple()[2])
-                     if (args.n_r, args.n_z) == (64, 64) else None,
-                     "kernel": "tdse_propagate_pair_stash_kernel" if tuned.config.as_tuple()[2] == 2
-                     else "tdse_propagate_kernel"},
+        "roofline": roofline,
         "cpu_baseline": cpu,
         "gpu_over_cpu_baseline": (value / cpu["value"]) if cpu else None,
         "parity_vs_reference": parity,
