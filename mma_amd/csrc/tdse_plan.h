@@ -82,7 +82,7 @@ inline int resident_warm(int reach) { return reach / 8 + 4; }
 
 // The windows of one instance alone: lanes of 16 points (24 where carries reach further), four waves, one
 // per SIMD, a window; as many steps per launch as leave at most kOneWindows windows.  With 16001
-// points: 39 windows of 4096 points, 13 steps a launch.
+// points at dt 0.25, dx 0.1 (carries reach 151): 30 windows of 4096 points, 12 steps a launch.
 inline constexpr int kOneWindows = 64;
 inline bool plan_one(int nx, int reach, TdseResident &R)
 {

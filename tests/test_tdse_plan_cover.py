@@ -50,8 +50,8 @@ def plans(tmp_path_factory):
     return get
 
 
-# reach: 139 points at dx 0.1, dt 0.25; the table builder takes 320 at most
-REACHES = [1, 20, 96, 139, 140, 192, 193, 256, 257, 320]
+# reach: 151 points at dx 0.1, dt 0.25; the table builder takes 320 at most
+REACHES = [1, 20, 96, 139, 151, 192, 193, 256, 257, 320]
 
 
 def test_every_point_in_one_window(plans):
@@ -86,7 +86,7 @@ def test_where_the_covers_change(plans):
     # a window of C points a lane has ceil((nx + C - 1) / 64 C) waves, 8 at most
     expect = {1009: (16, 1, 1), 8177: (16, 8, 1), 8178: (24, 6, 1), 12265: (24, 8, 1), 12266: (32, 7, 1),
               16353: (32, 8, 1), 16354: (24, 8, 2)}
-    cases = [(n, 139) for n in expect]
+    cases = [(n, 151) for n in expect]
     for (nx, _), (p, _) in zip(cases, plans(cases)):
         assert (p["chunk"], p["waves"], p["windows"]) == expect[nx], (nx, p)
     # one window ends at 16353 points for every reach that 32 points a lane serve
@@ -97,6 +97,6 @@ def test_where_the_covers_change(plans):
 
 def test_grids_beyond_32_bit_offsets_are_left_to_the_streaming_kernels(plans):
     last = (1 << 27) - (1 << 16)
-    for (batch, one), ok in zip(plans([(last, 139), (last + 1, 139), ((1 << 31) - 64, 139)]), (1, 0, 0)):
+    for (batch, one), ok in zip(plans([(last, 151), (last + 1, 151), ((1 << 31) - 64, 151)]), (1, 0, 0)):
         assert batch["ok"] == one["ok"] == ok
         assert ok or batch["chunk"] == one["chunk"] == 0
