@@ -4,7 +4,6 @@ lattice that start as far into a lane as they can; several windows with the scan
 8 lanes); and snapshots of a grid of several windows in one workgroup.
 
 Tolerance as in test_tdse_resident_gpu.py: 40 eps a step at dt / dx^2 = 25, in proportion at 100."""
-import os
 
 import numpy as np
 import pytest
@@ -72,3 +71,26 @@ def test_snapshots_of_several_windows(dll, monkeypatch, num_r, tprint):
         o.delete(dll)
     for i in (inputs, inputs2):
         i.delete(dll)
+
+
+def test_windows_on_a_shared_lattice_match_the_oracle():
+    """The library's own launch on members of the uneven workload that share one lattice: the smallest, the widest (31997
+    points) and the one with the most work, both in several windows, over 600 steps."""
+    from oracle import ctdse as O
+    num_r, n_e = W.uneven_work()
+    work = (num_r + 1) * (n_e + 2)
+    pick = [int(i) for i in np.argsort(work)[:6]] + [int(np.argmax(num_r)), int(np.argmax(work))]
+    sel, steps = W.uneven_batch(indices=pick), 600
+    geos = create([m["num_r"] for m in sel])
+    dev = torch.tensor(np.stack([m["field"][: steps + 1] for m in sel]), device="cuda")
+    plan = tdse.BatchPlan(geos, dev)
+    assert plan.config.library_choice
+    out = plan.replay().cpu().numpy()
+    plan.close()
+    for i in (0, 6, 7):
+        x, psi0 = geos[i].ground_state()
+        ref = O.propagate(sel[i]["num_r"], 0.1, W.GRID["a"], 2.0, 0.25, psi0, x, dev[i].cpu().numpy(), steps)
+        for r, k in enumerate(("sourceterm", "PopTot", "PopInt", "expval")):
+            e = float(np.abs(out[i, r] - ref[k][:steps]).max())
+            print(sel[i]["num_r"], k, "%.2e" % e, flush=True)
+            assert e <= ATOL[r, 0] * steps / 120, (sel[i]["num_r"], k)
