@@ -267,7 +267,7 @@ def hankel_cpu_baseline(zg, rg, og, rho, src, pre, distance, threads, target_s=6
 
 def single_measure(geo, field, n_steps, nx, reps=1):
     """Per-instance form: one instance alone, as the reference-compatible call1DTDSE runs it
-    (ctdse_propagate_one: the segments of a step side by side, one launch per step); best of
+    (ctdse_propagate_one: overlapping windows side by side, up to 16 steps per launch); best of
     `reps` timed calls after one untimed call, allocation and the final wait included."""
     import torch
     from mma_amd import tdse
@@ -283,7 +283,7 @@ def single_measure(geo, field, n_steps, nx, reps=1):
         torch.cuda.synchronize()
         best = min(best, time.perf_counter() - s0)
     return {"pt_steps_per_s": nx * n_steps / best, "seconds": best, "Nx": nx, "steps": n_steps,
-            "launches": n_steps, "form": "ctdse_propagate_one"}
+            "form": "ctdse_propagate_one"}
 
 
 def call1dtdse_measure():
